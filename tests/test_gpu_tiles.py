@@ -1,0 +1,75 @@
+"""The tile kernels over the launch shapes they accept and the grids they meet:
+one to three quads per thread, tiles smaller and larger than the grid, odd and
+even rows and columns, not square.  FP64 against the oracle's fast cycle, FP32
+refinement against the one-launch-per-half-sweep kernels, bit for bit."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+import oracle
+from qdeqcycle_fdm_amd import config, lib
+
+pytestmark = pytest.mark.gpu
+
+PROD = dict(cycle=config.CYCLE_FAST, n_pre=1, n_post=3, n_coarse=0, relax=1.15)
+
+# (tile x, tile y, thread rows): few quads, one per thread, two per thread,
+# the rows raised to hold the tile, tiles taller and wider than the grids
+SHAPES = [(2, 2, 4), (32, 34, 8), (32, 34, 4), (50, 50, 4), (6, 200, 16), (200, 6, 4)]
+
+
+def _problem(ni, nk, levels):
+    pb = config.make_reference_problem(ni, nk, 24000.0 / (ni - 1))
+    return dataclasses.replace(pb, params=dataclasses.replace(pb.params, n_levels=levels))
+
+
+def _perturbed(pb, seed):
+    rng = np.random.default_rng(seed)
+    U = pb.U0.copy()
+    U[1:-1, 2:-2] += rng.normal(scale=0.5, size=(pb.params.nk, pb.params.ni - 2))
+    return U
+
+
+def _solve(pb, me, U, shape=None, **kw):
+    with lib.Engine(pb, me, **{**PROD, "tol": 1e-300, "max_vcycles": 2, **kw}) as eng:
+        if shape is None:
+            eng.set_tiles(False)
+        else:
+            n = len(eng.tile_shapes())
+            eng.set_tile_shapes([(shape, shape)] * n)
+        V = U.copy()
+        with pytest.raises(lib.QdeqError) as e:
+            eng.ode_solve(V)
+        assert e.value.status == lib.QDEQ_ERR_MG_NOT_CONVERGED
+    return V
+
+
+GRIDS = [(129, 129, 3), (130, 97, 3), (66, 131, 3), (129, 67, 3), (64, 64, 2), (63, 65, 2)]
+
+
+@pytest.mark.parametrize("ni,nk,levels", GRIDS)
+@pytest.mark.parametrize("n_pre,n_post", [(1, 3), (2, 2), (0, 1)])
+def test_fp64_tiles_equal_oracle(ni, nk, levels, n_pre, n_post):
+    pb = _problem(ni, nk, levels)
+    me = oracle.mu_equi(pb.mu)
+    U = _perturbed(pb, 21)
+    p = pb.params
+    mg = oracle.MG(ni, nk, p.dh, levels, me, relax=PROD["relax"])
+    mg.set_cycle(n_pre, n_post, 0, True)
+    ref = U.copy()
+    mg.solve(ref, oracle.ORC_TOL_ABS, 1e-300, 2)
+    for shape in SHAPES:
+        got = _solve(pb, me, U, shape, n_pre=n_pre, n_post=n_post)
+        np.testing.assert_array_equal(got, ref, err_msg=str(shape))
+
+
+@pytest.mark.parametrize("ni,nk,levels", GRIDS)
+def test_fp32_tiles_equal_untiled(ni, nk, levels):
+    pb = _problem(ni, nk, levels)
+    me = oracle.mu_equi(pb.mu)
+    U = _perturbed(pb, 22)
+    ref = _solve(pb, me, U, precision=config.PREC_FP32_IR)
+    for shape in SHAPES + [(66, 66, 4), (250, 16, 4)]:  # three quads per thread
+        got = _solve(pb, me, U, shape, precision=config.PREC_FP32_IR)
+        np.testing.assert_array_equal(got, ref, err_msg=str(shape))
