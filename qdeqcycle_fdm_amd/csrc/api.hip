@@ -293,7 +293,7 @@ int qdeq_set_tiles(qdeq_ctx *c, int tiled, int tile_x, int tile_y) {
                        "tile too small: " + std::to_string(blocks) +
                            " level-0 tiles, at most " + std::to_string(kPartialCap));
   }
-  c->tiled = tiled != 0;
+  c->tiled = c->ref_tiles = tiled != 0;
   c->tile_tx = tile_x;
   c->tile_ty = tile_y;
   c->tuned = false;

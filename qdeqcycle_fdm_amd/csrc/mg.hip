@@ -635,11 +635,16 @@ static void launch_bdres(qdeq_ctx *c) {
                      mb_dev(c) + SC_NORM0);
 }
 
+// Whether the solver's kernels all obey the gate, so that V-cycles may be
+// launched in batches and behind a start decided on the device: the tile
+// kernels, of either cycle.
+static bool gated(const qdeq_ctx *c) { return use_tiled(c) || use_ref_tiles(c); }
+
 // Whether solves of this context decide their start on the device: tiled
 // solves (FP64, and FP32-IR without a candidate start), unless
 // QDEQ_HOST_START=1.  The choices and norms are the same either way; the
 // host then waits only for the V-cycles.
-bool device_start(const qdeq_ctx *c) { return !c->host_start && use_tiled(c); }
+bool device_start(const qdeq_ctx *c) { return !c->host_start && gated(c); }
 
 // The same for a solve with a candidate start (projection or learned
 // guess): FP64 only; FP32-IR candidates always take the host path, which
@@ -662,6 +667,8 @@ static void launch_iteration(qdeq_ctx *c) {
   if (c->cfg.precision == QDEQ_PREC_FP32_IR) {
     if (tiled) {
       vcycle_tiled_fp32_ir(c);
+    } else if (use_ref_tiles(c)) {
+      vcycle_ref_fp32_ir(c);
     } else {
       vcycle<float, false>(c, c->s, 0, true);
       const LevelDims &d = c->lv[0];
@@ -672,6 +679,10 @@ static void launch_iteration(qdeq_ctx *c) {
   } else if (tiled) {
     int nparts = 0;
     vcycle_tiled_fp64(c, c->partial, &nparts);
+    launch_norm_final(c, nparts);
+  } else if (use_ref_tiles(c)) {
+    int nparts = 0;
+    vcycle_ref_fp64(c, c->partial, &nparts);
     launch_norm_final(c, nparts);
   } else {
     vcycle<double, true>(c, c->d, 0, false);
@@ -689,6 +700,7 @@ void mg_destroy_graphs(qdeq_ctx *c) {
 
 static int ensure_graph(qdeq_ctx *c) {
   const int mode = c->cfg.precision * 2 + c->cfg.cycle + (c->tiled ? 4 : 0) +
+                   (c->ref_tiles ? 8 : 0) +
                    64 * (c->tile_tx * 1024 + c->tile_ty);
   if (c->g_cycle && c->g_cycle_mode == mode) return QDEQ_OK;
   mg_destroy_graphs(c);
@@ -1113,7 +1125,7 @@ static int launch_batch_of(qdeq_ctx *c, MgSolve &m, int k, bool allow_sample) {
 // contraction (the tiled cycles only; one at a time otherwise or when
 // kernels are being timed).
 static int batch_size(const qdeq_ctx *c, double delta, double thr) {
-  if (!use_tiled(c) || (c->timing != 0 && c->timing != QDEQ_TIME_FAULT)) return 1;
+  if (!gated(c) || (c->timing != 0 && c->timing != QDEQ_TIME_FAULT)) return 1;
   const double rho = std::min(std::max(c->rho_est, 1e-3), 0.9);
   if (!(delta > 0) || !(thr > 0)) return 1;
   const double need = std::log(thr / delta) / std::log(rho);

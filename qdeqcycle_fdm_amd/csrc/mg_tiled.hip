@@ -490,7 +490,7 @@ __global__ __launch_bounds__(TILE_THREADS) void k_down(
     const T *__restrict__ uin, T *__restrict__ uout, const T *__restrict__ f,
     const T *__restrict__ cx, const T *__restrict__ cz, int N, int K, int P,
     T DH2, T relax, int nu, int zero_u, T *__restrict__ r2, int Nc, int Kc,
-    int Pc, int TX, int TY, const int *__restrict__ gate, StartArgs sa) {
+    int Pc, int TX, int TY, int H, const int *__restrict__ gate, StartArgs sa) {
   extern __shared__ __align__(16) unsigned char smem[];
   __shared__ double sdec[16 * 2];
   const int nthr = blockDim.x * blockDim.y;
@@ -504,7 +504,6 @@ __global__ __launch_bounds__(TILE_THREADS) void k_down(
   if (SMODE == START_PARTIALS) leave = sa.spec && sa.gate[sa.spec] != 1;
   if (SMODE == START_TEST) leave = sa.spec && sa.gate[6] == 0;
 
-  const int H = 2 * nu + 2;
   constexpr int PS = kPlaneWords<T, S>;
   const QTile<T, PS> t = make_qtile<T, PS>(smem, TX, TY, H);
   Quad<T> q[S];
@@ -689,27 +688,31 @@ __global__ __launch_bounds__(TILE_THREADS) void k_down(
 // Level-0 finishing modes of k_up.
 enum { UP_STORE = 0, UP_NORM = 1, UP_ADD64 = 2 };
 
+// Prolongation at the load: none (further sweeps, or the first sweeps of a
+// level when zero_u), the reference's, or with the last row too.
+enum { PROL_NONE = 0, PROL_REF = 1, PROL_FULL = 2 };
+
 // Prolongation + correction + post-smoothing, S quads per thread.
-template <typename T, bool HAS_F, bool EXACT, bool FULL_TOP, int MODE, int S>
+template <typename T, bool HAS_F, bool EXACT, int PROL, int MODE, int S>
 __global__ __launch_bounds__(TILE_THREADS) void k_up(
     const T *__restrict__ uin, T *__restrict__ uout, const T *__restrict__ f,
     const T *__restrict__ cx, const T *__restrict__ cz, int N, int K, int P,
-    T DH2, T relax, int nu, const T *__restrict__ e, int Nc, int Kc, int Pc,
-    int TX, int TY, double *__restrict__ partial, double *__restrict__ u64,
+    T DH2, T relax, int nu, int zero_u, const T *__restrict__ e, int Nc, int Kc, int Pc,
+    int TX, int TY, int H, double *__restrict__ partial, double *__restrict__ u64,
     const int *__restrict__ gate) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int nthr = blockDim.x * blockDim.y;
   const int ltid = threadIdx.y * blockDim.x + threadIdx.x;
   const bool leave = gate && gate[0];  // the solve has converged
-  const int H = up_halo(nu, MODE == UP_NORM);
   constexpr int PS = kPlaneWords<T, S>;
   const QTile<T, PS> t = make_qtile<T, PS>(smem, TX, TY, H);
   Quad<T> q[S];
 #pragma unroll
   for (int i = 0; i < S; i++) {
     quad_place(t, q[i], ltid + i * nthr, N, K);
-    quad_load<T, HAS_F>(t, q[i], uin, f, cx, cz, N, K, P, false);
-    quad_prolong<T, FULL_TOP>(t, q[i], e, Nc, Kc, Pc, N, K);
+    quad_load<T, HAS_F>(t, q[i], uin, f, cx, cz, N, K, P, PROL == PROL_NONE && zero_u);
+    if (PROL != PROL_NONE)
+      quad_prolong<T, PROL == PROL_FULL>(t, q[i], e, Nc, Kc, Pc, N, K);
   }
 #pragma unroll
   for (int i = 0; i < S; i++) {
@@ -1182,18 +1185,66 @@ static void with_quads_all(Fn fn) {
   for (int s = 1; s <= kMaxQuads<T>; s++) with_quads<T>(s, fn);
 }
 
+// One launch of k_down on level l: nu sweeps of src (zero with zero_u), the
+// residual restricted onto level l + 1, the swept values into dst; tiles of
+// shape sh with a halo of H points.
+template <typename T, bool EXACT>
+static void run_down(qdeq_ctx *c, LevelBufs<T> *B, int l, bool has_f, bool zero_u,
+                     int smode, const TileShape &sh, int H, int nu, const T *src, T *dst,
+                     const StartArgs &sa) {
+  const LevelDims &d = c->lv[l];
+  const LevelDims &dc = c->lv[l + 1];
+  const QuadLaunch<T> ql(sh, H);
+  const dim3 grd((d.K + sh.tx - 1) / sh.tx, (d.N + sh.ty - 1) / sh.ty);
+  const dim3 blk(TX_THREADS, ql.rows);
+  const T DH2 = (T)(d.DH * d.DH), relax = (T)c->cfg.relax;
+#define DOWN_ARGS                                                                        \
+  grd, blk, ql.lds, c->stream, src, dst, B[l].f, B[l].cx, B[l].cz, d.N, d.K, d.P, DH2,   \
+      relax, nu, zero_u ? 1 : 0, B[l + 1].f, dc.N, dc.K, dc.P, sh.tx, sh.ty, H,          \
+      (const int *)c->gate_ptr, sa
+  auto launch = [&](auto quads) {
+    constexpr int S = decltype(quads)::value;
+    if (smode == START_PARTIALS)
+      hipLaunchKernelGGL((k_down<T, false, EXACT, START_PARTIALS, S>), DOWN_ARGS);
+    else if (smode == START_TEST)
+      hipLaunchKernelGGL((k_down<T, true, EXACT, START_TEST, S>), DOWN_ARGS);
+    else if (has_f)
+      hipLaunchKernelGGL((k_down<T, true, EXACT, DOWN_PLAIN, S>), DOWN_ARGS);
+    else
+      hipLaunchKernelGGL((k_down<T, false, EXACT, DOWN_PLAIN, S>), DOWN_ARGS);
+  };
+  with_quads<T>(ql.quads, launch);
+#undef DOWN_ARGS
+}
+
+// One launch of k_up on level l: src (zero with zero_u) with the prolonged
+// correction of level l + 1 (PROL), nu sweeps, finished as MODE says.
+// Returns the number of workgroups (norm partials).
+template <typename T, bool EXACT, bool HAS_F, int PROL, int MODE>
+static int run_up(qdeq_ctx *c, LevelBufs<T> *B, int l, const TileShape &sh, int H, int nu,
+                  bool zero_u, const T *src, T *dst, double *partial, double *u64) {
+  const LevelDims &d = c->lv[l];
+  const LevelDims &dc = c->lv[PROL == PROL_NONE ? l : l + 1];
+  const T *e = PROL == PROL_NONE ? nullptr : B[l + 1].u;
+  const dim3 grd((d.K + sh.tx - 1) / sh.tx, (d.N + sh.ty - 1) / sh.ty);
+  const QuadLaunch<T> ql(sh, H);
+  const T DH2 = (T)(d.DH * d.DH), relax = (T)c->cfg.relax;
+  auto launch = [&](auto quads) {
+    constexpr int S = decltype(quads)::value;
+    hipLaunchKernelGGL((k_up<T, HAS_F, EXACT, PROL, MODE, S>), grd,
+                       dim3(TX_THREADS, ql.rows), ql.lds, c->stream, src, dst, B[l].f,
+                       B[l].cx, B[l].cz, d.N, d.K, d.P, DH2, relax, nu, zero_u ? 1 : 0, e,
+                       dc.N, dc.K, dc.P, sh.tx, sh.ty, H, partial, u64,
+                       (const int *)c->gate_ptr);
+  };
+  with_quads<T>(ql.quads, launch);
+  return (int)(grd.x * grd.y);
+}
+
 template <typename T, bool EXACT>
 static void launch_down(qdeq_ctx *c, LevelBufs<T> *B, int l, bool has_f,
                         bool zero_u, int smode = DOWN_PLAIN) {
   const LevelDims &d = c->lv[l];
-  const LevelDims &dc = c->lv[l + 1];
-  const TileShape sh = tile_shape(c, l, true);
-  const int TX = sh.tx, TY = sh.ty;
-  const int nu = c->cfg.n_pre;
-  const QuadLaunch<T> ql(sh, 2 * nu + 2);
-  const dim3 grd((d.K + TX - 1) / TX, (d.N + TY - 1) / TY);
-  const dim3 blk(TX_THREADS, ql.rows);
-  const T DH2 = (T)(d.DH * d.DH), relax = (T)c->cfg.relax;
   StartArgs sa{};
   if (smode != DOWN_PLAIN) {
     const TileShape s0 = tile_shape(c, 0, true);
@@ -1220,23 +1271,9 @@ static void launch_down(qdeq_ctx *c, LevelBufs<T> *B, int l, bool has_f,
     sa.cap = c->cfg.max_vcycles;
     sa.tol = c->cfg.tol;
   }
-#define DOWN_ARGS                                                                       \
-  grd, blk, ql.lds, c->stream, B[l].u, B[l].r, B[l].f, B[l].cx, B[l].cz, d.N, d.K, d.P, \
-      DH2, relax, nu, zero_u ? 1 : 0, B[l + 1].f, dc.N, dc.K, dc.P, TX, TY,              \
-      (const int *)c->gate_ptr, sa
-  auto launch = [&](auto quads) {
-    constexpr int S = decltype(quads)::value;
-    if (smode == START_PARTIALS)
-      hipLaunchKernelGGL((k_down<T, false, EXACT, START_PARTIALS, S>), DOWN_ARGS);
-    else if (smode == START_TEST)
-      hipLaunchKernelGGL((k_down<T, true, EXACT, START_TEST, S>), DOWN_ARGS);
-    else if (has_f)
-      hipLaunchKernelGGL((k_down<T, true, EXACT, DOWN_PLAIN, S>), DOWN_ARGS);
-    else
-      hipLaunchKernelGGL((k_down<T, false, EXACT, DOWN_PLAIN, S>), DOWN_ARGS);
-  };
-  with_quads<T>(ql.quads, launch);
-#undef DOWN_ARGS
+  const int nu = c->cfg.n_pre;
+  run_down<T, EXACT>(c, B, l, has_f, zero_u, smode, tile_shape(c, l, true), 2 * nu + 2, nu,
+                     B[l].u, B[l].r, sa);
 }
 
 // Whether a batch launched kernel by kernel may fold its stop tests into the
@@ -1270,26 +1307,14 @@ bool fused_start_fits(const qdeq_ctx *c) {
 template <typename T, bool EXACT, bool HAS_F, int MODE>
 static void launch_up_t(qdeq_ctx *c, LevelBufs<T> *B, int l, double *partial,
                         double *u64, int *nblocks) {
-  const LevelDims &d = c->lv[l];
-  const LevelDims &dc = c->lv[l + 1];
-  const TileShape sh = tile_shape(c, l, false);
-  const int TX = sh.tx, TY = sh.ty;
-  const dim3 grd((d.K + TX - 1) / TX, (d.N + TY - 1) / TY);
-  if (nblocks) *nblocks = (int)(grd.x * grd.y);
   const int nu = c->cfg.n_post;
-  const QuadLaunch<T> ql(sh, up_halo(nu, MODE == UP_NORM));
-  const T DH2 = (T)(d.DH * d.DH), relax = (T)c->cfg.relax;
-  auto launch = [&](auto quads) {
-    constexpr int S = decltype(quads)::value;
-    hipLaunchKernelGGL((k_up<T, HAS_F, EXACT, true, MODE, S>), grd,
-                       dim3(TX_THREADS, ql.rows), ql.lds, c->stream, B[l].r, B[l].u, B[l].f,
-                       B[l].cx, B[l].cz, d.N, d.K, d.P, DH2, relax, nu, B[l + 1].u, dc.N,
-                       dc.K, dc.P, TX, TY, partial, u64, (const int *)c->gate_ptr);
-  };
-  with_quads<T>(ql.quads, launch);
+  const int n = run_up<T, EXACT, HAS_F, PROL_FULL, MODE>(
+      c, B, l, tile_shape(c, l, false), up_halo(nu, MODE == UP_NORM), nu, false, B[l].r,
+      B[l].u, partial, u64);
+  if (nblocks) *nblocks = n;
 }
 
-template <typename T, bool EXACT>
+template <typename T, bool EXACT, bool FULL_TOP = true>
 static void launch_tail(qdeq_ctx *c, LevelBufs<T> *B, int lt) {
   TailArgs a{};
   a.nlev = c->L - lt;
@@ -1306,7 +1331,7 @@ static void launch_tail(qdeq_ctx *c, LevelBufs<T> *B, int lt) {
   a.cn = c->coarse_n;
   a.minv = c->coarse_n > 0 ? (const void *)c->cinv32 : nullptr;
   a.gate = c->gate_ptr;
-  hipLaunchKernelGGL((k_tail<T, EXACT, true>), dim3(1), dim3(TAIL_THREADS),
+  hipLaunchKernelGGL((k_tail<T, EXACT, FULL_TOP>), dim3(1), dim3(TAIL_THREADS),
                      tail_lds_bytes<T>(c, lt), c->stream, a);
 }
 
@@ -1350,6 +1375,161 @@ void vcycle_tiled_fp64(qdeq_ctx *c, double *partial, int *nparts) {
 
 void vcycle_tiled_fp32_ir(qdeq_ctx *c) {
   vcycle_tiled<float, false>(c, c->s, true, nullptr, c->d[0].u, nullptr);
+}
+
+// ---- the reference's V-cycle on the tile kernels ----
+//
+// Its 32 sweeps per smoothing (odeSolver.cpp:4) run as a few launches of
+// several sweeps each: k_up without prolongation for the first ones of a
+// descent, k_down for the last (with residual and restriction), k_up with the
+// reference's prolongation (the last row left alone) for the first of the
+// ascent; the levels that fit go to the tail.  Same expressions as the
+// launches per half-sweep, so the same bits.  One launch per half-sweep cost
+// 2.6 us each whatever the size up to 257^2 (448 of them a V-cycle at 129^2);
+// here a half-sweep costs 0.2 to 0.7 us inside a launch.
+
+// Model of a launch's time in us, from launches measured back to back: start,
+// first loads and store; the tile data; the half-sweeps at their latency plus
+// the issue of the quads that share a CU.
+static double pass_us(int tiles, int nq, int sweeps, double mbytes) {
+  const int per_cu = (tiles + 255) / 256;
+  return 3.3 + mbytes / 6.0 + 2 * sweeps * (0.17 + 0.017 * per_cu * nq / 64.0);
+}
+
+// `sweeps` split into as even passes of at most `most` sweeps as there are.
+static std::vector<int> split_sweeps(int sweeps, int most) {
+  const int n = std::max(1, (sweeps + most - 1) / most);
+  std::vector<int> v;
+  for (int i = 0; i < n; i++) v.push_back(sweeps / n + (i < sweeps % n ? 1 : 0));
+  return v;
+}
+
+// Tiles and passes of one level: the tile side and the sweeps per launch that
+// the model finds fastest, among square tiles with a halo and, where the
+// grid's quads fit one workgroup, one tile of the whole level without a halo
+// and all sweeps in a launch.
+template <typename T>
+static bool plan_level(const qdeq_ctx *c, int l, int n_pre, int n_post, RefLevel *out) {
+  const LevelDims &d = c->lv[l];
+  const int most_quads = kMaxQuads<T> * TILE_THREADS;
+  double best = 1e300;
+  auto consider = [&](int tx, int ty, int sweeps, bool whole) {
+    const std::vector<int> pre = split_sweeps(n_pre, sweeps);
+    std::vector<int> post;
+    if (n_post >= 0) post = split_sweeps(n_post, sweeps);
+    const int tiles = ((d.K + tx - 1) / tx) * ((d.N + ty - 1) / ty);
+    if (l == 0 && tiles > kPartialCap) return;
+    double us = 0.0;
+    for (const auto *v : {&pre, static_cast<const std::vector<int> *>(&post)})
+      for (int s : *v) {
+        const int H = whole ? 0 : 2 * s + 2;
+        const int R = ty + 2 * H, C = tx + 2 * H, nq = (R / 2) * (C / 2);
+        if (nq > most_quads || C > 5 * TX_THREADS) return;
+        us += pass_us(tiles, nq, s, 1e-6 * tiles * nq * 4.0 * sizeof(T) * 4.0);
+      }
+    if (us < best) {
+      best = us;
+      *out = RefLevel{TileShape{tx, ty, TY_THREADS}, whole, pre, post};
+    }
+  };
+  consider(d.K + (d.K & 1), d.N + (d.N & 1), std::max(1, std::max(n_pre, n_post)), true);
+  for (int sweeps : {1, 2, 4, 6, 8, 11, 16})
+    for (int t : {4, 6, 8, 10, 12, 14, 18, 22, 26, 30, 34, 38, 42, 46, 50, 54, 58, 62, 66})
+      consider(t, t, sweeps, false);
+  return best < 1e300;
+}
+
+// The plan of every level above the tail (or of all of them when the
+// coarsest does not fit it), empty if some level has none.
+template <typename T>
+static void plan_reference(qdeq_ctx *c) {
+  c->ref_plan.clear();
+  if (c->cfg.cycle != QDEQ_CYCLE_REFERENCE) return;
+  const int lt = tail_fits(c, sizeof(T) == 8) ? tail_entry_level(c) : c->L;
+  c->ref_tail = lt;
+  for (int l = 0; l < lt; l++) {
+    const bool coarsest = l == c->L - 1;
+    RefLevel p;
+    if (!plan_level<T>(c, l, coarsest ? c->cfg.n_coarse : c->cfg.n_pre,
+                       coarsest ? -1 : c->cfg.n_post, &p)) {
+      c->ref_plan.clear();
+      return;
+    }
+    // level 0 starts and ends in u: an even number of passes
+    if (l == 0 && ((p.pre.size() + p.post.size()) & 1)) {
+      std::vector<int> &v = p.pre;
+      if (v[0] >= 2) {
+        v.insert(v.begin(), v[0] / 2);
+        v[1] -= v[0];
+      } else {
+        v.insert(v.begin(), 0);
+      }
+    }
+    c->ref_plan.push_back(p);
+  }
+}
+
+bool use_ref_tiles(const qdeq_ctx *c) { return c->ref_tiles && !c->ref_plan.empty(); }
+
+template <typename T, bool EXACT>
+static void vcycle_ref(qdeq_ctx *c, LevelBufs<T> *B, bool level0_has_f, double *partial,
+                       double *u64, int *nparts) {
+  const int lt = c->ref_tail;
+  // pass i of a level's n writes u when an even number follows, else r, and
+  // reads the other
+  auto pass = [&](int l, int i, bool down) {
+    const RefLevel &p = c->ref_plan[l];
+    const int np = (int)p.pre.size(), n = np + (int)p.post.size();
+    const int nu = i < np ? p.pre[i] : p.post[i - np];
+    const bool last = i == n - 1, zero = i == 0 && (l > 0 || level0_has_f);
+    const bool has_f = l > 0 || level0_has_f;
+    const bool prol = i == np, add = l == 0 && last && u64;
+    const bool norm = l == 0 && last && !level0_has_f;
+    T *dst = ((n - 1 - i) & 1) ? B[l].r : B[l].u;
+    const T *src = dst == B[l].u ? B[l].r : B[l].u;
+    const int H = p.whole ? 0 : (down ? 2 * nu + 2 : up_halo(nu, norm));
+    if (down) {
+      run_down<T, EXACT>(c, B, l, has_f, zero, DOWN_PLAIN, p.sh, H, nu, src, dst,
+                         StartArgs{});
+      return;
+    }
+    auto up = [&](auto pr) {
+      constexpr int PR = decltype(pr)::value;
+      if (norm)
+        *nparts = run_up<T, EXACT, false, PR, UP_NORM>(c, B, l, p.sh, H, nu, zero, src,
+                                                       dst, partial, nullptr);
+      else if (add)
+        run_up<T, EXACT, true, PR, UP_ADD64>(c, B, l, p.sh, H, nu, zero, src, dst, nullptr,
+                                             u64);
+      else if (has_f)
+        run_up<T, EXACT, true, PR, UP_STORE>(c, B, l, p.sh, H, nu, zero, src, dst, nullptr,
+                                             nullptr);
+      else
+        run_up<T, EXACT, false, PR, UP_STORE>(c, B, l, p.sh, H, nu, zero, src, dst,
+                                              nullptr, nullptr);
+    };
+    if (prol)
+      up(std::integral_constant<int, PROL_REF>{});
+    else
+      up(std::integral_constant<int, PROL_NONE>{});
+  };
+  for (int l = 0; l < lt; l++) {
+    const int np = (int)c->ref_plan[l].pre.size();
+    for (int i = 0; i < np; i++) pass(l, i, i == np - 1 && l < c->L - 1);
+  }
+  if (lt < c->L) launch_tail<T, EXACT, false>(c, B, lt);
+  for (int l = lt - 1; l >= 0; l--) {
+    const RefLevel &p = c->ref_plan[l];
+    for (int i = 0; i < (int)p.post.size(); i++) pass(l, (int)p.pre.size() + i, false);
+  }
+}
+
+void vcycle_ref_fp64(qdeq_ctx *c, double *partial, int *nparts) {
+  vcycle_ref<double, true>(c, c->d, false, partial, nullptr, nparts);
+}
+
+void vcycle_ref_fp32_ir(qdeq_ctx *c) {
+  vcycle_ref<float, false>(c, c->s, true, nullptr, c->d[0].u, nullptr);
 }
 
 // ---- tile-shape autotuner ----
@@ -1603,20 +1783,36 @@ int tiled_setup(qdeq_ctx *c) {
     SETA((k_down<double, false, true, DOWN_PLAIN, S>));
     SETA((k_down<double, false, true, START_PARTIALS, S>));
     SETA((k_down<double, true, true, START_TEST, S>));
-    SETA((k_up<double, true, true, true, UP_STORE, S>));
-    SETA((k_up<double, false, true, true, UP_NORM, S>));
+    SETA((k_up<double, true, true, PROL_FULL, UP_STORE, S>));
+    SETA((k_up<double, false, true, PROL_FULL, UP_NORM, S>));
+    SETA((k_up<double, true, true, PROL_REF, UP_STORE, S>));
+    SETA((k_up<double, true, true, PROL_NONE, UP_STORE, S>));
+    SETA((k_up<double, false, true, PROL_REF, UP_STORE, S>));
+    SETA((k_up<double, false, true, PROL_NONE, UP_STORE, S>));
+    SETA((k_up<double, false, true, PROL_REF, UP_NORM, S>));
+    SETA((k_up<double, false, true, PROL_NONE, UP_NORM, S>));
   });
   with_quads_all<float>([&](auto quads) {
     constexpr int S = decltype(quads)::value;
     SETA((k_down<float, true, false, DOWN_PLAIN, S>));
-    SETA((k_up<float, true, false, true, UP_STORE, S>));
-    SETA((k_up<float, true, false, true, UP_ADD64, S>));
+    SETA((k_up<float, true, false, PROL_FULL, UP_STORE, S>));
+    SETA((k_up<float, true, false, PROL_FULL, UP_ADD64, S>));
+    SETA((k_up<float, true, false, PROL_REF, UP_STORE, S>));
+    SETA((k_up<float, true, false, PROL_NONE, UP_STORE, S>));
+    SETA((k_up<float, true, false, PROL_REF, UP_ADD64, S>));
+    SETA((k_up<float, true, false, PROL_NONE, UP_ADD64, S>));
   });
   SETA((k_tail<double, true, true>));
   SETA((k_tail<float, false, true>));
+  SETA((k_tail<double, true, false>));
+  SETA((k_tail<float, false, false>));
 #undef SETA
   (void)hipGetLastError();
   if (!tiles_fit(c, c->tile_tx, c->tile_ty)) c->tiled = false;
+  if (c->cfg.precision == QDEQ_PREC_FP32_IR)
+    plan_reference<float>(c);
+  else
+    plan_reference<double>(c);
   return QDEQ_OK;
 }
 

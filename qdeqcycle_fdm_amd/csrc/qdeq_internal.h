@@ -32,6 +32,15 @@ struct TileShape {
   int tx, ty, tyt;
 };
 
+// Reference cycle on the tile kernels, one level: the tiles, whether one
+// tile is the whole level (no halo), and the sweeps of each launch of the
+// descent and the ascent.
+struct RefLevel {
+  TileShape sh;
+  bool whole;
+  std::vector<int> pre, post;
+};
+
 // Device buffers of one level.  u: level 0 = displacement (FP64 path) or the
 // IR correction (FP32 path); levels >= 1 = coarse correction.  f: right-hand
 // side (level 0 FP64 = zero, never read).  r: residual scratch.  cx: west-face
@@ -194,6 +203,11 @@ struct qdeq_ctx {
   // with 16 thread rows
   bool tuned = false;
   qdeq::TileShape tdown[QDEQ_MAX_LEVELS] = {}, tup[QDEQ_MAX_LEVELS] = {};
+  // reference cycle: the levels above the tail (empty: one launch per
+  // half-sweep), the tail's entry level, and whether it is used
+  std::vector<qdeq::RefLevel> ref_plan;
+  int ref_tail = 0;
+  bool ref_tiles = true;
   size_t lds_max = 65536;  // dynamic LDS per workgroup (queried at creation)
   // direct coarsest-level solve of the fast cycle (n_coarse == 0): inverse of
   // the coarsest operator, column-major, stored in FP32 (products and sums
@@ -304,6 +318,9 @@ int tail_entry_level(const qdeq_ctx *c);
 bool tail_fits(const qdeq_ctx *c, bool fp64);
 void vcycle_tiled_fp64(qdeq_ctx *c, double *partial, int *nparts);
 void vcycle_tiled_fp32_ir(qdeq_ctx *c);
+bool use_ref_tiles(const qdeq_ctx *c);
+void vcycle_ref_fp64(qdeq_ctx *c, double *partial, int *nparts);
+void vcycle_ref_fp32_ir(qdeq_ctx *c);
 int tiled_setup(qdeq_ctx *c);
 bool tiles_fit(const qdeq_ctx *c, int tx, int ty);
 bool fused_start_fits(const qdeq_ctx *c);

@@ -73,3 +73,27 @@ def test_fp32_tiles_equal_untiled(ni, nk, levels):
     for shape in SHAPES + [(66, 66, 4), (250, 16, 4)]:  # three quads per thread
         got = _solve(pb, me, U, shape, precision=config.PREC_FP32_IR)
         np.testing.assert_array_equal(got, ref, err_msg=str(shape))
+
+
+@pytest.mark.parametrize("ni,nk,levels", [(129, 129, 3), (130, 97, 3), (66, 131, 2), (41, 57, 1),
+                                          (257, 65, 4), (100, 101, 2)])
+@pytest.mark.parametrize("sweeps", [(32, 32, 32), (5, 8, 3), (0, 1, 1)])
+def test_reference_cycle_on_tiles_equals_oracle(ni, nk, levels, sweeps):
+    """The reference's V-cycle in passes of several sweeps: levels in tiles
+    with a halo, whole levels in one tile, with and without the tail, odd and
+    even numbers of passes."""
+    pb = _problem(ni, nk, levels)
+    me = oracle.mu_equi(pb.mu)
+    U = _perturbed(pb, 23)
+    p = pb.params
+    mg = oracle.MG(ni, nk, p.dh, levels, me)
+    mg.set_cycle(*sweeps, False)
+    ref = U.copy()
+    mg.solve(ref, oracle.ORC_TOL_ABS, 1e-300, 2)
+    with lib.Engine(pb, me, tol=1e-300, max_vcycles=2, n_pre=sweeps[0], n_post=sweeps[1],
+                    n_coarse=sweeps[2]) as eng:
+        V = U.copy()
+        with pytest.raises(lib.QdeqError) as e:
+            eng.ode_solve(V)
+        assert e.value.status == lib.QDEQ_ERR_MG_NOT_CONVERGED
+    np.testing.assert_array_equal(V, ref)
