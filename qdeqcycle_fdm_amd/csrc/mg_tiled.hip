@@ -35,22 +35,12 @@ constexpr int TY_THREADS = 16;   // 16 rows of lanes: 1024 threads per tile
 constexpr int TILE_THREADS = TX_THREADS * TY_THREADS;
 constexpr int TAIL_THREADS = 1024;
 constexpr int TAIL_MAX_N = 33;  // levels with N, K <= this run in the tail
-// the tail loads a level's arrays in at most two passes of its threads
-static_assert((TAIL_MAX_N + 1) * TAIL_MAX_N <= 2 * TAIL_THREADS, "tail load passes");
+// one quad of a tail level per thread
+static_assert(((TAIL_MAX_N + 1) / 2) * ((TAIL_MAX_N + 1) / 2) <= TAIL_THREADS, "tail quads");
 
-template <typename T, bool EXACT>
-__device__ inline T rbgs_update(T m1, T m2, T m3, T m4, T uW, T uE, T uS,
-                                T uN, T uC, T fDH2, bool has_f, T relax) {
-  T num = m1 * uW + m2 * uE + m3 * uS + m4 * uN;
-  if (has_f) num = num - fDH2;
-  if (EXACT) return (relax / (m1 + m2 + m3 + m4)) * num + (T(1) - relax) * uC;
-  const T unew = num / (m1 + m2 + m3 + m4);
-  return (relax == T(1)) ? unew : uC + relax * (unew - uC);
-}
-
-// The update of rbgs_update with the per-point quantity a formed once:
-// relax / (m1 + m2 + m3 + m4) (EXACT) or m1 + m2 + m3 + m4 (plain), the
-// same operations in the same order, so the same bits.
+// Update of one point with its quantity a = relax / (m1 + m2 + m3 + m4)
+// (EXACT, the reference's form) or m1 + m2 + m3 + m4 (plain) formed once: the
+// operations of k_rbgs in the same order, so the same bits.
 template <typename T, bool EXACT>
 __device__ inline T rbgs_update_pre(T a, T m1, T m2, T m3, T m4, T uW, T uE, T uS,
                                     T uN, T uC, T fDH2, bool has_f, T relax) {
@@ -410,6 +400,22 @@ __device__ inline void quad_residual(const QTile<T, PS> &t, const Quad<T> &p, T 
   r11 = p.k11 ? d : T(0);
 }
 
+// Full weighting onto the coarse point under a quad's (0, 0) (the expression
+// of k_restrict): the quad's own residuals and those of its west, south and
+// south-west quads in the planes of r.  The first and last coarse rows use
+// their one fine neighbour row twice.
+template <typename T, int PS>
+__device__ inline T quad_restrict(const QTile<T, PS> &r, int id, T r00, T r01, T r10, T r11,
+                                  bool first, bool last) {
+  const int s = id - r.C2;
+  const T nm = r.p11()[id - 1];
+  const T s0 = r.p10()[s], sm = r.p11()[s - 1], sp = r.p11()[s];
+  const T rs0 = first ? r10 : s0, rsm = first ? nm : sm, rsp = first ? r11 : sp;
+  const T rn0 = last ? s0 : r10, rnm = last ? sm : nm, rnp = last ? sp : r11;
+  return T(0.0625) * (T(4.0) * r00 + T(2.0) * r.p01()[id - 1] + T(2.0) * r01 +
+                      T(2.0) * rs0 + T(2.0) * rn0 + rsm + rsp + rnm + rnp);
+}
+
 // Whether the quad lies in the tile's interior (H and the tile are even),
 // and the global row and column of its point (0, 0).
 template <typename T, int PS>
@@ -672,15 +678,8 @@ __global__ __launch_bounds__(TILE_THREADS) void k_down(
     // coarse rows use their one fine neighbour row twice
     const int jc = j >> 1, kc = k >> 1;
     if (jc >= Nc || kc < 1 || kc > Kc - 2) continue;
-    const int s = p.id - t.C2;
-    const bool first = jc == 0, last = jc == Nc - 1;
-    const T n0 = r10[i], nm = t.p11()[p.id - 1], np = r11[i];
-    const T s0 = t.p10()[s], sm = t.p11()[s - 1], sp = t.p11()[s];
-    const T rs0 = first ? n0 : s0, rsm = first ? nm : sm, rsp = first ? np : sp;
-    const T rn0 = last ? s0 : n0, rnm = last ? sm : nm, rnp = last ? sp : np;
-    const T v = T(0.0625) *
-                (T(4.0) * r00[i] + T(2.0) * t.p01()[p.id - 1] + T(2.0) * r01[i] +
-                 T(2.0) * rs0 + T(2.0) * rn0 + rsm + rsp + rnm + rnp);
+    const T v = quad_restrict(t, p.id, r00[i], r01[i], r10[i], r11[i], jc == 0,
+                              jc == Nc - 1);
     r2[(size_t)jc * Pc + kc] = v;
   }
 }
@@ -767,8 +766,16 @@ __global__ __launch_bounds__(TILE_THREADS) void k_up(
 }
 
 // ---------------------------------------------------------------------------
-// Coarse tail: one workgroup, every level (values and coefficients) in LDS.
+// Coarse tail: one workgroup runs every level with N, K <= 33.
 // ---------------------------------------------------------------------------
+//
+// One quad per thread and level (289 of them at 33^2, so five wavefronts
+// sweep and the others only wait); values in planes, residuals, right-hand
+// sides and corrections in the LDS.  A V-cycle's tail is a serial chain of
+// small steps in one CU, bound by LDS and barrier latency and by its loads.
+// Against one point of each colour per thread over all 16 wavefronts, FP64
+// with entry level 33^2: the production cycle's tail 13.9 -> 10.4 us, the
+// reference's (192 half-sweeps) 84 -> 44 us.
 
 struct TailLevel {
   const void *cx, *cz;  // global coefficients of the level
@@ -788,288 +795,298 @@ struct TailArgs {
   const int *gate;      // skip flag of a batched solve, or null
 };
 
-// compact arrays of a tail level, stride K: u, f, cx and cz (N+1 rows)
-template <typename T>
-struct TailBufs {
-  T *u, *f, *cx, *cz;
-};
+constexpr int kTailAhead = 32;
 
+// LDS words of a tail level: its value planes, and its right-hand side
+// (rows 0..N, so that a quad's second row of the last one stays inside).
+__host__ __device__ inline int tail_quads(int N, int K) {
+  return ((N + 1) / 2) * ((K + 1) / 2);
+}
+constexpr int kTailPlane = ((TAIL_MAX_N + 1) / 2) * ((TAIL_MAX_N + 1) / 2) +
+                           (TAIL_MAX_N + 1) / 2 + 1;
+__host__ __device__ inline size_t tail_plane_words(int K) {
+  return 4 * (size_t)kTailPlane + (size_t)quad_guard((K + 1) / 2);
+}
 __host__ __device__ inline size_t tail_level_words(int N, int K) {
-  return 4 * (size_t)N * K + K;
+  return tail_plane_words(K) + (size_t)(N + 1) * K + 2;
 }
 
-// LDS arrays of tail level l, recomputed from the level dimensions (uniform
-// values) at each use: a per-level table indexed by a loop variable would
-// live in per-lane scratch memory.
+// Level l's planes as a tile that covers the level, and its right-hand side;
+// recomputed from the level dimensions (uniform values) at each use: a
+// per-level table indexed by a loop variable would live in per-lane scratch
+// memory.
 template <typename T>
-__device__ inline TailBufs<T> tail_bufs(T *base, const TailArgs &a, int l) {
-  size_t off = 0;
-  for (int i = 0; i < l; i++) off += tail_level_words(a.lv[i].N, a.lv[i].K);
-  const size_t n = (size_t)a.lv[l].N * a.lv[l].K;
-  T *b = base + off;
-  return TailBufs<T>{b, b + n, b + 2 * n, b + 3 * n};
+__device__ inline QTile<T, kTailPlane> tail_tile(T *base, const TailArgs &a, int l) {
+  for (int i = 0; i < l; i++) base += tail_level_words(a.lv[i].N, a.lv[i].K);
+  QTile<T, kTailPlane> t;
+  t.C2 = (a.lv[l].K + 1) / 2;
+  t.nq = tail_quads(a.lv[l].N, a.lv[l].K);
+  t.j0 = t.k0 = 0;
+  t.p = base + quad_guard(t.C2);
+  t.stride = 0;
+  return t;
+}
+template <typename T>
+__device__ inline T *tail_rhs(T *base, const TailArgs &a, int l) {
+  for (int i = 0; i < l; i++) base += tail_level_words(a.lv[i].N, a.lv[i].K);
+  return base + tail_plane_words(a.lv[l].K);
 }
 
-template <typename T>
-__device__ inline T *tail_end(T *base, const TailArgs &a) {
-  size_t off = 0;
-  for (int i = 0; i < a.nlev; i++) off += tail_level_words(a.lv[i].N, a.lv[i].K);
-  return base + off;
+// The thread's quad of level l: place, coefficients and factors (values zero).
+template <typename T, bool EXACT>
+__device__ inline void tail_quad(const QTile<T, kTailPlane> &t, Quad<T> &q, const TailLevel &L,
+                                 T relax) {
+  quad_place(t, q, (int)threadIdx.x, L.N, L.K);
+  if (!q.valid) return;
+  quad_load<T, false>(t, q, (const T *)nullptr, (const T *)nullptr, (const T *)L.cx,
+                      (const T *)L.cz, L.N, L.K, L.P, true);
+  quad_factors<T, EXACT>(q, relax);
 }
 
-// Sweeps on one tail level.  With one_wave, the first wavefront alone runs
-// them (small coarsest grids), ordering its own LDS traffic between
-// half-sweeps with wavefront fences instead of workgroup barriers.
-// One point of colour COL of a thread that holds its coefficients, DH^2 f
-// and relaxation factor in registers.
+// Its right-hand side from the LDS.
 template <typename T>
-struct TailPoint {
-  T m1, m2, m3, m4, a, fv;
-  int c, cS, cN;
-  bool ok;
+__device__ inline void tail_quad_rhs(const QTile<T, kTailPlane> &t, Quad<T> &q, const T *F, int K) {
+  if (!q.valid) return;
+  int j, k;
+  quad_rc(t, q.id, j, k);
+  const T *f = F + j * K + k;
+  q.f00 = f[0];
+  q.f01 = f[1];
+  q.f10 = f[K];
+  q.f11 = f[K + 1];
+}
+
+// Sweeps of the level by the threads that hold a quad.
+template <typename T, bool EXACT>
+__device__ inline void tail_sweep(const QTile<T, kTailPlane> &t, Quad<T> &q, int nu, T DH2, T relax) {
+  Quad<T>(&qs)[1] = reinterpret_cast<Quad<T>(&)[1]>(q);
+  for (int s = 0; s < nu; s++) {
+    if (q.valid) quads_half_sweep<T, true, EXACT, false, 0, 1>(t, qs, DH2, relax);
+    __syncthreads();
+    if (q.valid) quads_half_sweep<T, true, EXACT, false, 1, 1>(t, qs, DH2, relax);
+    __syncthreads();
+  }
+}
+
+// Values of the level into the row-major correction E (boundary columns too).
+template <typename T>
+__device__ inline void tail_put_e(const QTile<T, kTailPlane> &t, const Quad<T> &q, T *E, int N,
+                                  int K) {
+  if (!q.valid) return;
+  int j, k;
+  quad_rc(t, q.id, j, k);
+  T *e = E + j * K + k;
+  e[0] = q.u00;
+  if (k + 1 < K) e[1] = q.u01;
+  if (j + 1 < N) {
+    e[K] = q.u10;
+    if (k + 1 < K) e[K + 1] = q.u11;
+  }
+}
+
+// Residual of level l and its restriction into F (the next level's right-hand
+// side) and, for a direct coarsest solve, DH^2 times it into G.
+template <typename T>
+__device__ inline void tail_restrict(const QTile<T, kTailPlane> &t, const Quad<T> &q, T *R, T DH2,
+                                     T *F, T *G, T DH2c, int Nc, int Kc) {
+  QTile<T, kTailPlane> r = t;
+  r.p = R + quad_guard(t.C2);
+  T r00, r01, r10, r11;
+  if (q.valid) {
+    quad_residual<T, true>(t, q, DH2, r00, r01, r10, r11);
+    r.p01()[q.id] = r01;
+    r.p10()[q.id] = r10;
+    r.p11()[q.id] = r11;
+  }
+  __syncthreads();
+  if (q.valid) {
+    const int jc = q.id / t.C2, kc = q.id - jc * t.C2;
+    if (jc < Nc && kc >= 1 && kc <= Kc - 2) {
+      const T v = quad_restrict(r, q.id, r00, r01, r10, r11, jc == 0, jc == Nc - 1);
+      F[jc * Kc + kc] = v;
+      if (G) G[jc * (Kc - 2) + kc - 1] = DH2c * v;
+    }
+  }
+  __syncthreads();
+}
+
+// LDS behind the levels' arrays: residual planes, corrections, the direct
+// solve's right-hand side and partial sums.
+template <typename T>
+struct TailScratch {
+  T *R, *E, *G, *part;
+  __device__ TailScratch(T *base, const TailArgs &a) {
+    R = base;
+    for (int i = 0; i < a.nlev; i++) R += tail_level_words(a.lv[i].N, a.lv[i].K);
+    E = R + tail_plane_words(a.lv[0].K);
+    G = E + a.lv[0].N * a.lv[0].K;
+    part = G + a.cn;
+  }
 };
 
-template <typename T, bool EXACT>
-__device__ inline TailPoint<T> tail_point(const TailBufs<T> &b, int N, int K, T DH2,
-                                          T relax, bool act, int j, int q, int col) {
-  TailPoint<T> p;
-  const int k = 2 * q + ((j + col) & 1);
-  p.ok = act && k >= 1 && k <= K - 2;
-  const int kk = p.ok ? k : 1;  // a point that stays put reads in-range values
-  const int jS = (j == 0) ? 1 : j - 1;
-  const int jN = (j == N - 1) ? N - 2 : j + 1;
-  p.c = j * K + kk;
-  p.cS = jS * K + kk;
-  p.cN = jN * K + kk;
-  p.m1 = b.cx[p.c];
-  p.m2 = b.cx[p.c + 1];
-  p.m3 = b.cz[p.c];
-  p.m4 = b.cz[p.c + K];
-  p.a = rbgs_factor<T, EXACT>(p.m1, p.m2, p.m3, p.m4, relax);
-  p.fv = DH2 * b.f[p.c];
-  return p;
-}
-
-template <typename T, bool EXACT>
-__device__ inline void tail_point_update(const TailBufs<T> &b, const TailPoint<T> &p,
-                                         T relax) {
-  const T v = rbgs_update_pre<T, EXACT>(p.a, p.m1, p.m2, p.m3, p.m4, b.u[p.c - 1],
-                                        b.u[p.c + 1], b.u[p.cS], b.u[p.cN], b.u[p.c],
-                                        p.fv, true, relax);
-  if (p.ok) b.u[p.c] = v;
-}
-
-template <typename T, bool EXACT>
-__device__ inline void tail_smooth(const TailBufs<T> &b, int N, int K, T DH2,
-                                   T relax, int sweeps, bool one_wave) {
-  const int half = (K + 1) / 2;
-  const int tid = threadIdx.x;
-  const int nthr = one_wave ? 64 : (int)blockDim.x;
-  if (one_wave && tid >= 64) return;
-  if (N * half <= nthr && !one_wave) {
-    // one point of each colour per thread: its coefficients, right-hand
-    // side and factor read once into registers (f does not change while the
-    // level is smoothed), the same update expression
-    const bool act = tid < N * half;
-    const int j = act ? tid / half : 0, q = act ? tid - j * half : 0;
-    const TailPoint<T> p0 = tail_point<T, EXACT>(b, N, K, DH2, relax, act, j, q, 0);
-    const TailPoint<T> p1 = tail_point<T, EXACT>(b, N, K, DH2, relax, act, j, q, 1);
-    for (int s = 0; s < sweeps; s++) {
-      tail_point_update<T, EXACT>(b, p0, relax);
-      __syncthreads();
-      tail_point_update<T, EXACT>(b, p1, relax);
-      __syncthreads();
-    }
-    return;
-  }
-  for (int s = 0; s < 2 * sweeps; s++) {
-    const int colour = s & 1;
-    for (int idx = tid; idx < N * half; idx += nthr) {
-      const int j = idx / half, q = idx - j * half;
-      const int k = 2 * q + ((j + colour) & 1);
-      if (k < 1 || k > K - 2) continue;
-      const int jS = (j == 0) ? 1 : j - 1;
-      const int jN = (j == N - 1) ? N - 2 : j + 1;
-      const int c = j * K + k;
-      b.u[c] = rbgs_update<T, EXACT>(b.cx[c], b.cx[c + 1], b.cz[c], b.cz[c + K],
-                                     b.u[c - 1], b.u[c + 1], b.u[jS * K + k],
-                                     b.u[jN * K + k], b.u[c], DH2 * b.f[c], true,
-                                     relax);
-    }
-    if (one_wave) {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    } else {
-      __syncthreads();
+// Column sums of the direct coarsest solve by thread: row `row` and columns
+// c0 .. c1-1 (the split of coarse_matvec), the first AHEAD of the inverse's
+// entries fetched early.
+template <typename T, int AHEAD>
+struct TailDirect {
+  float ahead[AHEAD > 0 ? AHEAD : 1];
+  int row, c0, c1;
+  __device__ void fetch(const TailArgs &a) {
+    const float *minv = reinterpret_cast<const float *>(a.minv);
+    const int n = a.cn, tid = threadIdx.x;
+    const int Q = coarse_chunks(n), C = coarse_chunk_len(n), ch = tid / n;
+    row = tid - ch * n;
+    c0 = min(ch * C, n);
+    c1 = ch < Q ? min((ch + 1) * C, n) : c0;
+    // one 32-bit offset stepped from column to column (clamped to the last)
+    unsigned off = (unsigned)(min(c0, n - 1) * n + row) * 4u;
+    const unsigned end = (unsigned)((n - 1) * n + row) * 4u;
+#pragma unroll
+    for (int i = 0; i < AHEAD; i++) {
+      ahead[i] = load_at<float>(minv, off);
+      off = min(off + (unsigned)n * 4u, end);
     }
   }
-}
+  // corrections E of the coarsest level L from s.G; starts after and ends
+  // with a barrier
+  __device__ void solve(const TailArgs &a, const TailScratch<T> &s, const TailLevel &L) {
+    const float *minv = reinterpret_cast<const float *>(a.minv);
+    const int n = a.cn, tid = threadIdx.x, W = L.K - 2, Q = coarse_chunks(n);
+    T acc = T(0);
+#pragma unroll
+    for (int i = 0; i < AHEAD; i++)
+      if (c0 + i < c1) acc = acc + (T)ahead[i] * s.G[c0 + i];
+#pragma unroll 8
+    for (int col = c0 + AHEAD; col < c1; col++)
+      acc = acc + (T)load_at<float>(minv, (unsigned)(col * n + row) * 4u) * s.G[col];
+    s.part[tid] = acc;
+    __syncthreads();
+    for (int i = tid; i < n; i += TAIL_THREADS) {
+      T v = s.part[i];
+      for (int ch = 1; ch < Q; ch++) v = v + s.part[ch * n + i];
+      const int j = i / W, k = i - j * W + 1;
+      s.E[j * L.K + k] = v;
+      if (k == 1) s.E[j * L.K] = T(0);
+      if (k == W) s.E[j * L.K + W + 1] = T(0);
+    }
+    __syncthreads();
+  }
+};
 
+// Any tail: each visit of a level loads its quads' coefficients again.
 template <typename T, bool EXACT, bool FULL_TOP>
 __global__ __launch_bounds__(TAIL_THREADS) void k_tail(TailArgs a) {
   if (a.gate && a.gate[0]) return;  // the solve has converged
   extern __shared__ __align__(16) unsigned char smem[];
   T *base = reinterpret_cast<T *>(smem);
-  T *Rs = tail_end(base, a);  // residual scratch (entry level size)
-  T *Gs = Rs + (a.lv[0].N * a.lv[0].K > a.cn ? a.lv[0].N * a.lv[0].K : a.cn);
-  T *Ps = Gs + a.cn;
-  // Gs: right-hand side DH^2 f of the direct coarsest solve; Ps: its 1024
-  // partial sums
-  const int tid = threadIdx.x;
+  const TailScratch<T> s(base, a);
+  const int tid = threadIdx.x, last = a.nlev - 1;
   const T relax = (T)a.relax;
-  // Global loads through address-space-1 pointers, so the compiler may keep
-  // them in flight across the LDS stores.  The entry level's right-hand side
-  // is loaded first, together with the first level's coefficients.
-  typedef const __attribute__((address_space(1))) T GT;
-  const TailLevel &L0 = a.lv[0];
-  T fv[2];
-  bool fin[2];
-#pragma unroll
-  for (int it = 0; it < 2; it++) {
-    // clamped indices: every load is issued, unused values are dropped at
-    // the LDS store
-    const int n0 = L0.N * L0.K;
-    const int idx = tid + it * TAIL_THREADS;
-    const int ii = idx < n0 ? idx : n0 - 1;
-    const int j = ii / L0.K, k = ii - j * L0.K;
-    const int kc = k < 1 ? 1 : (k > L0.K - 2 ? L0.K - 2 : k);
-    fv[it] = ((GT *)a.f_in)[(size_t)j * L0.P + kc];
-    fin[it] = k == kc;
-  }
-  for (int l = 0; l < a.nlev; l++) {
-    const TailLevel &L = a.lv[l];
-    const TailBufs<T> b = tail_bufs(base, a, l);
-    GT *cx = (GT *)L.cx;
-    GT *cz = (GT *)L.cz;
-    const int nz = (L.N + 1) * L.K, nx = L.N * L.K;
-    T vx[2], vz[2];
-#pragma unroll
-    for (int it = 0; it < 2; it++) {
-      const int idx = tid + it * TAIL_THREADS;
-      const int ii = idx < nz ? idx : nz - 1;
-      const int j = ii / L.K, k = ii - j * L.K;
-      const int jx = j < L.N ? j : L.N - 1;
-      vz[it] = cz[(size_t)j * L.P + k];
-      vx[it] = cx[(size_t)jx * L.P + k];
-    }
-#pragma unroll
-    for (int it = 0; it < 2; it++) {
-      const int idx = tid + it * TAIL_THREADS;
-      if (idx < nz) b.cz[idx] = vz[it];
-      if (idx < nx) b.cx[idx] = vx[it];
-    }
-  }
+  const bool direct = a.minv != nullptr;
+  const TailLevel &L0 = a.lv[0], &LC = a.lv[last];
   {
-    const TailBufs<T> b = tail_bufs(base, a, 0);
-#pragma unroll
-    for (int it = 0; it < 2; it++) {
-      const int idx = tid + it * TAIL_THREADS;
-      if (idx < L0.N * L0.K) {
-        b.u[idx] = T(0);
-        b.f[idx] = fin[it] ? fv[it] : T(0);
-      }
+    T *F = tail_rhs(base, a, 0);
+    for (int i = tid; i < L0.N * L0.K; i += TAIL_THREADS) {
+      const int j = i / L0.K, k = i - j * L0.K;
+      const T v = ((const T *)a.f_in)[(size_t)j * L0.P + k];
+      F[i] = v;
+      if (direct && last == 0 && k >= 1 && k <= L0.K - 2)
+        s.G[j * (L0.K - 2) + k - 1] = (T)L0.DH2 * v;
     }
+  }
+  Quad<T> p;
+  for (int l = 0; l < last; l++) {
+    const TailLevel &L = a.lv[l], &C = a.lv[l + 1];
+    const QTile<T, kTailPlane> t = tail_tile(base, a, l);
+    tail_quad<T, EXACT>(t, p, L, relax);
+    if (p.valid) quad_put(t, p);
+    __syncthreads();
+    tail_quad_rhs(t, p, tail_rhs(base, a, l), L.K);
+    tail_sweep<T, EXACT>(t, p, a.nu_pre, (T)L.DH2, relax);
+    tail_restrict(t, p, s.R, (T)L.DH2, tail_rhs(base, a, l + 1),
+                  direct && l + 1 == last ? s.G : nullptr, (T)C.DH2, C.N, C.K);
+  }
+  if (direct) {
+    TailDirect<T, 0> d;
+    d.fetch(a);
+    if (last == 0) __syncthreads();
+    d.solve(a, s, LC);
+  } else {
+    const QTile<T, kTailPlane> t = tail_tile(base, a, last);
+    tail_quad<T, EXACT>(t, p, LC, relax);
+    if (p.valid) quad_put(t, p);
+    __syncthreads();
+    tail_quad_rhs(t, p, tail_rhs(base, a, last), LC.K);
+    tail_sweep<T, EXACT>(t, p, a.nu_coarse, (T)LC.DH2, relax);
+    tail_put_e(t, p, s.E, LC.N, LC.K);
+    __syncthreads();
+  }
+  for (int l = last - 1; l >= 0; l--) {
+    const TailLevel &L = a.lv[l], &C = a.lv[l + 1];
+    const QTile<T, kTailPlane> t = tail_tile(base, a, l);
+    tail_quad<T, EXACT>(t, p, L, relax);
+    tail_quad_rhs(t, p, tail_rhs(base, a, l), L.K);
+    if (p.valid) {
+      p.u00 = t.p00()[p.id];
+      p.u01 = t.p01()[p.id];
+      p.u10 = t.p10()[p.id];
+      p.u11 = t.p11()[p.id];
+      quad_prolong<T, FULL_TOP>(t, p, s.E, C.N, C.K, C.K, L.N, L.K);
+    }
+    __syncthreads();
+    if (p.valid) quad_put(t, p);
+    __syncthreads();
+    tail_sweep<T, EXACT>(t, p, a.nu_post, (T)L.DH2, relax);
+    tail_put_e(t, p, s.E, L.N, L.K);
+    __syncthreads();
+  }
+  T *eo = reinterpret_cast<T *>(a.e_out);
+  for (int i = tid; i < L0.N * L0.K; i += TAIL_THREADS) {
+    const int j = i / L0.K, k = i - j * L0.K;
+    eo[(size_t)j * L0.P + k] = s.E[i];
+  }
+}
+
+// The tail of the production cycle: one level and the direct coarsest solve.
+// The level's quads stay in registers from the load to the store, and each
+// thread fetches the first kTailAhead of its entries of the coarsest inverse
+// (255^2 floats at 1025^2, from the memory side) before the sweeps.
+template <typename T, bool EXACT>
+__global__ __launch_bounds__(TAIL_THREADS) void k_tail_direct(TailArgs a) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  T *base = reinterpret_cast<T *>(smem);
+  const TailScratch<T> s(base, a);
+  const T relax = (T)a.relax;
+  const bool leave = a.gate && a.gate[0];  // the solve has converged
+  const TailLevel &L = a.lv[0], &C = a.lv[1];
+  const QTile<T, kTailPlane> t = tail_tile(base, a, 0);
+  const T DH2 = (T)L.DH2;
+  Quad<T> q;
+  quad_place(t, q, (int)threadIdx.x, L.N, L.K);
+  if (q.valid)
+    quad_load<T, true>(t, q, (const T *)nullptr, (const T *)a.f_in, (const T *)L.cx,
+                       (const T *)L.cz, L.N, L.K, L.P, true);
+  TailDirect<T, kTailAhead> d;
+  d.fetch(a);
+  if (q.valid) {
+    quad_factors<T, EXACT>(q, relax);
+    quad_put(t, q);
   }
   __syncthreads();
-  for (int l = 0; l < a.nlev; l++) {
-    const TailLevel &L = a.lv[l];
-    const T DH2 = (T)L.DH2;
-    const TailBufs<T> Bl = tail_bufs(base, a, l);
-    if (l == a.nlev - 1) {
-      if (a.minv) {
-        // e = B^{-1} (DH^2 f), rows summed in column order; Gs was filled by
-        // the restriction onto this level unless it is the entry level
-        const float *minv = reinterpret_cast<const float *>(a.minv);
-        const int W = L.K - 2;
-        if (l == 0) {
-          for (int i = tid; i < a.cn; i += blockDim.x) {
-            const int j = i / W, k = i - j * W + 1;
-            Gs[i] = DH2 * Bl.f[j * L.K + k];
-          }
-          __syncthreads();
-        }
-        coarse_matvec<T>(minv, Gs, Ps, a.cn, Bl.u, W, L.K, (size_t)L.K);
-      } else {
-        const bool one_wave = L.N * L.K <= 512;
-        tail_smooth<T, EXACT>(Bl, L.N, L.K, DH2, relax, a.nu_coarse, one_wave);
-      }
-      __syncthreads();
-      break;
-    }
-    tail_smooth<T, EXACT>(Bl, L.N, L.K, DH2, relax, a.nu_pre, false);
-    for (int idx = tid; idx < L.N * L.K; idx += blockDim.x) {
-      const int j = idx / L.K, k = idx - j * L.K;
-      T r = T(0);
-      if (k >= 1 && k <= L.K - 2) {
-        const int jS = (j == 0) ? 1 : j - 1;
-        const int jN = (j == L.N - 1) ? L.N - 2 : j + 1;
-        const T m1 = Bl.cx[idx], m2 = Bl.cx[idx + 1], m3 = Bl.cz[idx],
-                m4 = Bl.cz[idx + L.K];
-        const T *u = Bl.u;
-        r = Bl.f[idx] - (m1 * u[idx - 1] + m2 * u[idx + 1] + m3 * u[jS * L.K + k] +
-                           m4 * u[jN * L.K + k] - (m1 + m2 + m3 + m4) * u[idx]) /
-                              DH2;
-      }
-      Rs[idx] = r;
-    }
-    __syncthreads();
-    const TailLevel &C = a.lv[l + 1];
-    const TailBufs<T> Bc = tail_bufs(base, a, l + 1);
-    // onto the coarsest level of a direct solve: also its right-hand side
-    const bool direct = a.minv && l + 1 == a.nlev - 1;
-    const T DH2c = (T)C.DH2;
-    for (int idx = tid; idx < C.N * C.K; idx += blockDim.x) {
-      const int j = idx / C.K, k = idx - j * C.K;
-      T v = T(0);
-      if (k >= 1 && k <= C.K - 2) {
-        const int jS = (j == 0) ? 1 : 2 * j - 1;
-        const int jN = (j == C.N - 1) ? 2 * j - 1 : 2 * j + 1;
-        const T *rc = Rs + (2 * j) * L.K;
-        const T *rs = Rs + jS * L.K;
-        const T *rn = Rs + jN * L.K;
-        const int kf = 2 * k;
-        v = T(0.0625) *
-            (T(4.0) * rc[kf] + T(2.0) * rc[kf - 1] + T(2.0) * rc[kf + 1] +
-             T(2.0) * rs[kf] + T(2.0) * rn[kf] + rs[kf - 1] + rs[kf + 1] +
-             rn[kf - 1] + rn[kf + 1]);
-        if (direct) Gs[j * (C.K - 2) + (k - 1)] = DH2c * v;
-      }
-      Bc.f[idx] = v;
-      Bc.u[idx] = T(0);
-    }
-    __syncthreads();
+  if (leave) return;
+  tail_sweep<T, EXACT>(t, q, a.nu_pre, DH2, relax);
+  tail_restrict(t, q, s.R, DH2, tail_rhs(base, a, 1), s.G, (T)C.DH2, C.N, C.K);
+  d.solve(a, s, C);
+  if (q.valid) {
+    quad_prolong<T, true>(t, q, s.E, C.N, C.K, C.K, L.N, L.K);
+    quad_put(t, q);
   }
-  for (int l = a.nlev - 2; l >= 0; l--) {
-    const TailLevel &L = a.lv[l];
-    const TailLevel &C = a.lv[l + 1];
-    const TailBufs<T> Bl = tail_bufs(base, a, l), Bc = tail_bufs(base, a, l + 1);
-    const int jmax = FULL_TOP ? C.N : C.N - 1;
-    for (int idx = tid; idx < jmax * (C.K - 1); idx += blockDim.x) {
-      const int j = idx / (C.K - 1), k = idx - j * (C.K - 1);
-      const T *ec = Bc.u + j * C.K + k;
-      T *uf = Bl.u + (2 * j) * L.K + 2 * k;
-      const T e00 = ec[0], e01 = ec[1];
-      uf[0] += e00;
-      uf[1] += T(0.5) * (e00 + e01);
-      if (!FULL_TOP || j < C.N - 1) {
-        const T e10 = ec[C.K], e11 = ec[C.K + 1];
-        T *uf1 = uf + L.K;
-        uf1[0] += T(0.5) * (e00 + e10);
-        uf1[1] += T(0.25) * (e00 + e01 + e10 + e11);
-      }
-    }
-    __syncthreads();
-    tail_smooth<T, EXACT>(Bl, L.N, L.K, (T)L.DH2, relax, a.nu_post, false);
-  }
-  {
-    const TailLevel &L0 = a.lv[0];
-    T *eo = reinterpret_cast<T *>(a.e_out);
-    const T *u0 = tail_bufs(base, a, 0).u;
-    for (int idx = tid; idx < L0.N * L0.K; idx += blockDim.x) {
-      const int j = idx / L0.K, k = idx - j * L0.K;
-      eo[(size_t)j * L0.P + k] = u0[idx];
-    }
+  __syncthreads();
+  tail_sweep<T, EXACT>(t, q, a.nu_post, DH2, relax);
+  if (q.valid) {
+    int j, k;
+    quad_rc(t, q.id, j, k);
+    quad_store(q, j, k, reinterpret_cast<T *>(a.e_out), L.N, L.K, L.P);
   }
 }
 
@@ -1121,8 +1138,8 @@ template <typename T>
 static size_t tail_lds_bytes(const qdeq_ctx *c, int lt) {
   size_t n = 0;
   for (int l = lt; l < c->L; l++) n += tail_level_words(c->lv[l].N, c->lv[l].K);
-  const size_t nr = (size_t)c->lv[lt].N * c->lv[lt].K;
-  n += nr > (size_t)c->coarse_n ? nr : (size_t)c->coarse_n;
+  n += tail_plane_words(c->lv[lt].K);  // residuals
+  n += (size_t)c->lv[lt].N * c->lv[lt].K;           // corrections
   n += c->coarse_n;  // right-hand side of the direct coarsest solve
   n += 1024;         // its partial sums
   return n * sizeof(T);
@@ -1331,8 +1348,13 @@ static void launch_tail(qdeq_ctx *c, LevelBufs<T> *B, int lt) {
   a.cn = c->coarse_n;
   a.minv = c->coarse_n > 0 ? (const void *)c->cinv32 : nullptr;
   a.gate = c->gate_ptr;
-  hipLaunchKernelGGL((k_tail<T, EXACT, FULL_TOP>), dim3(1), dim3(TAIL_THREADS),
-                     tail_lds_bytes<T>(c, lt), c->stream, a);
+  const size_t lds = tail_lds_bytes<T>(c, lt);
+  if (FULL_TOP && a.nlev == 2 && a.minv)
+    hipLaunchKernelGGL((k_tail_direct<T, EXACT>), dim3(1), dim3(TAIL_THREADS), lds,
+                       c->stream, a);
+  else
+    hipLaunchKernelGGL((k_tail<T, EXACT, FULL_TOP>), dim3(1), dim3(TAIL_THREADS), lds,
+                       c->stream, a);
 }
 
 // Fast V-cycle for the FP64 solve (level 0 = the displacement, f = 0) or
@@ -1802,6 +1824,8 @@ int tiled_setup(qdeq_ctx *c) {
     SETA((k_up<float, true, false, PROL_REF, UP_ADD64, S>));
     SETA((k_up<float, true, false, PROL_NONE, UP_ADD64, S>));
   });
+  SETA((k_tail_direct<double, true>));
+  SETA((k_tail_direct<float, false>));
   SETA((k_tail<double, true, true>));
   SETA((k_tail<float, false, true>));
   SETA((k_tail<double, true, false>));
