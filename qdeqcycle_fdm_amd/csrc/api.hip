@@ -731,14 +731,11 @@ enum {
   RK_DONE
 };
 
-// Host readback of n ints of flags (and the embedded error) + an event
-static int rk_readback(qdeq_ctx *c, bool toterr) {
+// Host readback of the NaN flag + an event
+static int rk_readback(qdeq_ctx *c) {
   RkMachine &r = c->rk;
   if (!r.ev) QDEQ_HIP(c, hipEventCreateWithFlags(&r.ev, hipEventDisableTiming));
   QDEQ_HIP(c, hipGetLastError());
-  if (toterr)
-    QDEQ_HIP(c, hipMemcpyAsync(c->scal_host + SC_TOTERR, c->scal + SC_TOTERR,
-                               sizeof(double), hipMemcpyDeviceToHost, c->stream));
   QDEQ_HIP(c, hipMemcpyAsync(c->flags_host, c->flags, sizeof(int),
                              hipMemcpyDeviceToHost, c->stream));
   QDEQ_HIP(c, hipEventRecord(r.ev, c->stream));
@@ -823,7 +820,7 @@ static int rk_advance(qdeq_ctx *c, bool block, int *done) {
         if (r.steps_left <= 0 || !(c->t < p.tmax)) {
           if (r.spec)
             return set_error(c, QDEQ_ERR_STATE, "a stage is queued for a step that does not run");
-          if ((st = rk_readback(c, false))) return st;
+          if ((st = rk_readback(c))) return st;
           r.phase = RK_WAIT_END;
           break;
         }
@@ -852,6 +849,7 @@ static int rk_advance(qdeq_ctx *c, bool block, int *done) {
           // launched ahead behind the previous solve, which converged with
           // the work already queued: take it over
           c->mg = c->mg_next;
+          c->mg_next.stop_due = false;  // moved with it
           c->mb_page = c->mg.page;
           c->spec_pending = false;
           c->spec_taken++;
@@ -883,7 +881,7 @@ static int rk_advance(qdeq_ctx *c, bool block, int *done) {
           // stage s + 1 queued behind this solve: the fault update of stage
           // s with stage s + 1's state, its start and first batch, all
           // gated on this solve's outcome
-          launch_update_stage(c, r.s, c->gate);
+          launch_update_stage(c, r.s, c->gate, mg_take_stop(c, c->mg));
           const int key = c->solve_key;
           c->solve_key = r.s + 1;
           st = mg_begin_spec(c);
@@ -896,7 +894,7 @@ static int rk_advance(qdeq_ctx *c, bool block, int *done) {
           // state, start and first batch, with the dt the step will hand on
           double dt = step_finish_dt(c);
           if (c->t + dt > p.tmax) dt = p.tmax - c->t;
-          launch_update_next(c, c->t, dt, c->gate);
+          launch_update_next(c, c->t, dt, c->gate, mg_take_stop(c, c->mg));
           const int key = c->solve_key;
           c->solve_key = 2;
           st = mg_begin_spec(c);
@@ -947,13 +945,12 @@ static int rk_advance(qdeq_ctx *c, bool block, int *done) {
             r.phase = RK_STAGE_BEGIN;
           } else {
             launch_combine(c);
-            if ((st = rk_readback(c, true))) return st;
+            QDEQ_HIP(c, hipGetLastError());
             if (accept_spec_allowed(c)) {
-              // the accepted case queued behind the readback, gated on the
+              // the accepted case queued behind it, gated on the
               // combination's own accept decision (gate[7]): the commit, the final
               // stage 1's state, and that solve's start and first batch
-              launch_commit(c, c->t + c->dt, c->gate);
-              launch_stage(c, 1, c->gate);
+              launch_commit_stage(c, c->t + c->dt, c->gate);
               const int key = c->solve_key;
               c->solve_key = 8 + 1;
               st = mg_begin_spec(c, 7);
@@ -964,7 +961,7 @@ static int rk_advance(qdeq_ctx *c, bool block, int *done) {
             r.phase = RK_WAIT_COMBINE;
           }
         } else if (!c->rk_ready) {
-          if ((st = rk_readback(c, false))) return st;
+          if ((st = rk_readback(c))) return st;
           r.phase = RK_WAIT_FIRST;
         } else {
           r.phase = RK_STEP_FINISH;
@@ -979,10 +976,11 @@ static int rk_advance(qdeq_ctx *c, bool block, int *done) {
         r.phase = RK_STEP_BEGIN;
         break;
       case RK_WAIT_COMBINE: {
-        if ((st = rk_readback_ready(c, block, &ready))) return st;
+        if ((st = mg_combine_ready(c, block, &ready))) return st;
         if (!ready) return QDEQ_OK;
+        c->flags_host[0] = (int)c->mbox_host[MB_FLAG];
         if ((st = check_flags(c))) return st;
-        c->totErr = c->scal_host[SC_TOTERR];
+        c->totErr = c->scal_host[SC_TOTERR] = c->mbox_host[MB_ERR];
         bool accept = c->totErr < p.totTol;
         if (r.spec && !accept) {
           // rejected on the device too: the work queued for the accepted
@@ -990,6 +988,7 @@ static int rk_advance(qdeq_ctx *c, bool block, int *done) {
           r.spec = false;
           c->spec_pending = false;
           c->spec_abandoned++;
+          mg_flush_stop(c, c->mg_next);
         }
         if (!accept) {
           c->dt = qdeq_compute_step_size(c->it, c->dt, p.mindt, p.maxdt, c->totErr,

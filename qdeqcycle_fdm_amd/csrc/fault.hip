@@ -224,14 +224,11 @@ __device__ inline void stage_node_in(int k, int s, double dt, double t, double r
 }
 
 // tdt: t and dt of the attempt on the device
-// go: launched ahead of the accept decision, it runs only if the attempt was
-// accepted on the device (go[7] == 1, written by k_combine)
 __global__ void k_stage(int s, const double *tdt, double ratio, double Vini,
                         const double *slip, const double *psi,
                         const double *ss, double *const *FV,
                         double *const *Fd, double *Ys, double *Yp, double *u,
-                        int nk, int K, int P, const int *go) {
-  if (go && go[7] != 1) return;
+                        int nk, int K, int P) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x + 1;
   if (k > nk) return;
   stage_node(k, s, tdt[1], tdt[0], ratio, Vini, slip, psi, ss, FV, Fd, Ys, Yp, u, K,
@@ -240,59 +237,91 @@ __global__ void k_stage(int s, const double *tdt, double ratio, double Vini,
 
 // Fault update after a stage solve: Ts from the compact u (columns 0..3 are
 // the fault and its three neighbours), NR for V from the stage's previous
-// rate (zeroed, odeSolver.cpp:1484-1488), then dpsi.
-// Returns the node's new rate and state rate (also stored).
-struct NodeRates {
-  double V, dpsi;
-};
-__device__ inline NodeRates update_node(int k, const double *u, int P,
-                                        const double *mu_f, const double *tau_n0,
-                                        const double *Yp, const double *a,
-                                        const double *b, const double *eta, double V0,
-                                        double f0, double L, double c0, double c1,
-                                        double c2, double c3, double *Ts, double *Tn,
-                                        double *V, double *dpsi, int *flags) {
-  const double *row = u + (size_t)(k - 1) * P;
-  const double du = c0 * row[0] + c1 * row[1] + c2 * row[2] + c3 * row[3];
-  const double ts = mu_f[k] * du * 1.0e3;
-  const double tn = tau_n0[k];
-  Ts[k] = ts;
-  Tn[k] = tn;
-  const double psi = Yp[k];
-  double Vn;
-  if (!nr_node(ts, tn, psi, a[k], eta[k], V0, V[k], &Vn)) {
-    flags[0] = 1;
-    Vn = V[k];
-  }
-  V[k] = Vn;
-  const double dp = dpsi_node(psi, Vn, b[k], f0, V0, L);
-  dpsi[k] = dp;
-  return NodeRates{Vn, dp};
-}
-
-__global__ void k_fault_update(const double *u, int P, int nk,
-                               const double *mu_f, const double *tau_n0,
-                               const double *Yp, const double *a,
-                               const double *b, const double *eta, double V0,
-                               double f0, double L, double c0, double c1,
-                               double c2, double c3, double *Ts, double *Tn,
-                               double *V, double *dpsi, int *flags) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x + 1;
-  if (k > nk) return;
-  update_node(k, u, P, mu_f, tau_n0, Yp, a, b, eta, V0, f0, L, c0, c1, c2, c3, Ts,
-              Tn, V, dpsi, flags);
-}
-
-// The fault update after the solve of stage s and the stage state and
-// boundary data of stage s + 1, in one launch: both are per node (node k
-// reads and writes only its own row of u and its own entries), so each
-// thread runs the two in order.
+// rate (zeroed, odeSolver.cpp:1484-1488), then dpsi.  The node's inputs are
+// loaded first, so that they are in flight together and with what else the
+// kernel waits for.
 struct UpdateArgs {
   const double *mu_f, *tau_n0, *Yp, *a, *b, *eta;
   double V0, f0, L, c0, c1, c2, c3;
   double *Ts, *Tn, *V, *dpsi;
   int *flags;
 };
+struct NodeIn {
+  double u0, u1, u2, u3, mu, tn, psi, a, b, eta, V;
+};
+__device__ inline NodeIn load_node(int k, const double *u, int P, const UpdateArgs &ua) {
+  const double *row = u + (size_t)(k - 1) * P;
+  return NodeIn{row[0], row[1], row[2], row[3], ua.mu_f[k], ua.tau_n0[k],
+                ua.Yp[k], ua.a[k], ua.b[k], ua.eta[k], ua.V[k]};
+}
+// Returns the node's new rate and state rate (also stored).
+struct NodeRates {
+  double V, dpsi;
+};
+__device__ inline NodeRates update_node(int k, const NodeIn &n, const UpdateArgs &ua) {
+  const double du = ua.c0 * n.u0 + ua.c1 * n.u1 + ua.c2 * n.u2 + ua.c3 * n.u3;
+  const double ts = n.mu * du * 1.0e3;
+  ua.Ts[k] = ts;
+  ua.Tn[k] = n.tn;
+  double Vn;
+  if (!nr_node(ts, n.tn, n.psi, n.a, n.eta, ua.V0, n.V, &Vn)) {
+    ua.flags[0] = 1;
+    Vn = n.V;
+  }
+  ua.V[k] = Vn;
+  const double dp = dpsi_node(n.psi, Vn, n.b, ua.f0, ua.V0, ua.L);
+  ua.dpsi[k] = dp;
+  return NodeRates{Vn, dp};
+}
+
+// Whether the work queued behind a solve goes on: with stop.nb it runs the
+// solve's last stop test itself (k_norm_gate's on one partial per thread, in
+// its order, so every workgroup takes the same decision; workgroup 0 records
+// it; the cap cannot be reached), else it reads the outcome in spec[2].
+// gate[0] is not written here: the start that follows reads gate[2] and sets
+// it.  Ends with a barrier; every thread of the workgroup calls it.
+__device__ inline bool solve_converged(const StopArgs &stop, const int *spec) {
+  if (stop.nb == 0) return !spec || spec[2] == 1;
+  __shared__ double sh[16];
+  const int tid = threadIdx.x;
+  const bool stopped = stop.gate[0] != 0;
+  const int before = stop.gate[2];
+  const double p = tid < stop.nb ? stop.part[tid] : 0.0;
+  const double v = sqrt(block_sum1(0.0 + p, sh));
+  const double thr = stop.rel ? stop.tol * stop.scal[SC_NORM0] : stop.tol;
+  int code = 0;
+  if (isnan(v) || isinf(v))
+    code = 2;
+  else if (!(v > thr))
+    code = 1;
+  if (blockIdx.x == 0 && tid == 0) {
+    const int seq = stop.gate[3] + 1;
+    stop.gate[3] = seq;
+    if (!stopped) {
+      const int cnt = stop.gate[1] + 1;
+      stop.gate[1] = cnt;
+      stop.gate[2] = code;
+      stop.scal[SC_NORM] = v;
+      stop.mb[SC_NORM] = v;
+      stop.mb[MB_COUNT] = (double)cnt;
+      stop.mb[MB_CODE] = (double)code;
+    }
+    __threadfence_system();
+    stop.mb[MB_SEQ] = (double)seq;
+  }
+  return stopped ? before == 1 : code == 1;
+}
+
+__global__ void k_fault_update(const double *u, int P, int nk, UpdateArgs ua) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x + 1;
+  if (k > nk) return;
+  update_node(k, load_node(k, u, P, ua), ua);
+}
+
+// The fault update after the solve of stage s and the stage state and
+// boundary data of stage s + 1, in one launch: both are per node (node k
+// reads and writes only its own row of u and its own entries), so each
+// thread runs the two in order.
 struct StageArgs {
   int s;
   const double *tdt;  // t, dt of the attempt
@@ -303,32 +332,33 @@ struct StageArgs {
   double *Ys, *Yp;
 };
 
-__global__ void k_update_stage(double *u, int nk, int K, int P, UpdateArgs ua,
-                               StageArgs sa, const int *spec) {
-  // launched ahead, behind a solve still in flight: runs only if that solve
-  // ended converged (its outcome in spec[2])
-  if (spec && spec[2] != 1) return;
+__global__ __launch_bounds__(FT) void k_update_stage(double *u, int nk, int K, int P,
+                                                     UpdateArgs ua, StageArgs sa,
+                                                     const int *spec, StopArgs stop) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x + 1;
-  if (k > nk) return;
   // the next stage's inputs that the update leaves unchanged, loaded before
   // it (after its stores the loads could not be issued early: the pointers
   // may alias); the rates of the stage just solved (index s - 1 of FV and
   // Fd, the update's V and dpsi) come from the update itself
   const int s = sa.s;  // 2 .. 6
+  const int kl = min(k, nk);
   const double t = sa.tdt[0], dt = sa.tdt[1];
-  const double sl = sa.slip[k], ps = sa.psi[k], ssk = sa.ss[k];
+  const double sl = sa.slip[kl], ps = sa.psi[kl], ssk = sa.ss[kl];
   double fv[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   double fd[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll
   for (int jj = 1; jj < 5; jj++) {
     if (jj < s - 1) {
-      fv[jj] = sa.FV[jj][k];
-      fd[jj] = sa.Fd[jj][k];
+      fv[jj] = sa.FV[jj][kl];
+      fd[jj] = sa.Fd[jj][kl];
     }
   }
-  const NodeRates r = update_node(k, u, P, ua.mu_f, ua.tau_n0, ua.Yp, ua.a, ua.b, ua.eta,
-                                  ua.V0, ua.f0, ua.L, ua.c0, ua.c1, ua.c2, ua.c3, ua.Ts,
-                                  ua.Tn, ua.V, ua.dpsi, ua.flags);
+  const NodeIn n = load_node(kl, u, P, ua);
+  // launched ahead, behind a solve still in flight: runs only if that solve
+  // ended converged
+  if (!solve_converged(stop, spec)) return;
+  if (k > nk) return;
+  const NodeRates r = update_node(k, n, ua);
 #pragma unroll
   for (int jj = 1; jj < 6; jj++) {
     if (jj == s - 1) {
@@ -345,11 +375,17 @@ __global__ void k_update_stage(double *u, int nk, int K, int P, UpdateArgs ua,
 // queued behind that solve: it runs only if the solve ended converged
 // (spec[2]).  The attempt's t and dt come by value (thread 0 also stores
 // them for the later stages), so no thread reads what another one writes.
-__global__ void k_update_next(double *u, int nk, int nz, int K, int P, UpdateArgs ua,
-                              StageArgs sa, double t, double dt, double *tdt,
-                              const int *spec) {
-  if (spec[2] != 1) return;
+__global__ __launch_bounds__(FT) void k_update_next(double *u, int nk, int nz, int K, int P,
+                                                    UpdateArgs ua, StageArgs sa, double t,
+                                                    double dt, double *tdt,
+                                                    const int *spec, StopArgs stop) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  // stage 2 reads slip, psi, SlipShift (loaded before the update, as in
+  // k_update_stage) and F_1, the rates the update forms
+  const int kl = min(max(k, 1), nk);
+  const double sl = sa.slip[kl], ps = sa.psi[kl], ssk = sa.ss[kl];
+  const NodeIn n = load_node(kl, u, P, ua);
+  if (!solve_converged(stop, spec)) return;
   if (k == 0) {
     tdt[0] = t;
     tdt[1] = dt;
@@ -360,12 +396,7 @@ __global__ void k_update_next(double *u, int nk, int nz, int K, int P, UpdateArg
     sa.Fd[s][k] = 0.0;
   }
   if (k < 1 || k > nk) return;
-  // stage 2 reads slip, psi, SlipShift (loaded before the update, as in
-  // k_update_stage) and F_1, the rates the update forms
-  const double sl = sa.slip[k], ps = sa.psi[k], ssk = sa.ss[k];
-  const NodeRates r = update_node(k, u, P, ua.mu_f, ua.tau_n0, ua.Yp, ua.a, ua.b, ua.eta,
-                                  ua.V0, ua.f0, ua.L, ua.c0, ua.c1, ua.c2, ua.c3, ua.Ts,
-                                  ua.Tn, ua.V, ua.dpsi, ua.flags);
+  const NodeRates r = update_node(k, n, ua);
   double fv[6] = {0.0, r.V, 0.0, 0.0, 0.0, 0.0};
   double fd[6] = {0.0, r.dpsi, 0.0, 0.0, 0.0, 0.0};
   stage_node_in(k, 2, dt, t, sa.ratio, sa.Vini, sl, ps, ssk, fv, fd, sa.Ys, sa.Yp, u, K,
@@ -389,11 +420,16 @@ __global__ void k_zero_rates(double *const *FV, double *const *Fd, int nz,
 // y3 (embedded, hb weights) and y4 (b weights, propagated) and the error
 // norm (odeSolver.cpp:1569-1595, computeError 1211-1238).  One block; the
 // squared differences are summed by one lane in node order, so totErr has
-// the reference's summation order.
+// the reference's summation order.  That chain of dependent FP64 additions
+// bounds the kernel (about 10 ns a node, 14 us at 1025 nodes, whichever way
+// its operands are fed).
+// The error, the NaN flag and the sequence number go to the mailbox, where
+// the host waits for them.
 __global__ __launch_bounds__(1024) void k_combine(
     const double *tdt, const double *slip, const double *psi, double *const *FV,
     double *const *Fd, double *y3s, double *y3p, double *y4s, double *y4p,
-    int nk, double *out, int *gate, double totTol) {
+    int nk, double *out, int *gate, double totTol, const int *flags, double *mb,
+    double seq) {
   __shared__ double s1[1024], s2[1024];
   const int tid = threadIdx.x;
   const double dt = tdt[1];
@@ -446,6 +482,10 @@ __global__ __launch_bounds__(1024) void k_combine(
     // the accept test the host applies first (odeSolver.cpp:1596), for
     // work launched ahead of the host's decision
     gate[7] = err < totTol ? 1 : 0;
+    mb[MB_ERR] = err;
+    mb[MB_FLAG] = (double)flags[0];
+    __threadfence_system();
+    mb[MB_RKSEQ] = seq;
   }
 }
 
@@ -453,8 +493,7 @@ __global__ __launch_bounds__(1024) void k_combine(
 // becomes t_new = t + dt.
 __global__ void k_commit(double *slip, double *psi, const double *y4s,
                          const double *y4p, double *V1, double *d1, int nk,
-                         double *tdt, double t_new, const int *go) {
-  if (go && go[7] != 1) return;  // launched ahead: only if accepted
+                         double *tdt, double t_new) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x + 1;
   if (k == 1) tdt[0] = t_new;
   if (k > nk) return;
@@ -462,6 +501,29 @@ __global__ void k_commit(double *slip, double *psi, const double *y4s,
   psi[k] = y4p[k];
   V1[k] = 0.0;
   d1[k] = 0.0;
+}
+
+// k_commit and the state and boundary data of the final stage 1 (stage_node
+// with s = 1 at the new time) in one launch, queued ahead of the accept
+// decision: it runs only if the attempt was accepted on the device (go[7] ==
+// 1, written by k_combine).
+__global__ void k_commit_stage(double *slip, double *psi, const double *y4s,
+                               const double *y4p, double *V1, double *d1, int nk,
+                               double *tdt, double t_new, double ratio, double Vini,
+                               const double *ss, double *Ys, double *Yp, double *u, int K,
+                               int P, const int *go) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x + 1;
+  const int kl = min(k, nk);
+  const double ys = y4s[kl], yp = y4p[kl], ssk = ss[kl], dt = tdt[1];
+  if (go[7] != 1) return;
+  if (k == 1) tdt[0] = t_new;
+  if (k > nk) return;
+  slip[k] = ys;
+  psi[k] = yp;
+  V1[k] = 0.0;
+  d1[k] = 0.0;
+  const double none[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+  stage_node_in(k, 1, dt, t_new, ratio, Vini, ys, yp, ssk, none, none, Ys, Yp, u, K, P);
 }
 
 // maxval (fault.cpp:22-52) of V and Ts.  One block.
@@ -552,46 +614,45 @@ static double *const *dev_FV(qdeq_ctx *c) {
 }
 static double *const *dev_Fd(qdeq_ctx *c) { return dev_FV(c) + 7; }
 
-void launch_stage(qdeq_ctx *c, int s, const int *go) {
+void launch_stage(qdeq_ctx *c, int s) {
   FaultBufs &f = c->fb;
   hipLaunchKernelGGL(k_stage, nodes_grid(c->cfg.nk), dim3(FT), 0, c->stream, s,
                      c->scal + SC_T, kC[s], c->cfg.Vini, f.slip, f.psi, f.slip_shift,
                      dev_FV(c), dev_Fd(c), f.Ys[s], f.Yp[s], c->d[0].u,
-                     c->cfg.nk, c->lv[0].K, c->lv[0].P, go);
+                     c->cfg.nk, c->lv[0].K, c->lv[0].P);
+}
+
+static UpdateArgs update_args(const qdeq_ctx *c, int s) {
+  const FaultBufs &f = c->fb;
+  return UpdateArgs{f.mu_f, f.tau_n0, f.Yp[s], f.a, f.b, f.eta, c->cfg.V0,
+                    c->cfg.f0, c->cfg.L, c->c_stress[0], c->c_stress[1],
+                    c->c_stress[2], c->c_stress[3], f.Ts, f.Tn, f.FV[s], f.Fd[s],
+                    c->flags};
 }
 
 void launch_fault_update(qdeq_ctx *c, int s) {
-  FaultBufs &f = c->fb;
   hipLaunchKernelGGL(k_fault_update, nodes_grid(c->cfg.nk), dim3(FT), 0,
-                     c->stream, c->d[0].u, c->lv[0].P, c->cfg.nk, f.mu_f,
-                     f.tau_n0, f.Yp[s], f.a, f.b, f.eta, c->cfg.V0, c->cfg.f0,
-                     c->cfg.L, c->c_stress[0], c->c_stress[1], c->c_stress[2],
-                     c->c_stress[3], f.Ts, f.Tn, f.FV[s], f.Fd[s], c->flags);
+                     c->stream, c->d[0].u, c->lv[0].P, c->cfg.nk, update_args(c, s));
 }
 
-void launch_update_stage(qdeq_ctx *c, int s, const int *spec) {
+void launch_update_stage(qdeq_ctx *c, int s, const int *spec, const StopArgs &stop) {
   FaultBufs &f = c->fb;
-  const UpdateArgs ua{f.mu_f, f.tau_n0, f.Yp[s], f.a, f.b, f.eta, c->cfg.V0,
-                      c->cfg.f0, c->cfg.L, c->c_stress[0], c->c_stress[1],
-                      c->c_stress[2], c->c_stress[3], f.Ts, f.Tn, f.FV[s], f.Fd[s],
-                      c->flags};
+  const UpdateArgs ua = update_args(c, s);
   const StageArgs sa{s + 1, c->scal + SC_T, kC[s + 1], c->cfg.Vini, f.slip, f.psi,
                      f.slip_shift, dev_FV(c), dev_Fd(c), f.Ys[s + 1], f.Yp[s + 1]};
   hipLaunchKernelGGL(k_update_stage, nodes_grid(c->cfg.nk), dim3(FT), 0, c->stream,
-                     c->d[0].u, c->cfg.nk, c->lv[0].K, c->lv[0].P, ua, sa, spec);
+                     c->d[0].u, c->cfg.nk, c->lv[0].K, c->lv[0].P, ua, sa, spec, stop);
 }
 
-void launch_update_next(qdeq_ctx *c, double t, double dt, const int *spec) {
+void launch_update_next(qdeq_ctx *c, double t, double dt, const int *spec,
+                        const StopArgs &stop) {
   FaultBufs &f = c->fb;
-  const UpdateArgs ua{f.mu_f, f.tau_n0, f.Yp[1], f.a, f.b, f.eta, c->cfg.V0,
-                      c->cfg.f0, c->cfg.L, c->c_stress[0], c->c_stress[1],
-                      c->c_stress[2], c->c_stress[3], f.Ts, f.Tn, f.FV[1], f.Fd[1],
-                      c->flags};
+  const UpdateArgs ua = update_args(c, 1);
   const StageArgs sa{2, c->scal + SC_T, kC[2], c->cfg.Vini, f.slip, f.psi,
                      f.slip_shift, dev_FV(c), dev_Fd(c), f.Ys[2], f.Yp[2]};
   hipLaunchKernelGGL(k_update_next, nodes_grid(c->nz), dim3(FT), 0, c->stream,
                      c->d[0].u, c->cfg.nk, c->nz, c->lv[0].K, c->lv[0].P, ua, sa, t,
-                     dt, c->scal + SC_T, spec);
+                     dt, c->scal + SC_T, spec, stop);
 }
 
 void launch_zero_stage_rates(qdeq_ctx *c, double t, double dt) {
@@ -603,14 +664,23 @@ void launch_combine(qdeq_ctx *c) {
   FaultBufs &f = c->fb;
   hipLaunchKernelGGL(k_combine, dim3(1), dim3(1024), 0, c->stream, c->scal + SC_T, f.slip,
                      f.psi, dev_FV(c), dev_Fd(c), f.y3s, f.y3p, f.y4s, f.y4p,
-                     c->cfg.nk, c->scal + SC_TOTERR, c->gate, c->cfg.totTol);
+                     c->cfg.nk, c->scal + SC_TOTERR, c->gate, c->cfg.totTol, c->flags,
+                     c->mbox_dev, (double)++c->rk.seq);
 }
 
-void launch_commit(qdeq_ctx *c, double t_new, const int *go) {
+void launch_commit(qdeq_ctx *c, double t_new) {
   FaultBufs &f = c->fb;
   hipLaunchKernelGGL(k_commit, nodes_grid(c->cfg.nk), dim3(FT), 0, c->stream,
                      f.slip, f.psi, f.y4s, f.y4p, f.FV[1], f.Fd[1], c->cfg.nk,
-                     c->scal + SC_T, t_new, go);
+                     c->scal + SC_T, t_new);
+}
+
+void launch_commit_stage(qdeq_ctx *c, double t_new, const int *go) {
+  FaultBufs &f = c->fb;
+  hipLaunchKernelGGL(k_commit_stage, nodes_grid(c->cfg.nk), dim3(FT), 0, c->stream,
+                     f.slip, f.psi, f.y4s, f.y4p, f.FV[1], f.Fd[1], c->cfg.nk,
+                     c->scal + SC_T, t_new, kC[1], c->cfg.Vini, f.slip_shift, f.Ys[1],
+                     f.Yp[1], c->d[0].u, c->lv[0].K, c->lv[0].P, go);
 }
 
 void launch_maxima(qdeq_ctx *c) {

@@ -837,6 +837,30 @@ static void launch_plain_dev_start(qdeq_ctx *c, bool fuse) {
                      c->scal, mb_dev(c), c->gate, c->spec_launch ? c->spec_go : 0);
 }
 
+StopArgs mg_take_stop(qdeq_ctx *c, MgSolve &m) {
+  StopArgs a;
+  if (!m.stop_due) return a;
+  m.stop_due = false;
+  a.part = c->partial;
+  a.nb = norm_parts(c);
+  a.rel = c->cfg.tol_mode == QDEQ_TOL_REL ? 1 : 0;
+  a.tol = c->cfg.tol;
+  a.scal = c->scal;
+  a.mb = c->mbox_dev + m.page * SC_COUNT;
+  a.gate = c->gate;
+  c->folded_tests++;
+  return a;
+}
+
+void mg_flush_stop(qdeq_ctx *c, MgSolve &m) {
+  if (!m.stop_due) return;
+  m.stop_due = false;
+  hipLaunchKernelGGL(k_norm_gate, dim3(1), dim3(NORM_THREADS), 0, c->stream, c->partial,
+                     norm_parts(c), c->scal, c->mbox_dev + m.page * SC_COUNT, c->gate,
+                     c->cfg.tol_mode == QDEQ_TOL_REL ? 1 : 0, c->cfg.tol,
+                     c->cfg.max_vcycles);
+}
+
 // V-cycles of the first batch of a solve: what the same RK43 stage needed in
 // the previous step (c->last_it_key), else what the last solve needed.
 static int first_batch(const qdeq_ctx *c) {
@@ -850,7 +874,10 @@ int mg_begin(qdeq_ctx *c) {
   int st = ensure_graph(c);
   if (st != QDEQ_OK) return st;
   MgSolve &m = c->mg;
-  // no other solve is in flight: mailbox page 0
+  // no other solve is in flight: mailbox page 0 (a stop test that an error
+  // left due still takes its step of the sequence)
+  mg_flush_stop(c, c->mg);
+  mg_flush_stop(c, c->mg_next);
   m.page = 0;
   c->mb_page = 0;
   m.ir = c->cfg.precision == QDEQ_PREC_FP32_IR;
@@ -945,6 +972,8 @@ int mg_begin_stage(qdeq_ctx *c, int kind, int s) {
   int st = ensure_graph(c);
   if (st != QDEQ_OK) return st;
   MgSolve &m = c->mg;
+  mg_flush_stop(c, c->mg);
+  mg_flush_stop(c, c->mg_next);
   m.page = 0;
   c->mb_page = 0;
   m.ir = c->cfg.precision == QDEQ_PREC_FP32_IR;
@@ -1037,10 +1066,10 @@ static int mg_finish(qdeq_ctx *c, int st) {
   return st;
 }
 
-// Non-blocking (or blocking) check that the batch's last V-cycle has been
-// seen by the device: mb[MB_SEQ] reaches the batch's sequence number.
-static int seq_check(qdeq_ctx *c, long long target, bool block, int *ready) {
-  volatile double *p = reinterpret_cast<volatile double *>(mb_host(c)) + MB_SEQ;
+// Non-blocking (or blocking) check that a mailbox sequence number (the batch's
+// last V-cycle seen by the device in mb[MB_SEQ]) has reached its target.
+static int mailbox_check(qdeq_ctx *c, volatile double *p, long long target, bool block,
+                         int *ready, const char *lost) {
   for (;;) {
     if ((long long)*p >= target) {
       std::atomic_thread_fence(std::memory_order_acquire);
@@ -1061,12 +1090,23 @@ static int seq_check(qdeq_ctx *c, long long target, bool block, int *ready) {
           c->mb_idle_since = now;
         } else if (now - c->mb_idle_since > std::chrono::milliseconds(200)) {
           c->mb_idle = false;
-          return set_error(c, QDEQ_ERR_STATE, "V-cycle sequence was not written");
+          return set_error(c, QDEQ_ERR_STATE, lost);
         }
       }
     }
     if (!block) return QDEQ_OK;
   }
+}
+
+static int seq_check(qdeq_ctx *c, long long target, bool block, int *ready) {
+  volatile double *p = reinterpret_cast<volatile double *>(mb_host(c)) + MB_SEQ;
+  return mailbox_check(c, p, target, block, ready, "V-cycle sequence was not written");
+}
+
+// The same for the mailbox's last combination (page 0).
+int mg_combine_ready(qdeq_ctx *c, bool block, int *ready) {
+  volatile double *p = reinterpret_cast<volatile double *>(c->mbox_host) + MB_RKSEQ;
+  return mailbox_check(c, p, c->rk.seq, block, ready, "combination was not written");
 }
 
 // Launches up to k V-cycles back to back; each skips once the solve has
@@ -1080,7 +1120,7 @@ static int launch_batch_of(qdeq_ctx *c, MgSolve &m, int k, bool allow_sample) {
   m.sample = false;
   // the stop test of every V-cycle but the batch's last (and one that could
   // reach the V-cycle cap) runs in the next V-cycle's level-0 down kernel
-  const bool fold = fold_fits(c);
+  const bool fold = fold_fits(c), defer = defer_fits(c);
   bool folded = false;
   struct FoldReset {  // also on an error return: no later launch folds
     qdeq_ctx *c;
@@ -1094,9 +1134,11 @@ static int launch_batch_of(qdeq_ctx *c, MgSolve &m, int k, bool allow_sample) {
                         use_tiled(c) && (c->timed_seq++ % kTimingEvery) == 0;
     m.launched++;
     c->fold_next = folded;
-    c->skip_gate = fold && i + 1 < k && m.launched < c->cfg.max_vcycles;
-    folded = c->skip_gate;
+    folded = fold && i + 1 < k && m.launched < c->cfg.max_vcycles;
     if (folded) c->folded_tests++;
+    // the last one's may run in the fault update behind the solve
+    m.stop_due = defer && i + 1 == k && m.launched < c->cfg.max_vcycles;
+    c->skip_gate = folded || m.stop_due;
     if (sample) {
       c->emit_events = true;
       c->gate_ptr = c->gate;
@@ -1139,6 +1181,7 @@ int mg_poll(qdeq_ctx *c, bool block, int *done) {
   const double *mb = mb_host(c);
   *done = 0;
   int st = QDEQ_OK, ready;
+  mg_flush_stop(c, m);
   if (m.phase == 1) {
     if ((st = mbox_check(c, SC_NORM, block, &ready)) || !ready) goto out;
     if (c->cfg.tol_mode == QDEQ_TOL_REL &&
@@ -1175,6 +1218,7 @@ int mg_poll(qdeq_ctx *c, bool block, int *done) {
     }
     QDEQ_HIP(c, hipMemsetAsync(c->gate, 0, 3 * sizeof(int), c->stream));
     if ((st = launch_batch(c, batch_size(c, m.delta, m.thr)))) goto out;
+    mg_flush_stop(c, m);
     m.phase = 2;
     if (!block) return QDEQ_OK;
   }
@@ -1228,10 +1272,12 @@ int mg_poll(qdeq_ctx *c, bool block, int *done) {
     // not there yet: another batch sized from the residual left.  A solve
     // launched ahead behind this one was abandoned and stopped the gate.
     if (c->spec_pending) {
+      mg_flush_stop(c, c->mg_next);
       hipLaunchKernelGGL(k_gate_resume, dim3(1), dim3(1), 0, c->stream, c->gate);
       c->spec_pending = false;
     }
     if ((st = launch_batch(c, batch_size(c, m.delta, m.thr)))) goto out;
+    mg_flush_stop(c, m);
     if (!block) return QDEQ_OK;
   }
 out:

@@ -523,44 +523,24 @@ __global__ __launch_bounds__(TILE_THREADS) void k_down(
   // k_norm_gate's order, so every workgroup takes the same decision
   double fold_p = 0.0;
   if (folding && ltid < sa.nb) fold_p = sa.part[ltid];
-  if (SMODE == START_TEST && threadIdx.y == 0 && !leave) {
-    // wavefront 0: the start norms from the level-0 tiles' partials
-    double a = 0.0, b = 0.0;
-    for (int i = threadIdx.x; i < sa.nb; i += 64) {
-      a += sa.part[i];
-      b += sa.part[kStartCap + i];
-    }
-    a = wave_sum(a);
-    b = wave_sum(b);
-    if (threadIdx.x == 0) {
-      const double du = sqrt(a);
-      const double r0 = sa.rel ? sqrt(b) : du;
-      const double thr = sa.rel ? sa.tol * r0 : sa.tol;
-      int code = 0;
-      if (!(du > thr))
-        code = 1;
-      else if (sa.cap < 1)
-        code = 3;
-      sdec[0] = (double)code;
-      if (blockIdx.x == 0 && blockIdx.y == 0) {
-        sa.scal[SC_NORM] = du;
-        sa.scal[SC_NORM0] = r0;
-        sa.gate[0] = code ? 1 : 0;
-        sa.gate[1] = 0;
-        sa.gate[2] = code;
-        sa.gate[4] = 0;
-        sa.gate[5] = 0;
-        sa.mb[SC_NORM] = du;
-        sa.mb[SC_NORM0] = r0;
-        sa.mb[MB_START] = du;
-        sa.mb[MB_USED] = 0.0;
-        sa.mb[MB_COUNT] = 0.0;
-        sa.mb[MB_CODE] = (double)code;
-        const int seq = sa.gate[3] + 1;
-        sa.gate[3] = seq;
-        __threadfence_system();
-        sa.mb[MB_SEQ] = (double)seq;
+  // the start norms from the level-0 tiles' partials, summed by the whole
+  // workgroup (every workgroup alike), four loads of a thread in flight
+  double v2[2] = {0.0, 0.0};
+  if (SMODE == START_TEST) {
+    for (int i0 = ltid; i0 < sa.nb; i0 += 4 * nthr) {
+      double p[4], b[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int at = min(i0 + i * nthr, sa.nb - 1);
+        p[i] = sa.part[at];
+        b[i] = sa.part[kStartCap + at];
       }
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if (i0 + i * nthr < sa.nb) {
+          v2[0] += p[i];
+          v2[1] += b[i];
+        }
     }
   }
 #pragma unroll
@@ -573,7 +553,10 @@ __global__ __launch_bounds__(TILE_THREADS) void k_down(
     const double w = wave_sum(0.0 + fold_p);
     if ((ltid & 63) == 0) sdec[ltid >> 6] = w;
   }
-  __syncthreads();
+  if (SMODE == START_TEST)
+    block_sums<2>(v2, sdec);  // with the tile's barrier
+  else
+    __syncthreads();
   if (SMODE == START_PARTIALS && sa.spec && wg0) sa.gate[6] = leave ? 0 : 1;
   if (leave) {
     // a folded stop test still takes its step of the mailbox sequence
@@ -588,7 +571,36 @@ __global__ __launch_bounds__(TILE_THREADS) void k_down(
     }
     return;
   }
-  if (SMODE == START_TEST && sdec[0] != 0.0) return;  // no V-cycle needed
+  if (SMODE == START_TEST) {
+    const double du = sqrt(v2[0]);
+    const double r0 = sa.rel ? sqrt(v2[1]) : du;
+    const double thr = sa.rel ? sa.tol * r0 : sa.tol;
+    int code = 0;
+    if (!(du > thr))
+      code = 1;
+    else if (sa.cap < 1)
+      code = 3;
+    if (wg0) {
+      sa.scal[SC_NORM] = du;
+      sa.scal[SC_NORM0] = r0;
+      sa.gate[0] = code ? 1 : 0;
+      sa.gate[1] = 0;
+      sa.gate[2] = code;
+      sa.gate[4] = 0;
+      sa.gate[5] = 0;
+      sa.mb[SC_NORM] = du;
+      sa.mb[SC_NORM0] = r0;
+      sa.mb[MB_START] = du;
+      sa.mb[MB_USED] = 0.0;
+      sa.mb[MB_COUNT] = 0.0;
+      sa.mb[MB_CODE] = (double)code;
+      const int seq = sa.gate[3] + 1;
+      sa.gate[3] = seq;
+      __threadfence_system();
+      sa.mb[MB_SEQ] = (double)seq;
+    }
+    if (code) return;  // no V-cycle needed
+  }
   if (folding) {
     const double v = sqrt(((sdec[0] + sdec[1]) + sdec[2]) + sdec[3]);
     const double thr = sa.rel ? sa.tol * sa.scal[SC_NORM0] : sa.tol;
@@ -618,7 +630,6 @@ __global__ __launch_bounds__(TILE_THREADS) void k_down(
   if (SMODE == START_PARTIALS) {
     // the start as loaded: residual norm and boundary-data norm partials of
     // the interior points
-    double v2[2] = {0.0, 0.0};
 #pragma unroll
     for (int i = 0; i < S; i++) {
       const Quad<T> &p = q[i];
@@ -1293,18 +1304,28 @@ static void launch_down(qdeq_ctx *c, LevelBufs<T> *B, int l, bool has_f,
                      B[l].u, B[l].r, sa);
 }
 
-// Whether a batch launched kernel by kernel may fold its stop tests into the
-// next V-cycle's level-0 down kernel: the FP64 tiled cycle, at most 256
-// level-0 up tiles (k_norm_gate's threads each sum one partial) and a
-// level-0 down workgroup of four wavefronts or more.
-bool fold_fits(const qdeq_ctx *c) {
-  if (c->fold_off || c->cfg.precision != QDEQ_PREC_FP64 || !use_tiled(c) ||
-      !launch_direct(c) || tail_entry_level(c) < 1)
-    return false;
+// Norm partials of an FP64 V-cycle on the tile kernels: the level-0 tiles of
+// its last launch.
+int norm_parts(const qdeq_ctx *c) {
   const LevelDims &d = c->lv[0];
-  const TileShape dn = tile_shape(c, 0, true), up = tile_shape(c, 0, false);
-  const long nb = (long)((d.K + up.tx - 1) / up.tx) * ((d.N + up.ty - 1) / up.ty);
-  return nb <= 256 && TX_THREADS * dn.tyt >= 256;
+  const TileShape up = use_tiled(c) ? tile_shape(c, 0, false) : c->ref_plan[0].sh;
+  return ((d.K + up.tx - 1) / up.tx) * ((d.N + up.ty - 1) / up.ty);
+}
+
+// Whether a kernel that follows a V-cycle launched kernel by kernel may run
+// its stop test: the FP64 tile kernels and at most 256 norm partials
+// (k_norm_gate's threads each sum one).
+bool defer_fits(const qdeq_ctx *c) {
+  return !c->fold_off && c->cfg.precision == QDEQ_PREC_FP64 && launch_direct(c) &&
+         (use_tiled(c) || use_ref_tiles(c)) && norm_parts(c) <= 256;
+}
+
+// Whether a batch may fold its stop tests into the next V-cycle's level-0
+// down kernel: that of the fast cycle, with a workgroup of four wavefronts or
+// more.
+bool fold_fits(const qdeq_ctx *c) {
+  return defer_fits(c) && use_tiled(c) && tail_entry_level(c) >= 1 &&
+         TX_THREADS * tile_shape(c, 0, true).tyt >= 256;
 }
 
 // Whether the start of the next FP64 solve may be folded into its first

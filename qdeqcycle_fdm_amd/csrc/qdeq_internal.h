@@ -76,6 +76,9 @@ enum {
   MB_CODE = 10,      //   outcome of the last V-cycle (k_norm_gate)
   MB_USED = 11,      //   1 if the solve started from the candidate
   MB_START = 12,     //   residual norm of the start used
+  MB_ERR = 13,       //   embedded error of the last combination
+  MB_FLAG = 14,      //   and the NaN flag then
+  MB_RKSEQ = 15,     //   and its sequence number (these three: page 0)
   SC_COUNT = 16
 };
 
@@ -94,6 +97,19 @@ struct MgSolve {
   double delta = 0, delta0 = 0, r0 = 0, thr = 0;
   long long seq_target = 0;  // sequence number ending the launched batch
   int page = 0;              // mailbox page its kernels write (see mb_dev)
+  // the stop test of its last V-cycle is still to be launched: by the fault
+  // update queued behind the solve (stop_args), or else by mg_flush_stop
+  bool stop_due = false;
+};
+
+// The stop test of a solve's last V-cycle run by another kernel
+// (k_norm_gate's, on at most 256 partials; nb = 0: none).
+struct StopArgs {
+  const double *part = nullptr;
+  int nb = 0, rel = 0;
+  double tol = 0.0;
+  double *scal = nullptr, *mb = nullptr;
+  int *gate = nullptr;
 };
 
 // State of the resumable RK43 driver (api.hip).
@@ -110,6 +126,7 @@ struct RkMachine {
   // for the final stage 1: the next attempt's dt the queued stage 2 used
   double spec_dt = 0.0;
   hipEvent_t ev = nullptr;   // completion of the last host readback
+  long long seq = 0;         // combinations launched (MB_RKSEQ)
 };
 
 }  // namespace qdeq
@@ -281,6 +298,12 @@ int mg_begin(qdeq_ctx *c);
 bool stage_graphs(const qdeq_ctx *c);
 int mg_begin_stage(qdeq_ctx *c, int kind, int s);
 int mg_begin_spec(qdeq_ctx *c, int go = 2);
+// the due stop test of solve m: handed to the kernel launched next (which
+// takes it over), or launched as a kernel of its own
+StopArgs mg_take_stop(qdeq_ctx *c, MgSolve &m);
+void mg_flush_stop(qdeq_ctx *c, MgSolve &m);
+// waits (or checks once) for the combination r.seq to reach the mailbox
+int mg_combine_ready(qdeq_ctx *c, bool block, int *ready);
 int mg_poll(qdeq_ctx *c, bool block, int *done);
 int mg_build_coefficients(qdeq_ctx *c);
 void mg_destroy_graphs(qdeq_ctx *c);
@@ -325,6 +348,8 @@ int tiled_setup(qdeq_ctx *c);
 bool tiles_fit(const qdeq_ctx *c, int tx, int ty);
 bool fused_start_fits(const qdeq_ctx *c);
 bool fold_fits(const qdeq_ctx *c);
+bool defer_fits(const qdeq_ctx *c);
+int norm_parts(const qdeq_ctx *c);
 int autotune_tiles(qdeq_ctx *c, int reps);
 int set_tile_shapes(qdeq_ctx *c, int nlevels, const int *shapes);
 int kernel_breakdown(qdeq_ctx *c, int reps, int *n, double *us);
@@ -481,16 +506,20 @@ void launch_nr(qdeq_ctx *c, const double *Ts, const double *Tn,
 void launch_dpsi(qdeq_ctx *c, const double *psi, const double *V,
                  const double *b, double *dpsi);
 // stage kernels: t and dt from scal[SC_T], scal[SC_DT]
-void launch_stage(qdeq_ctx *c, int s, const int *go = nullptr);
+void launch_stage(qdeq_ctx *c, int s);
 // fault update of stage s and the stage state of s + 1 in one launch
-void launch_update_stage(qdeq_ctx *c, int s, const int *spec = nullptr);
+void launch_update_stage(qdeq_ctx *c, int s, const int *spec = nullptr,
+                         const StopArgs &stop = StopArgs{});
 void launch_fault_update(qdeq_ctx *c, int s);
 // zeroes the stage rates of a new attempt and sets its t, dt on the device
 void launch_zero_stage_rates(qdeq_ctx *c, double t, double dt);
-void launch_update_next(qdeq_ctx *c, double t, double dt, const int *spec);
+void launch_update_next(qdeq_ctx *c, double t, double dt, const int *spec,
+                        const StopArgs &stop);
 void launch_combine(qdeq_ctx *c);
 // accepts y4 and sets the device time to t_new
-void launch_commit(qdeq_ctx *c, double t_new, const int *go = nullptr);
+void launch_commit(qdeq_ctx *c, double t_new);
+// the same with the state of the final stage 1, if the device accepted
+void launch_commit_stage(qdeq_ctx *c, double t_new, const int *go);
 void launch_maxima(qdeq_ctx *c);
 
 }  // namespace qdeq

@@ -97,3 +97,28 @@ def test_reference_cycle_on_tiles_equals_oracle(ni, nk, levels, sweeps):
             eng.ode_solve(V)
         assert e.value.status == lib.QDEQ_ERR_MG_NOT_CONVERGED
     np.testing.assert_array_equal(V, ref)
+
+
+@pytest.mark.parametrize("n,levels,cap", [(129, 4, 2), (257, 5, 3)])
+def test_run_after_a_solve_that_fails_behind_a_queued_stage(n, levels, cap):
+    """A stage solve that ends at the V-cycle cap, with the next stage queued
+    behind it and its stop test handed to that stage's fault update, reports
+    the cap; set up again, the context steps as a fresh one does."""
+    pb = config.make_bp1_problem(n, basin=True, levels=levels, tol_mode=config.TOL_REL,
+                                 tol=1e-10)
+    me = oracle.mu_equi(pb.mu)
+    kw = {**PROD, "ini_dt": 1e5, "max_vcycles": cap}
+    runs = []
+    for tries in (1, 3):
+        with lib.Engine(pb, me, **kw) as eng:
+            for _ in range(tries):
+                eng.rk43_setup()
+                with pytest.raises(lib.QdeqError) as e:
+                    eng.rk43_step(60)
+                assert e.value.status == lib.QDEQ_ERR_MG_NOT_CONVERGED
+                st = eng.state()
+            runs.append(st)
+    a, b = runs
+    for key in ("t", "vcycles", "solves"):
+        assert a["info"][key] == b["info"][key], key
+    np.testing.assert_array_equal(a["U"], b["U"])
