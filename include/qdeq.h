@@ -104,7 +104,9 @@ int qdeq_destroy(qdeq_ctx *ctx);
  * runs it on the temporally blocked LDS kernels with interior tiles of
  * tile_x by tile_y points (even sizes, limited by the 160 KiB LDS at the
  * configured sweep counts); tiled == 0 uses one launch per half-sweep.
- * Results are identical either way. */
+ * Without this call, qdeq_autotune_tiles or qdeq_set_tile_shapes, each level
+ * has the shapes that a model of the launch time picks.  Results are
+ * identical either way. */
 int qdeq_set_tiles(qdeq_ctx *ctx, int tiled, int tile_x, int tile_y);
 /* 1 if solves of ctx currently run the fast cycle on the tiled kernels. */
 int qdeq_uses_tiled_cycle(const qdeq_ctx *ctx);

@@ -297,6 +297,7 @@ int qdeq_set_tiles(qdeq_ctx *c, int tiled, int tile_x, int tile_y) {
   c->tile_tx = tile_x;
   c->tile_ty = tile_y;
   c->tuned = false;
+  c->user_tiles = true;
   mg_destroy_graphs(c);
   return QDEQ_OK;
 }
@@ -321,8 +322,7 @@ int qdeq_get_tile_shapes(const qdeq_ctx *c, int *nlevels, int *shapes) {
   const int lt = use_tiled(c) ? tail_entry_level(c) : 0;
   *nlevels = lt;
   for (int l = 0; l < lt; l++) {
-    const TileShape dn = c->tuned ? c->tdown[l] : TileShape{c->tile_tx, c->tile_ty, 16};
-    const TileShape up = c->tuned ? c->tup[l] : TileShape{c->tile_tx, c->tile_ty, 16};
+    const TileShape dn = tile_shape(c, l, true), up = tile_shape(c, l, false);
     const int v[6] = {dn.tx, dn.ty, dn.tyt, up.tx, up.ty, up.tyt};
     for (int i = 0; i < 6; i++) shapes[6 * l + i] = v[i];
   }

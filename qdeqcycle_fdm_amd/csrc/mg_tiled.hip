@@ -1164,11 +1164,22 @@ bool tail_fits(const qdeq_ctx *c, bool fp64) {
 }
 
 // Shape of the down (smoothing + restriction) or up (prolongation +
-// smoothing) kernel of a level.
-static TileShape tile_shape(const qdeq_ctx *c, int level, bool down) {
+// smoothing) kernel of a level: tuned or pinned, else the caller's
+// (qdeq_set_tiles), else the model's.
+TileShape tile_shape(const qdeq_ctx *c, int level, bool down) {
   if (c->tuned) return down ? c->tdown[level] : c->tup[level];
-  return TileShape{c->tile_tx, c->tile_ty, TY_THREADS};
+  if (c->user_tiles) return TileShape{c->tile_tx, c->tile_ty, TY_THREADS};
+  return down ? c->mdown[level] : c->mup[level];
 }
+
+// Model of a launch's time in us, from launches measured back to back: start,
+// first loads and store; the tile data; the half-sweeps at their latency plus
+// the issue of the quads that share a CU.
+static double pass_us(int tiles, int nq, int sweeps, double mbytes) {
+  const int per_cu = (tiles + 255) / 256;
+  return 3.3 + mbytes / 6.0 + 2 * sweeps * (0.17 + 0.017 * per_cu * nq / 64.0);
+}
+
 
 // Whether a shape fits the kernels: even sizes, tile rows (with halo) of at
 // most 320 points, and the LDS with 8 KiB to spare.
@@ -1181,6 +1192,94 @@ static bool shape_fits(const qdeq_ctx *c, const TileShape &s, bool down,
   if (s.tx + 2 * H > 5 * TX_THREADS) return false;
   return tile_budget_bytes(s.tx, s.ty, H, has_f, esz, down, TX_THREADS * s.tyt) + 8192 <=
          c->lds_max;
+}
+
+// Candidate tile sizes of a level.
+static const int kTuneTX[] = {32, 64, 96, 128, 192, 256};
+static const int kTuneTY[] = {2, 4, 8, 16, 32, 64};
+static const int kTuneTYT[] = {4, 8, 16};
+// Tile sizes that split a level into a whole number of tiles: the grids are
+// 2^k + 1 points wide, so the power-of-two sizes leave a last tile of one
+// or two points.  With one tile per CU per round, a grid of 16 x 16 tiles
+// of 66 points at 1025^2 runs in one round where 96 x 32 needs two.
+static const int kFitTX[] = {4, 8, 12, 16};
+static const int kFitTY[] = {8, 12, 16, 24, 32};
+
+static void add_fitted(std::vector<int> &v, int n, const int *parts, int np) {
+  for (int i = 0; i < np; i++) {
+    int t = (n + parts[i] - 1) / parts[i];
+    t += t & 1;
+    if (t >= 2 && std::find(v.begin(), v.end(), t) == v.end()) v.push_back(t);
+  }
+}
+
+static void tile_candidates(const LevelDims &d, std::vector<int> &txs, std::vector<int> &tys) {
+  txs.assign(std::begin(kTuneTX), std::end(kTuneTX));
+  tys.assign(std::begin(kTuneTY), std::end(kTuneTY));
+  add_fitted(txs, d.K, kFitTX, (int)(sizeof(kFitTX) / sizeof(int)));
+  add_fitted(tys, d.N, kFitTY, (int)(sizeof(kFitTY) / sizeof(int)));
+}
+
+// The model's time of a tile kernel: the tile's arrays (three, one more with
+// a right-hand side), the half-sweeps, residual and restriction counted as
+// one sweep.  In FP32, with two or more workgroups on a CU at a time and three
+// or more rounds of them, one's loads run during another's sweeps (2049^2:
+// 110 us a V-cycle against 124 without this; FP64 tiles that small re-read
+// too much halo, 181 against 168).  A level-0 up kernel of more than 256
+// tiles costs a stop-test kernel per V-cycle (see defer_fits).  With these
+// shapes a V-cycle's kernels take 68.6 us at 1025^2 FP64 (93 with tiles of
+// 64 x 16 on every level, 66.0 tuned), 52 at 801 x 481 (51 tuned).
+template <typename T>
+static double shape_us(const qdeq_ctx *c, int l, bool down, bool has_f, const TileShape &s) {
+  const LevelDims &d = c->lv[l];
+  const bool norm = !down && l == 0 && !has_f;
+  const int nu = down ? c->cfg.n_pre : c->cfg.n_post;
+  const int H = down ? 2 * nu + 2 : up_halo(nu, norm);
+  const int nq = ((s.tx + 2 * H) / 2) * ((s.ty + 2 * H) / 2);
+  const int tiles = ((d.K + s.tx - 1) / s.tx) * ((d.N + s.ty - 1) / s.ty);
+  const double mem = 1e-6 * tiles * nq * 4.0 * (has_f ? 4 : 3) * sizeof(T) / 6.0;
+  const int quads = (nq + TILE_THREADS - 1) / TILE_THREADS;
+  const int waves = (nq + 64 * quads - 1) / (64 * quads);
+  const int resident = std::max(1, (quads == 1 ? 20 : 16) / waves);
+  const int per_cu = (tiles + 255) / 256, rounds = (per_cu + resident - 1) / resident;
+  const double sweeps = 2 * (down || norm ? nu + 1 : nu) *
+                        (0.17 * rounds + 0.017 * per_cu * nq / 64.0);
+  const double body = sizeof(T) == 4 && resident >= 2 && rounds >= 3
+                          ? std::max(mem, sweeps) + 0.25 * std::min(mem, sweeps)
+                          : mem + sweeps;
+  return 3.3 + body + (norm && tiles > 256 ? 4.0 : 0.0);
+}
+
+// The model's choice per level, for contexts that neither tune nor pin their
+// shapes.  One quad per thread where a kernel with two spills (FP64 down).
+template <typename T>
+static void model_shapes(qdeq_ctx *c) {
+  const int lt = tail_entry_level(c);
+  for (int l = 0; l < lt && l < QDEQ_MAX_LEVELS; l++)
+    for (int dir = 0; dir < 2; dir++) {
+      const bool down = dir == 0, hf = l > 0 || sizeof(T) == 4;
+      TileShape best{c->tile_tx, c->tile_ty, TY_THREADS};
+      double best_us = 1e300;
+      std::vector<int> txs, tys;
+      tile_candidates(c->lv[l], txs, tys);
+      for (int tx : txs)
+        for (int ty : tys) {
+          const TileShape s{tx, ty, TY_THREADS};
+          if (!shape_fits(c, s, down, hf, sizeof(T))) continue;
+          const int H = 2 * c->cfg.n_pre + 2;
+          if (down && sizeof(T) == 8 && (tx / 2 + H) * (ty / 2 + H) > TILE_THREADS) continue;
+          const LevelDims &d = c->lv[l];
+          if (!down && l == 0 && !hf &&
+              (long)((d.K + tx - 1) / tx) * ((d.N + ty - 1) / ty) > kPartialCap)
+            continue;
+          const double us = shape_us<T>(c, l, down, hf, s);
+          if (us < best_us) {
+            best_us = us;
+            best = s;
+          }
+        }
+      (down ? c->mdown[l] : c->mup[l]) = best;
+    }
 }
 
 // Largest dynamic LDS the tile kernels of this context would request.
@@ -1431,14 +1530,6 @@ void vcycle_tiled_fp32_ir(qdeq_ctx *c) {
 // 2.6 us each whatever the size up to 257^2 (448 of them a V-cycle at 129^2);
 // here a half-sweep costs 0.2 to 0.7 us inside a launch.
 
-// Model of a launch's time in us, from launches measured back to back: start,
-// first loads and store; the tile data; the half-sweeps at their latency plus
-// the issue of the quads that share a CU.
-static double pass_us(int tiles, int nq, int sweeps, double mbytes) {
-  const int per_cu = (tiles + 255) / 256;
-  return 3.3 + mbytes / 6.0 + 2 * sweeps * (0.17 + 0.017 * per_cu * nq / 64.0);
-}
-
 // `sweeps` split into as even passes of at most `most` sweeps as there are.
 static std::vector<int> split_sweeps(int sweeps, int most) {
   const int n = std::max(1, (sweeps + most - 1) / most);
@@ -1594,24 +1685,6 @@ static void launch_one(qdeq_ctx *c, LevelBufs<T> *B, int l, bool down,
   }
 }
 
-static const int kTuneTX[] = {32, 64, 96, 128, 192, 256};
-static const int kTuneTY[] = {2, 4, 8, 16, 32, 64};
-static const int kTuneTYT[] = {4, 8, 16};
-// Tile sizes that split a level into a whole number of tiles: the grids are
-// 2^k + 1 points wide, so the power-of-two sizes leave a last tile of one
-// or two points.  With one tile per CU per round, a grid of 16 x 16 tiles
-// of 66 points at 1025^2 runs in one round where 96 x 32 needs two.
-static const int kFitTX[] = {4, 8, 12, 16};
-static const int kFitTY[] = {8, 12, 16, 24, 32};
-
-static void add_fitted(std::vector<int> &v, int n, const int *parts, int np) {
-  for (int i = 0; i < np; i++) {
-    int t = (n + parts[i] - 1) / parts[i];
-    t += t & 1;
-    if (t >= 2 && std::find(v.begin(), v.end(), t) == v.end()) v.push_back(t);
-  }
-}
-
 template <typename T, bool EXACT>
 static int autotune_t(qdeq_ctx *c, LevelBufs<T> *B, bool level0_has_f,
                       double *u64, int reps) {
@@ -1626,13 +1699,12 @@ static int autotune_t(qdeq_ctx *c, LevelBufs<T> *B, bool level0_has_f,
     for (int dir = 0; dir < 2 && st == QDEQ_OK; dir++) {
       const bool down = dir == 0;
       const bool hf = l > 0 || level0_has_f;
-      // every candidate's time, in a fixed order; the first one within 3%
-      // of the fastest wins (stable against timing noise between runs)
+      // every candidate's time, in a fixed order.  Among those within 3% of
+      // the fastest (small levels' kernels all take as long as a launch by
+      // the host) the model's best wins, the first of equals.
       std::vector<std::pair<TileShape, float>> times;
-      std::vector<int> txs(std::begin(kTuneTX), std::end(kTuneTX));
-      std::vector<int> tys(std::begin(kTuneTY), std::end(kTuneTY));
-      add_fitted(txs, c->lv[l].K, kFitTX, (int)(sizeof(kFitTX) / sizeof(int)));
-      add_fitted(tys, c->lv[l].N, kFitTY, (int)(sizeof(kFitTY) / sizeof(int)));
+      std::vector<int> txs, tys;
+      tile_candidates(c->lv[l], txs, tys);
       for (int tx : txs)
         for (int ty : tys) {
           int last_quads = 0, last_rows = 0;
@@ -1665,11 +1737,15 @@ static int autotune_t(qdeq_ctx *c, LevelBufs<T> *B, bool level0_has_f,
       if (times.empty()) continue;
       float best_ms = times[0].second;
       for (const auto &t : times) best_ms = std::min(best_ms, t.second);
-      for (const auto &t : times)
-        if (t.second <= 1.03f * best_ms) {
+      double best_us = 1e300;
+      for (const auto &t : times) {
+        if (t.second > 1.03f * best_ms) continue;
+        const double us = shape_us<T>(c, l, down, hf, t.first);
+        if (us < best_us) {
+          best_us = us;
           (down ? c->tdown[l] : c->tup[l]) = t.first;
-          break;
         }
+      }
     }
   }
   (void)hipEventDestroy(e0);
@@ -1854,10 +1930,13 @@ int tiled_setup(qdeq_ctx *c) {
 #undef SETA
   (void)hipGetLastError();
   if (!tiles_fit(c, c->tile_tx, c->tile_ty)) c->tiled = false;
-  if (c->cfg.precision == QDEQ_PREC_FP32_IR)
+  if (c->cfg.precision == QDEQ_PREC_FP32_IR) {
+    model_shapes<float>(c);
     plan_reference<float>(c);
-  else
+  } else {
+    model_shapes<double>(c);
     plan_reference<double>(c);
+  }
   return QDEQ_OK;
 }
 

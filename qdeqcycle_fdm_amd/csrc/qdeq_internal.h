@@ -220,6 +220,10 @@ struct qdeq_ctx {
   // with 16 thread rows
   bool tuned = false;
   qdeq::TileShape tdown[QDEQ_MAX_LEVELS] = {}, tup[QDEQ_MAX_LEVELS] = {};
+  // without either (user_tiles: qdeq_set_tiles was called), shapes by a model
+  // of the launch time
+  bool user_tiles = false;
+  qdeq::TileShape mdown[QDEQ_MAX_LEVELS] = {}, mup[QDEQ_MAX_LEVELS] = {};
   // reference cycle: the levels above the tail (empty: one launch per
   // half-sweep), the tail's entry level, and whether it is used
   std::vector<qdeq::RefLevel> ref_plan;
@@ -346,6 +350,7 @@ void vcycle_ref_fp64(qdeq_ctx *c, double *partial, int *nparts);
 void vcycle_ref_fp32_ir(qdeq_ctx *c);
 int tiled_setup(qdeq_ctx *c);
 bool tiles_fit(const qdeq_ctx *c, int tx, int ty);
+TileShape tile_shape(const qdeq_ctx *c, int level, bool down);
 bool fused_start_fits(const qdeq_ctx *c);
 bool fold_fits(const qdeq_ctx *c);
 bool defer_fits(const qdeq_ctx *c);

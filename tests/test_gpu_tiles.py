@@ -35,7 +35,7 @@ def _solve(pb, me, U, shape=None, **kw):
     with lib.Engine(pb, me, **{**PROD, "tol": 1e-300, "max_vcycles": 2, **kw}) as eng:
         if shape is None:
             eng.set_tiles(False)
-        else:
+        elif shape != "default":
             n = len(eng.tile_shapes())
             eng.set_tile_shapes([(shape, shape)] * n)
         V = U.copy()
@@ -73,6 +73,18 @@ def test_fp32_tiles_equal_untiled(ni, nk, levels):
     for shape in SHAPES + [(66, 66, 4), (250, 16, 4)]:  # three quads per thread
         got = _solve(pb, me, U, shape, precision=config.PREC_FP32_IR)
         np.testing.assert_array_equal(got, ref, err_msg=str(shape))
+
+
+@pytest.mark.parametrize("ni,nk,levels", [(65, 65, 4), (130, 97, 3), (801, 481, 6), (1030, 67, 5),
+                                          (67, 1030, 5)])
+@pytest.mark.parametrize("precision", [config.PREC_FP64, config.PREC_FP32_IR])
+def test_default_shapes_equal_untiled(ni, nk, levels, precision):
+    pb = _problem(ni, nk, levels)
+    me = oracle.mu_equi(pb.mu)
+    U = _perturbed(pb, 23)
+    ref = _solve(pb, me, U, precision=precision)
+    got = _solve(pb, me, U, "default", precision=precision)
+    np.testing.assert_array_equal(got, ref)
 
 
 @pytest.mark.parametrize("ni,nk,levels", [(129, 129, 3), (130, 97, 3), (66, 131, 2), (41, 57, 1),
