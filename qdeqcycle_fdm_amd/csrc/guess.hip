@@ -33,7 +33,7 @@ struct qdeq_guess {
   int count = 0;
   // training scratch for Mb rows
   int tb_M = 0;
-  float *X = nullptr, *Tg = nullptr, *Z = nullptr, *Y = nullptr, *dZ0 = nullptr;
+  float *X = nullptr, *Tg = nullptr, *Y = nullptr, *dZ0 = nullptr;
   bf16 *Hb[4] = {}, *HbT[4] = {};     // H0..H3 and transposes
   bf16 *dY = nullptr, *dYT = nullptr;
   bf16 *dZb[2] = {}, *dZbT[2] = {};
@@ -84,14 +84,13 @@ void refresh_bf16(qdeq_guess *g, hipStream_t st) {
   for (int l = 0; l < 4; l++) {
     int rows, cols, rp;
     tensor_shape(g, l + 1, &rows, &cols, &rp);
-    nn::epilogue(st, g->w + g->off[l + 1], rp, cols, nn::EPI_PLAIN, nullptr,
-                 g->W[l], g->WT[l], nullptr);
+    nn::epilogue(st, g->w + g->off[l + 1], rp, cols, nn::EPI_PLAIN, g->W[l], g->WT[l]);
   }
 }
 
 int ensure_train_bufs(qdeq_guess *g, int Mb) {
   if (g->tb_M >= Mb) return QDEQ_OK;
-  void *old[] = {g->X, g->Tg, g->Z, g->Y, g->dZ0, g->dY, g->dYT, g->split,
+  void *old[] = {g->X, g->Tg, g->Y, g->dZ0, g->dY, g->dYT, g->split,
                  g->mse_part, g->loss};
   for (void *p : old) (void)hipFree(p);
   for (int i = 0; i < 4; i++) {
@@ -106,7 +105,6 @@ int ensure_train_bufs(qdeq_guess *g, int Mb) {
   const size_t M = (size_t)Mb, wmax = (size_t)std::max(g->F0, g->H);
   GHIP(g, dalloc(&g->X, M * g->nk));
   GHIP(g, dalloc(&g->Tg, M * g->noutp));
-  GHIP(g, dalloc(&g->Z, M * wmax));
   GHIP(g, dalloc(&g->Y, M * g->noutp));
   GHIP(g, dalloc(&g->dZ0, M * g->F0));
   GHIP(g, dalloc(&g->dY, M * g->noutp));
@@ -122,66 +120,89 @@ int ensure_train_bufs(qdeq_guess *g, int Mb) {
   }
   g->split_n = (size_t)64 * M * wmax;
   GHIP(g, dalloc(&g->split, g->split_n));
-  GHIP(g, dalloc(&g->mse_part, (size_t)nn::MSE_BLOCKS));
+  GHIP(g, dalloc(&g->mse_part, (M / 128) * (size_t)(g->noutp / 128)));
   GHIP(g, dalloc(&g->loss, (size_t)1 << 16));
   g->tb_M = Mb;
   return QDEQ_OK;
 }
 
-int gemm(qdeq_guess *g, hipStream_t st, const bf16 *A, int lda, const bf16 *B,
-         int ldb, float *C, int M, int N, int K) {
-  if (nn::gemm_nt(st, nn::GEMM_CFG_WIDE, A, lda, B, ldb, C, N, M, N, K, g->split,
-                  g->split_n, 512))
+int gemm(qdeq_guess *g, int out, const bf16 *A, const bf16 *B, int M, int N, int K,
+         const nn::GemmOut &o) {
+  if (nn::gemm(g->stream, out, A, K, B, K, M, N, K, g->split, g->split_n, o))
     return gset_error(g, QDEQ_ERR_ARG, "GEMM shape not covered by the tiles");
   return QDEQ_OK;
 }
 
-// Forward pass on rows X[0..Mb) (already in g->X); Y = output (FP32).
-int forward(qdeq_guess *g, hipStream_t st, int Mb) {
-  nn::conv_forward(st, g->X, Mb, g->nk, g->w + g->off[0], g->C, g->T, g->f,
+// A minibatch on the device: rows idx[b] (row b without idx) of x and t.
+struct Batch {
+  const float *x, *t;
+  const int *idx;
+  int B, Mb;  // rows, and rows padded to 128 (zero)
+};
+
+// Encoder and hidden layers: H0..H3 and their transposes.
+int forward_hidden(qdeq_guess *g, const Batch &b) {
+  nn::conv_forward(g->stream, b.x, b.idx, b.B, b.Mb, g->nk, g->w + g->off[0], g->C, g->T, g->f,
                    g->P0, g->Hb[0], g->HbT[0]);
   for (int l = 0; l < 3; l++) {
-    const int in = l == 0 ? g->F0 : g->H;
-    int st_ = gemm(g, st, g->Hb[l], in, g->W[l], in, g->Z, Mb, g->H, in);
-    if (st_) return st_;
-    nn::epilogue(st, g->Z, Mb, g->H, nn::EPI_RELU, nullptr, g->Hb[l + 1],
-                 g->HbT[l + 1], nullptr);
+    nn::GemmOut o{};
+    o.out = g->Hb[l + 1];
+    o.outT = g->HbT[l + 1];
+    const int st = gemm(g, nn::OUT_RELU, g->Hb[l], g->W[l], b.Mb, g->H, l == 0 ? g->F0 : g->H, o);
+    if (st) return st;
   }
-  return gemm(g, st, g->Hb[3], g->H, g->W[3], g->H, g->Y, Mb, g->noutp, g->H);
+  return QDEQ_OK;
 }
 
-// Backward pass after forward + mse (g->Y holds dloss/dY): gradients in g->g.
-int backward(qdeq_guess *g, hipStream_t st, int Mb) {
+// Forward and backward pass, mean squared error in *loss (device).  With Adam
+// coefficients the weights are updated, each layer's once the gradient has
+// passed through it, else the gradients go to g->g.
+int forward_backward(qdeq_guess *g, const Batch &b, const nn::AdamCoef *adam, double *loss) {
+  const int Mb = b.Mb;
   int s;
-  nn::epilogue(st, g->Y, Mb, g->noutp, nn::EPI_PLAIN, nullptr, g->dY, g->dYT,
-               nullptr);
-  // W4: [noutp x H] = dY^T [noutp x Mb] * H3^T [H x Mb]^T
-  if ((s = gemm(g, st, g->dYT, Mb, g->HbT[3], Mb, g->g + g->off[4], g->noutp,
-                g->H, Mb)))
-    return s;
-  // dH3 [Mb x H] = dY [Mb x noutp] * W4^T [H x noutp]^T
-  if ((s = gemm(g, st, g->dY, g->noutp, g->WT[3], g->noutp, g->Z, Mb, g->H,
-                g->noutp)))
-    return s;
-  const bf16 *dz = nullptr, *dzT = nullptr;
-  for (int l = 2; l >= 0; l--) {
-    bf16 *o = g->dZb[l & 1], *oT = g->dZbT[l & 1];
-    // dZ_{l+1} = dH_{l+1} * (H_{l+1} > 0)
-    nn::epilogue(st, g->Z, Mb, g->H, nn::EPI_MASK, g->Hb[l + 1], o, oT, nullptr);
-    dz = o;
-    dzT = oT;
-    const int in = l == 0 ? g->F0 : g->H;
-    // W_{l+1}: [H x in] = dZ^T [H x Mb] * H_l^T [in x Mb]^T
-    if ((s = gemm(g, st, dzT, Mb, g->HbT[l], Mb, g->g + g->off[l + 1], g->H, in, Mb)))
-      return s;
-    // dH_l [Mb x in] = dZ [Mb x H] * W_{l+1}^T [in x H]^T
-    if ((s = gemm(g, st, dz, g->H, g->WT[l], g->H, g->Z, Mb, in, g->H))) return s;
+  if ((s = forward_hidden(g, b))) return s;
+  nn::GemmOut y{};
+  y.out = g->dY;
+  y.outT = g->dYT;
+  y.target = b.t;
+  y.idx = b.idx;
+  y.B = b.B;
+  y.nout = g->nout;
+  y.partial = g->mse_part;
+  if ((s = gemm(g, nn::OUT_MSE, g->Hb[3], g->W[3], Mb, g->noutp, g->H, y))) return s;
+  for (int l = 3; l >= 0; l--) {
+    const int in = l == 0 ? g->F0 : g->H, out = l == 3 ? g->noutp : g->H;
+    const bf16 *dz = l == 3 ? g->dY : g->dZb[l & 1], *dzT = l == 3 ? g->dYT : g->dZbT[l & 1];
+    // dZ_l [Mb x in] = dZ [Mb x out] * W_{l+1}^T [in x out]^T where H_l > 0
+    nn::GemmOut h{};
+    h.mask = g->Hb[l];
+    if (l == 0) {
+      h.outF = g->dZ0;
+    } else {
+      h.out = g->dZb[(l - 1) & 1];
+      h.outT = g->dZbT[(l - 1) & 1];
+    }
+    if ((s = gemm(g, nn::OUT_MASK, dz, g->WT[l], Mb, in, out, h))) return s;
+    // W_{l+1}: [out x in] = dZ^T [out x Mb] * H_l^T [in x Mb]^T
+    nn::GemmOut w{};
+    const long long off = g->off[l + 1];
+    if (adam) {
+      w.outF = g->w + off;
+      w.m = g->m + off;
+      w.v = g->v + off;
+      w.out = g->W[l];
+      w.outT = g->WT[l];
+      w.adam = *adam;
+    } else {
+      w.outF = g->g + off;
+    }
+    if ((s = gemm(g, adam ? nn::OUT_ADAM : nn::OUT_F32, dzT, g->HbT[l], out, in, Mb, w))) return s;
   }
-  // encoder: dZ0 = dH0 * (H0 > 0) (FP32), then the conv weight gradient
-  nn::epilogue(st, g->Z, Mb, g->F0, nn::EPI_MASK, g->Hb[0], nullptr, nullptr,
-               g->dZ0);
-  nn::conv_backward(st, g->X, Mb, g->nk, g->dZ0, g->C, g->T, g->f, g->P0,
-                    g->g + g->off[0]);
+  const long long o0 = g->off[0];
+  nn::conv_backward(g->stream, b.x, b.idx, b.B, g->nk, g->dZ0, g->C, g->T, g->f, g->P0,
+                    g->g + o0, adam ? g->w + o0 : nullptr, g->m + o0, g->v + o0,
+                    adam ? *adam : nn::AdamCoef{}, g->mse_part, (Mb / 128) * (g->noutp / 128),
+                    1.0 / ((double)b.B * (double)g->nout), loss);
   return QDEQ_OK;
 }
 
@@ -326,17 +347,16 @@ static void launch_predict_chain(qdeq_ctx *c) {
   hipLaunchKernelGGL(k_guess_prep, dim3(1), dim3(PREP_THREADS), 0, st, c->d[0].u,
                      d.N, d.K, d.P, c->gprev, c->gx, c->gs, (double *)nullptr,
                      g->f, g->nc);
-  nn::conv_forward(st, c->gx, 16, g->nk, g->w + g->off[0], g->C, g->T, g->f,
-                   g->P0, c->gh[0], nullptr);
+  nn::conv_forward(st, c->gx, nullptr, 16, 16, g->nk, g->w + g->off[0], g->C, g->T,
+                   g->f, g->P0, c->gh[0], nullptr);
   for (int l = 0; l < 3; l++) {
     const int in = l == 0 ? g->F0 : g->H;
-    nn::gemm_nt(st, nn::GEMM_CFG_SKINNY, c->gh[l], in, g->W[l], in, c->gz, g->H,
-                16, g->H, in, c->gsplit, c->gsplit_n, 64);
-    nn::epilogue(st, c->gz, 16, g->H, nn::EPI_RELU, nullptr, c->gh[l + 1], nullptr,
-                 nullptr);
+    nn::gemm_skinny(st, c->gh[l], in, g->W[l], in, c->gz, 16, g->H, in, c->gsplit,
+                    c->gsplit_n, 64);
+    nn::epilogue(st, c->gz, 16, g->H, nn::EPI_RELU, c->gh[l + 1], nullptr);
   }
-  nn::gemm_nt(st, nn::GEMM_CFG_SKINNY, c->gh[3], g->H, g->W[3], g->H, c->gy,
-              g->noutp, 16, g->noutp, g->H, c->gsplit, c->gsplit_n, 64);
+  nn::gemm_skinny(st, c->gh[3], g->H, g->W[3], g->H, c->gy, 16, g->noutp, g->H,
+                  c->gsplit, c->gsplit_n, 64);
   const dim3 blk(256);
   const dim3 grd((d.P + 255) / 256, d.N);
   hipLaunchKernelGGL(k_guess_apply, grd, blk, 0, st, c->d[0].u, c->wr, c->gy, c->gx,
@@ -571,7 +591,7 @@ int qdeq_guess_create(const qdeq_guess_config *cfg, qdeq_guess **out) {
 int qdeq_guess_destroy(qdeq_guess *g) {
   if (!g) return QDEQ_OK;
   void *p[] = {g->w, g->m, g->v, g->g, g->xs, g->ts, g->scales, g->mags, g->X, g->Tg,
-               g->Z, g->Y, g->dZ0, g->dY, g->dYT, g->split, g->mse_part,
+               g->Y, g->dZ0, g->dY, g->dYT, g->split, g->mse_part,
                g->loss, g->idx};
   for (void *q : p) (void)hipFree(q);
   for (int i = 0; i < 4; i++) {
@@ -689,9 +709,8 @@ int qdeq_guess_forward_backward(qdeq_guess *g, int batch, const float *x,
   if ((st = ensure_train_bufs(g, Mb))) return st;
   if ((st = upload_rows(g, g->X, Mb, g->nk, x, batch, g->nk))) return st;
   if ((st = upload_rows(g, g->Tg, Mb, g->noutp, t, batch, g->nout))) return st;
-  if ((st = forward(g, g->stream, Mb))) return st;
-  nn::mse(g->stream, g->Y, g->Tg, Mb, batch, g->nout, g->noutp, g->mse_part, g->loss);
-  if ((st = backward(g, g->stream, Mb))) return st;
+  const Batch b{g->X, g->Tg, nullptr, batch, Mb};
+  if ((st = forward_backward(g, b, nullptr, g->loss))) return st;
   GHIP(g, hipGetLastError());
   GHIP(g, hipStreamSynchronize(g->stream));
   if (loss) GHIP(g, hipMemcpy(loss, g->loss, sizeof(double), hipMemcpyDeviceToHost));
@@ -705,7 +724,11 @@ int qdeq_guess_forward(qdeq_guess *g, int batch, const float *x, float *y) {
   int st;
   if ((st = ensure_train_bufs(g, Mb))) return st;
   if ((st = upload_rows(g, g->X, Mb, g->nk, x, batch, g->nk))) return st;
-  if ((st = forward(g, g->stream, Mb))) return st;
+  const Batch b{g->X, nullptr, nullptr, batch, Mb};
+  if ((st = forward_hidden(g, b))) return st;
+  nn::GemmOut o{};
+  o.outF = g->Y;
+  if ((st = gemm(g, nn::OUT_F32, g->Hb[3], g->W[3], Mb, g->noutp, g->H, o))) return st;
   GHIP(g, hipGetLastError());
   GHIP(g, hipMemcpy2DAsync(y, (size_t)g->nout * sizeof(float), g->Y,
                            (size_t)g->noutp * sizeof(float),
@@ -762,21 +785,15 @@ int qdeq_guess_train(qdeq_guess *g, const qdeq_train_config *tc,
     GHIP(g, hipStreamSynchronize(g->stream));
     const int nbl = std::min(nb, (1 << 16));
     for (int b = 0; b < nbl; b++, step++) {
-      nn::gather(g->stream, g->xs, g->ts, g->idx + (size_t)b * B, B, Mb, g->nk,
-                 g->noutp, g->X, g->Tg);
-      if ((st = forward(g, g->stream, Mb))) return st;
-      nn::mse(g->stream, g->Y, g->Tg, Mb, B, g->nout, g->noutp, g->mse_part,
-              g->loss + b);
-      if ((st = backward(g, g->stream, Mb))) return st;
       g->adam_t++;
       const double frac = total > 1 ? (double)step / (double)(total - 1) : 0.0;
       const double lr = tc->lr * std::pow(tc->lr_final / tc->lr, frac);
       const double c1 = 1.0 - std::pow(tc->beta1, (double)g->adam_t);
       const double c2 = 1.0 - std::pow(tc->beta2, (double)g->adam_t);
-      nn::adam(g->stream, g->w, g->m, g->v, g->g, g->ntot, (float)lr,
-               (float)tc->beta1, (float)tc->beta2, (float)tc->eps, (float)c1,
-               (float)c2);
-      refresh_bf16(g, g->stream);
+      const nn::AdamCoef adam{(float)lr, (float)tc->beta1, (float)tc->beta2,
+                              (float)tc->eps, (float)c1, (float)c2};
+      const Batch bt{g->xs, g->ts, g->idx + (size_t)b * B, B, Mb};
+      if ((st = forward_backward(g, bt, &adam, g->loss + b))) return st;
     }
     GHIP(g, hipGetLastError());
     losses.assign((size_t)nbl, 0.0);
@@ -863,17 +880,16 @@ int qdeq_guess_infer(qdeq_ctx *c, const float *x, float *y) {
   if (!g) return set_error(c, QDEQ_ERR_STATE, "no guess attached");
   QDEQ_HIP(c, hipMemcpyAsync(c->gx, x, (size_t)g->nk * sizeof(float),
                              hipMemcpyHostToDevice, c->stream));
-  nn::conv_forward(c->stream, c->gx, 16, g->nk, g->w + g->off[0], g->C, g->T,
-                   g->f, g->P0, c->gh[0], nullptr);
+  nn::conv_forward(c->stream, c->gx, nullptr, 16, 16, g->nk, g->w + g->off[0], g->C,
+                   g->T, g->f, g->P0, c->gh[0], nullptr);
   for (int l = 0; l < 3; l++) {
     const int in = l == 0 ? g->F0 : g->H;
-    nn::gemm_nt(c->stream, nn::GEMM_CFG_SKINNY, c->gh[l], in, g->W[l], in, c->gz,
-                g->H, 16, g->H, in, c->gsplit, c->gsplit_n, 64);
-    nn::epilogue(c->stream, c->gz, 16, g->H, nn::EPI_RELU, nullptr, c->gh[l + 1],
-                 nullptr, nullptr);
+    nn::gemm_skinny(c->stream, c->gh[l], in, g->W[l], in, c->gz, 16, g->H, in, c->gsplit,
+                    c->gsplit_n, 64);
+    nn::epilogue(c->stream, c->gz, 16, g->H, nn::EPI_RELU, c->gh[l + 1], nullptr);
   }
-  nn::gemm_nt(c->stream, nn::GEMM_CFG_SKINNY, c->gh[3], g->H, g->W[3], g->H, c->gy,
-              g->noutp, 16, g->noutp, g->H, c->gsplit, c->gsplit_n, 64);
+  nn::gemm_skinny(c->stream, c->gh[3], g->H, g->W[3], g->H, c->gy, 16, g->noutp, g->H,
+                  c->gsplit, c->gsplit_n, 64);
   QDEQ_HIP(c, hipGetLastError());
   QDEQ_HIP(c, hipMemcpyAsync(y, c->gy, (size_t)g->nout * sizeof(float),
                              hipMemcpyDeviceToHost, c->stream));

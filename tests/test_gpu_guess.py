@@ -204,3 +204,71 @@ def test_learned_guess_lowers_vcycles_per_solve():
     assert st["accepted"] > 0.5 * st["predicted"]
     assert dslip <= 1e-6
     g.close()
+
+
+@pytest.mark.parametrize("nk,hidden,batch", [(33 + 32, 128, 1), (129, 256, 129), (129, 512, 4000),
+                                             (257, 384, 300)])
+def test_gradient_over_the_product_splits(nk, hidden, batch):
+    """Products of one to many blocks and K chunks: wide, over the wavefronts of
+    a block, and with partial sums in memory."""
+    g = lib.Guess(nk, hidden=hidden, capacity=1, **({"channels": 16} if nk == 65 else {}))
+    d = _dims(g)
+    rng = np.random.default_rng(nk + batch)
+    flat = onn.init_params(d, seed=nk)
+    g.set_params(flat)
+    x = rng.standard_normal((batch, nk)).astype(np.float32)
+    t = (0.1 * rng.standard_normal((batch, d.nout))).astype(np.float32)
+    loss, grad = g.forward_backward(x, t)
+    rl, rg = onn.forward_backward(d, flat.astype(np.float64), x.astype(np.float64),
+                                  t.astype(np.float64), bf16=True)
+    assert abs(loss - rl) <= 1e-4 * rl
+    o = 0
+    for i, (r, c) in enumerate(d.shapes()):
+        n = r * c
+        assert _rel(grad[o:o + n].astype(np.float64), rg[o:o + n]) < 2e-2, i
+        o += n
+    g.close()
+
+
+def test_training_step_is_adam_on_the_gradient():
+    """One step on all pairs from zero moments moves a weight by lr g / (|g| +
+    eps) of the gradient on those pairs, whose sums run in another order here:
+    the sign and 1% where |g| is above 1e-3 of its tensor's largest.  The BF16
+    copies that the step leaves equal the ones made from its parameters."""
+    pb, me = _engine(129, 4)
+    g = lib.Guess(129, hidden=256, capacity=150)
+    with lib.Engine(pb, me, **FAST) as eng:
+        eng.rk43_setup()
+        U = [eng.state()["U"]]
+        eng.attach_guess(g, lib.GUESS_HARVEST)
+        eng.rk43_step(30)
+        eng.attach_guess(None, lib.GUESS_OFF)
+        U.append(eng.state()["U"])
+    n = g.pairs
+    x, t, s = g.read_pairs(0, n)
+    # training skips pairs whose increment is below 1e-7 of the boundary data,
+    # which grow over the 30 steps; no pair falls between the two ends' lines
+    lo, hi = (max(np.abs(u[1:-1, 1]).max(), abs(u[1, -2])) for u in U)
+    assert lo <= hi and not np.any((s >= 1e-7 * lo) & (s <= 1e-7 * hi))
+    x, t = x[s > 1e-7 * hi], t[s > 1e-7 * hi]
+    assert len(x) > 20
+    w0 = g.get_params()
+    _, grad = g.forward_backward(x, t)
+    g.train(epochs=1, batch=n, lr=1e-3, lr_final=1e-3)
+    w1 = g.get_params()
+    if np.array_equal(w0, w1):
+        pytest.fail("the step changed no weight")
+    o = 0
+    for r, c in _dims(g).shapes():
+        a, b = w0[o:o + r * c].astype(np.float64), w1[o:o + r * c].astype(np.float64)
+        k = grad[o:o + r * c].astype(np.float64)
+        big = np.abs(k) > 1e-3 * np.abs(k).max()
+        step = 1e-3 * k / (np.abs(k) + 1e-8)
+        np.testing.assert_allclose((a - b)[big], step[big], atol=1e-5)
+        o += r * c
+    h = lib.Guess(129, hidden=256, capacity=1)
+    h.set_params(w1)
+    for u, v in zip(g.forward_backward(x, t), h.forward_backward(x, t)):
+        np.testing.assert_array_equal(u, v)
+    g.close()
+    h.close()
