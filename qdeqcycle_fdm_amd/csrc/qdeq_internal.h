@@ -129,6 +129,8 @@ struct RkMachine {
   long long seq = 0;         // combinations launched (MB_RKSEQ)
 };
 
+constexpr int kStageVecs = 8;  // staged nz vectors of the drop-in entry points
+
 }  // namespace qdeq
 
 struct qdeq_ctx {
@@ -146,7 +148,8 @@ struct qdeq_ctx {
   int *flags = nullptr;        // [0] NR NaN flag
   int *flags_host = nullptr;
   double *stage_U = nullptr;   // nx*nz staging for drop-in entry points
-  double *stage_v[8] = {};     // nz staging vectors
+  double *stage_v[qdeq::kStageVecs] = {};  // nz staging vectors, one allocation
+  double *host_v = nullptr;    // their pinned host side
   qdeq::FaultBufs fb{};
   hipStream_t stream = nullptr;
   hipGraphExec_t g_cycle = nullptr;   // one V-cycle (or IR sweep) + residual norm
