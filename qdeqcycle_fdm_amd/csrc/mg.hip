@@ -161,21 +161,50 @@ __device__ inline double residual_at2(const double *__restrict__ ui,
                    DH2;
 }
 
+// First row of this workgroup in the row kernels below.  Workgroups go to the
+// 8 XCDs in turn, each with an L2 of its own; here XCD x gets the x-th of 8
+// bands of consecutive rows, so that a row's neighbours above and below come
+// from the L2 that holds them (with row = workgroup the displacement was read
+// by three XCDs and cz by two: the FP32-IR residual at 2049^2 took 33 us, 20
+// now, 5.9 TB/s of what it must move; the start's norms with a candidate at
+// 1025^2 16 us, 11 now).  The partial sums stay indexed by row.
+__device__ inline int band_row() {
+  const int n = gridDim.x, x = blockIdx.x & 7;
+  return x * (n >> 3) + min(x, n & 7) + ((int)blockIdx.x >> 3);
+}
+
+// a[t] + a[t + NORM_THREADS] + ... of thread t, from 0.0 in this order, with
+// the loads of eight terms in flight (2048 partial sums: the stop test's
+// kernel 5.0 -> 4.1 us).
+__device__ inline double strided_sum(const double *__restrict__ a, int n) {
+  double acc = 0.0;
+  for (int i0 = threadIdx.x; i0 < n; i0 += 8 * NORM_THREADS) {
+    double v[8];
+#pragma unroll
+    for (int q = 0; q < 8; q++) v[q] = a[min(i0 + q * NORM_THREADS, n - 1)];
+#pragma unroll
+    for (int q = 0; q < 8; q++)
+      if (i0 + q * NORM_THREADS < n) acc += v[q];
+  }
+  return acc;
+}
+
 // Level-0 residual norm, pass 1: fixed-grid partial sums of r^2 (the
 // reference uses calcuDelta_dev + cublasDnrm2, odeSolver.cpp:693-700).
-// Optionally stores r as FP32 (the IR right-hand side) and zeroes the FP32
-// correction.  Deterministic: fixed grid, fixed per-thread order, fixed tree.
+// Optionally stores r as FP32 (the IR right-hand side).  Deterministic: fixed
+// grid, fixed per-thread order, fixed tree.
 template <bool STORE32>
 __global__ __launch_bounds__(NORM_THREADS) void k_resnorm_partial(
     const double *__restrict__ u, const double *__restrict__ cx,
     const double *__restrict__ cz, int N, int K, int P, double DH2,
     double *__restrict__ partial, float *__restrict__ r32,
-    float *__restrict__ e32, const int *__restrict__ gate) {
+    const int *__restrict__ gate) {
   if (gate && gate[0]) return;  // batched solve already converged
   __shared__ double sh[NORM_THREADS];
   double acc = 0.0;
   constexpr int UNR = 4;  // as in k_start_partials
-  for (int j = blockIdx.x; j < N; j += gridDim.x) {
+  const int row0 = band_row();
+  for (int j = row0; j < N; j += gridDim.x) {
     const int jS = (j == 0) ? 1 : j - 1;
     const int jN = (j == N - 1) ? N - 2 : j + 1;
     for (int k0 = 1 + threadIdx.x; k0 <= K - 2; k0 += UNR * NORM_THREADS) {
@@ -192,17 +221,13 @@ __global__ __launch_bounds__(NORM_THREADS) void k_resnorm_partial(
         const int k = k0 + q * NORM_THREADS;
         if (k <= K - 2) {
           acc += r[q] * r[q];
-          if (STORE32) {
-            const size_t c = (size_t)j * P + k;
-            r32[c] = (float)r[q];
-            e32[c] = 0.0f;
-          }
+          if (STORE32) r32[(size_t)j * P + k] = (float)r[q];
         }
       }
     }
   }
   const double s = block_sum_256(acc, sh);
-  if (threadIdx.x == 0) partial[blockIdx.x] = s;
+  if (threadIdx.x == 0) partial[row0] = s;
 }
 
 // Boundary-data residual ||r(u_interior = 0)||^2 partials: only the columns
@@ -236,9 +261,7 @@ __global__ __launch_bounds__(NORM_THREADS) void k_norm_final(
     const double *__restrict__ partial, int n, double *__restrict__ out,
     double *__restrict__ mb) {
   __shared__ double sh[NORM_THREADS];
-  double acc = 0.0;
-  for (int i = threadIdx.x; i < n; i += NORM_THREADS) acc += partial[i];
-  const double s = block_sum_256(acc, sh);
+  const double s = block_sum_256(strided_sum(partial, n), sh);
   if (threadIdx.x == 0) {
     const double v = sqrt(s);
     out[0] = v;
@@ -259,10 +282,7 @@ __global__ __launch_bounds__(NORM_THREADS) void k_norm_gate(
     int cap) {
   __shared__ double sh[NORM_THREADS];
   const bool skip = gate[0] != 0;
-  double acc = 0.0;
-  if (!skip)
-    for (int i = threadIdx.x; i < n; i += NORM_THREADS) acc += partial[i];
-  const double s = block_sum_256(acc, sh);
+  const double s = block_sum_256(skip ? 0.0 : strided_sum(partial, n), sh);
   if (threadIdx.x == 0) {
     const int seq = gate[3] + 1;
     gate[3] = seq;
@@ -314,7 +334,8 @@ __global__ __launch_bounds__(NORM_THREADS) void k_start_partials(
   // each thread's points of a row are evaluated together (their loads in
   // flight at once), then added in order
   constexpr int UNR = 4;
-  for (int j = blockIdx.x; j < N; j += gridDim.x) {
+  const int row0 = band_row();
+  for (int j = row0; j < N; j += gridDim.x) {
     const int jS = (j == 0) ? 1 : j - 1;
     const int jN = (j == N - 1) ? N - 2 : j + 1;
     for (int k0 = 1 + threadIdx.x; k0 <= K - 2; k0 += UNR * NORM_THREADS) {
@@ -355,8 +376,8 @@ __global__ __launch_bounds__(NORM_THREADS) void k_start_partials(
   double v3[3] = {acc, accc, accb};
   block_sums<3>(v3, &sh[0][0]);
   if (threadIdx.x == 0) {
-    partial[blockIdx.x] = v3[0];
-    if (CAND) partial[2 * NORM_BLOCKS + blockIdx.x] = v3[1];
+    partial[row0] = v3[0];
+    if (CAND) partial[2 * NORM_BLOCKS + row0] = v3[1];
     if (bd && blockIdx.x < BDRES_BLOCKS) partial[NORM_BLOCKS + blockIdx.x] = v3[2];
   }
 }
@@ -388,14 +409,9 @@ __global__ __launch_bounds__(NORM_THREADS) void k_start_gate(
   }
   // the three sums of k_norm_final's order, in one tree
   __shared__ double sh[3][NORM_THREADS];
-  const int tid = threadIdx.x;
-  double a = 0.0, b = 0.0, cc = 0.0;
-  for (int i = tid; i < nb; i += NORM_THREADS) a += partial[i];
-  if (rel)
-    for (int i = tid; i < BDRES_BLOCKS; i += NORM_THREADS) b += partial[NORM_BLOCKS + i];
-  if (cand)
-    for (int i = tid; i < nb; i += NORM_THREADS) cc += partial[2 * NORM_BLOCKS + i];
-  double v3[3] = {a, b, cc};
+  double v3[3] = {strided_sum(partial, nb),
+                  rel ? strided_sum(partial + NORM_BLOCKS, BDRES_BLOCKS) : 0.0,
+                  cand ? strided_sum(partial + 2 * NORM_BLOCKS, nb) : 0.0};
   block_sums<3>(v3, &sh[0][0]);
   const double su = v3[0], sb = v3[1], sc = v3[2];
   if (threadIdx.x == 0) {
@@ -454,6 +470,13 @@ __global__ void k_restore_if(double *__restrict__ u, const double *__restrict__ 
   for (int j = blockIdx.x; j < N; j += gridDim.x)
     for (int k = 1 + threadIdx.x; k <= K - 2; k += blockDim.x)
       u[(size_t)j * P + k] = src[(size_t)j * P + k];
+}
+
+template <typename T>
+__global__ void k_zero(T *__restrict__ a, size_t n) {
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (size_t)gridDim.x * blockDim.x)
+    a[i] = T(0);
 }
 
 // IR update u += e (interior columns), FP64 += FP32.
@@ -594,7 +617,7 @@ static void launch_norm_final(qdeq_ctx *c, int nparts) {
                        c->partial, nparts, c->scal + SC_NORM, mb_dev(c) + SC_NORM);
 }
 
-// Level-0 residual norm into scal[SC_NORM] (and r32/e32 for IR).
+// Level-0 residual norm into scal[SC_NORM] (and r32 for IR).
 static void launch_resnorm(qdeq_ctx *c, bool store32) {
   const LevelDims &d = c->lv[0];
   const double DH2 = d.DH * d.DH;
@@ -602,12 +625,12 @@ static void launch_resnorm(qdeq_ctx *c, bool store32) {
     hipLaunchKernelGGL((k_resnorm_partial<true>), dim3(norm_blocks(c)),
                        dim3(NORM_THREADS), 0, c->stream, c->d[0].u, c->d[0].cx,
                        c->d[0].cz, d.N, d.K, d.P, DH2, c->partial, c->s[0].f,
-                       c->s[0].u, (const int *)c->gate_ptr);
+                       (const int *)c->gate_ptr);
   else
     hipLaunchKernelGGL((k_resnorm_partial<false>), dim3(norm_blocks(c)),
                        dim3(NORM_THREADS), 0, c->stream, c->d[0].u, c->d[0].cx,
                        c->d[0].cz, d.N, d.K, d.P, DH2, c->partial,
-                       (float *)nullptr, (float *)nullptr, (const int *)c->gate_ptr);
+                       (float *)nullptr, (const int *)c->gate_ptr);
   launch_norm_final(c, norm_blocks(c));
 }
 
@@ -618,7 +641,7 @@ void launch_resnorm_of(qdeq_ctx *c, const double *u, int off, int slot) {
   hipLaunchKernelGGL((k_resnorm_partial<false>), dim3(norm_blocks(c)),
                      dim3(NORM_THREADS), 0, c->stream, u, c->d[0].cx, c->d[0].cz,
                      d.N, d.K, d.P, d.DH * d.DH, c->partial + off,
-                     (float *)nullptr, (float *)nullptr, (const int *)nullptr);
+                     (float *)nullptr, (const int *)nullptr);
   hipLaunchKernelGGL(k_norm_final, dim3(1), dim3(NORM_THREADS), 0, c->stream,
                      c->partial + off, norm_blocks(c), c->scal + slot,
                      mb_dev(c) + slot);
@@ -670,6 +693,8 @@ static void launch_iteration(qdeq_ctx *c) {
     } else if (use_ref_tiles(c)) {
       vcycle_ref_fp32_ir(c);
     } else {
+      hipLaunchKernelGGL((k_zero<float>), dim3(256), dim3(256), 0, c->stream, c->s[0].u,
+                         (size_t)c->lv[0].N * c->lv[0].P);
       vcycle<float, false>(c, c->s, 0, true);
       const LevelDims &d = c->lv[0];
       hipLaunchKernelGGL(k_add_correction, grid_cols(d.K - 2, d.N), dim3(BX, BY),
@@ -821,7 +846,7 @@ static void launch_plain_dev_start(qdeq_ctx *c, bool fuse) {
     hipLaunchKernelGGL((k_resnorm_partial<true>), dim3(norm_blocks(c)),
                        dim3(NORM_THREADS), 0, c->stream, c->d[0].u, c->d[0].cx,
                        c->d[0].cz, d.N, d.K, d.P, d.DH * d.DH, c->partial, c->s[0].f,
-                       c->s[0].u, (const int *)nullptr);
+                       (const int *)nullptr);
   } else if (fuse) {
     c->fuse_start_next = true;
     return;
@@ -929,7 +954,7 @@ int mg_begin(qdeq_ctx *c) {
     }
     if (in_u) {
       // the plain start back over a candidate that was not chosen
-      hipLaunchKernelGGL(k_restore_if, dim3(std::min(d.N, 1024)), dim3(256), 0,
+      hipLaunchKernelGGL(k_restore_if, dim3(std::min(d.N, 256)), dim3(256), 0,
                          c->stream, c->d[0].u, plain, d.N, d.K, d.P, c->gate + 5);
     } else if (m.cand) {
       // the chosen candidate from r into u
