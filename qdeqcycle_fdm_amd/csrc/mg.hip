@@ -198,8 +198,10 @@ __global__ __launch_bounds__(NORM_THREADS) void k_resnorm_partial(
     const double *__restrict__ u, const double *__restrict__ cx,
     const double *__restrict__ cz, int N, int K, int P, double DH2,
     double *__restrict__ partial, float *__restrict__ r32,
-    const int *__restrict__ gate) {
+    const int *__restrict__ gate, const int *__restrict__ spec, int go) {
   if (gate && gate[0]) return;  // batched solve already converged
+  // a start launched ahead: as in k_start_partials
+  if (spec && spec[go] != 1) return;
   __shared__ double sh[NORM_THREADS];
   double acc = 0.0;
   constexpr int UNR = 4;  // as in k_start_partials
@@ -625,12 +627,13 @@ static void launch_resnorm(qdeq_ctx *c, bool store32) {
     hipLaunchKernelGGL((k_resnorm_partial<true>), dim3(norm_blocks(c)),
                        dim3(NORM_THREADS), 0, c->stream, c->d[0].u, c->d[0].cx,
                        c->d[0].cz, d.N, d.K, d.P, DH2, c->partial, c->s[0].f,
-                       (const int *)c->gate_ptr);
+                       (const int *)c->gate_ptr, (const int *)nullptr, 0);
   else
     hipLaunchKernelGGL((k_resnorm_partial<false>), dim3(norm_blocks(c)),
                        dim3(NORM_THREADS), 0, c->stream, c->d[0].u, c->d[0].cx,
                        c->d[0].cz, d.N, d.K, d.P, DH2, c->partial,
-                       (float *)nullptr, (const int *)c->gate_ptr);
+                       (float *)nullptr, (const int *)c->gate_ptr, (const int *)nullptr,
+                       0);
   launch_norm_final(c, norm_blocks(c));
 }
 
@@ -641,7 +644,7 @@ void launch_resnorm_of(qdeq_ctx *c, const double *u, int off, int slot) {
   hipLaunchKernelGGL((k_resnorm_partial<false>), dim3(norm_blocks(c)),
                      dim3(NORM_THREADS), 0, c->stream, u, c->d[0].cx, c->d[0].cz,
                      d.N, d.K, d.P, d.DH * d.DH, c->partial + off,
-                     (float *)nullptr, (const int *)nullptr);
+                     (float *)nullptr, (const int *)nullptr, (const int *)nullptr, 0);
   hipLaunchKernelGGL(k_norm_final, dim3(1), dim3(NORM_THREADS), 0, c->stream,
                      c->partial + off, norm_blocks(c), c->scal + slot,
                      mb_dev(c) + slot);
@@ -846,7 +849,8 @@ static void launch_plain_dev_start(qdeq_ctx *c, bool fuse) {
     hipLaunchKernelGGL((k_resnorm_partial<true>), dim3(norm_blocks(c)),
                        dim3(NORM_THREADS), 0, c->stream, c->d[0].u, c->d[0].cx,
                        c->d[0].cz, d.N, d.K, d.P, d.DH * d.DH, c->partial, c->s[0].f,
-                       (const int *)nullptr);
+                       (const int *)nullptr,
+                       (const int *)(c->spec_launch ? c->gate : nullptr), c->spec_go);
   } else if (fuse) {
     c->fuse_start_next = true;
     return;
@@ -1044,7 +1048,7 @@ int mg_begin_stage(qdeq_ctx *c, int kind, int s) {
   return QDEQ_OK;
 }
 
-// The next FP64 solve launched ahead, behind the current solve's launched
+// The next solve launched ahead, behind the current solve's launched
 // V-cycles (its fault update already queued by the caller): the plain
 // device start and a first batch, into c->mg_next, on the other mailbox
 // page.  Its kernels go on only if the current solve ends converged with
@@ -1055,6 +1059,7 @@ int mg_begin_stage(qdeq_ctx *c, int kind, int s) {
 int mg_begin_spec(qdeq_ctx *c, int go) {
   MgSolve &m = c->mg_next;
   m = MgSolve{};
+  m.ir = c->cfg.precision == QDEQ_PREC_FP32_IR;
   m.dev_start = true;
   m.page = 1 - c->mg.page;
   c->mb_page = m.page;

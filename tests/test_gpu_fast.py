@@ -434,6 +434,52 @@ def test_stages_launched_ahead_equal_waiting_runs(n, levels, timed, monkeypatch)
     assert sa["next_step"] > 0.3 * 120
 
 
+@pytest.mark.parametrize("n,levels,kw", [
+    (257, 5, dict(precision=config.PREC_FP32_IR)),
+    (65, 3, dict(precision=config.PREC_FP32_IR)),
+    (257, 5, dict(precision=config.PREC_FP32_IR, events=True)),
+])
+def test_refinement_launched_ahead_equals_waiting_runs(n, levels, kw, monkeypatch):
+    """The same for FP32 refinement, whose start and stop tests are kernels of
+    their own."""
+    _ahead_equals_waiting(n, levels, kw, monkeypatch)
+
+
+def _ahead_equals_waiting(n, levels, kw, monkeypatch):
+    pb = config.make_bp1_problem(n, basin=True, levels=levels,
+                                 tol_mode=config.TOL_REL, tol=1e-10)
+    me = oracle.mu_equi(pb.mu)
+    kw = dict(kw)
+    slots, events = kw.pop("slots", 0), kw.pop("events", False)
+    runs = []
+    for spec in (True, False):
+        if spec:
+            monkeypatch.delenv("QDEQ_SPECULATE", raising=False)
+        else:
+            monkeypatch.setenv("QDEQ_SPECULATE", "0")
+        with lib.Engine(pb, me, **{**PROD, **kw}) as eng:
+            eng.rk43_setup()
+            if slots:
+                eng.projection_enable(slots)
+            if events:
+                eng.events_enable(1e-3)
+            eng.rk43_step(70)
+            eng.rk43_step(1)
+            eng.rk43_step(50)
+            runs.append((eng.state(), eng.launch_ahead_stats(),
+                         eng.projection_stats() if slots else None))
+    (a, sa, pa), (b, sb, pb_) = runs
+    for key in ("t", "dt", "vcycles", "solves", "attempts"):
+        assert a["info"][key] == b["info"][key], key
+    for k in ("slip", "psi", "V", "U"):
+        np.testing.assert_array_equal(a[k], b[k])
+    assert pa == pb_
+    assert sb == {"taken": 0, "abandoned": 0, "next_step": 0}
+    assert sa["taken"] > 0.5 * a["info"]["solves"]
+    assert sa["abandoned"] > 0
+    assert (sa["next_step"] > 0.3 * 120) != events
+
+
 def test_next_step_launched_ahead_ends_at_tmax_and_stays_off_between_records(
         monkeypatch):
     """Stage 2 of the next step is queued behind an accepted step's final
