@@ -793,17 +793,27 @@ static int rk_readback_ready(qdeq_ctx *c, bool block, int *ready) {
 
 // Work may be launched ahead of a decision the host has not read yet for a
 // single simulation launching kernel by kernel (start decided on the device,
-// no candidate start, no fault-update timing) with nothing else launched
-// ahead.  QDEQ_SPECULATE=0 turns it off.
+// also from the projection, not from the learned guess; no fault-update
+// timing) with nothing else launched ahead.  QDEQ_SPECULATE=0 turns it off.
 static bool spec_base_allowed(const qdeq_ctx *c) {
   return !c->spec_off && launch_direct(c) && !stage_graphs(c) && device_start(c) &&
-         c->timing != QDEQ_TIME_FAULT && c->proj_slots == 0 && (c->guess == nullptr || c->guess_mode == QDEQ_GUESS_OFF) &&
+         c->timing != QDEQ_TIME_FAULT && (c->proj_slots == 0 || device_start_cand(c)) && (c->guess == nullptr || c->guess_mode == QDEQ_GUESS_OFF) &&
          !c->spec_pending;
 }
 // The next stage behind the current solve: its V-cycles in flight, started
-// on the device from the plain start.
+// on the device.
 static bool spec_allowed(const qdeq_ctx *c) {
-  return spec_base_allowed(c) && c->mg.phase == 2 && c->mg.dev_start && !c->mg.cand;
+  return spec_base_allowed(c) && c->mg.phase == 2 && c->mg.dev_start;
+}
+// What the current solve's end needs before its fault update may be queued
+// behind it: the projection keeps the solution, and then makes the last stop
+// test.
+static int queue_solve_end(qdeq_ctx *c, StopArgs *stop) {
+  *stop = mg_take_stop(c, c->mg);
+  if (c->proj_slots == 0) return QDEQ_OK;
+  const int st = proj_after_solve_ahead(c, *stop);
+  *stop = StopArgs{};
+  return st;
 }
 
 // Whether the accepted attempt's commit and final stage-1 solve may be
@@ -882,6 +892,7 @@ static int rk_advance(qdeq_ctx *c, bool block, int *done) {
           c->mg_next.stop_due = false;  // moved with it
           c->mb_page = c->mg.page;
           c->spec_pending = false;
+          proj_ahead_done(c, true);
           c->spec_taken++;
           if (r.s == 2 && !r.final_stage) c->spec_taken_next++;
           r.spec = false;
@@ -911,7 +922,9 @@ static int rk_advance(qdeq_ctx *c, bool block, int *done) {
           // stage s + 1 queued behind this solve: the fault update of stage
           // s with stage s + 1's state, its start and first batch, all
           // gated on this solve's outcome
-          launch_update_stage(c, r.s, c->gate, mg_take_stop(c, c->mg));
+          StopArgs stop;
+          if ((st = queue_solve_end(c, &stop))) return st;
+          launch_update_stage(c, r.s, c->gate, stop);
           const int key = c->solve_key;
           c->solve_key = r.s + 1;
           st = mg_begin_spec(c);
@@ -924,7 +937,9 @@ static int rk_advance(qdeq_ctx *c, bool block, int *done) {
           // state, start and first batch, with the dt the step will hand on
           double dt = step_finish_dt(c);
           if (c->t + dt > p.tmax) dt = p.tmax - c->t;
-          launch_update_next(c, c->t, dt, c->gate, mg_take_stop(c, c->mg));
+          StopArgs stop;
+          if ((st = queue_solve_end(c, &stop))) return st;
+          launch_update_next(c, c->t, dt, c->gate, stop);
           const int key = c->solve_key;
           c->solve_key = 2;
           st = mg_begin_spec(c);
@@ -939,15 +954,18 @@ static int rk_advance(qdeq_ctx *c, bool block, int *done) {
         if (r.spec && !c->spec_pending) {
           r.spec = false;
           c->spec_abandoned++;
+          proj_ahead_done(c, false);
         }
         if (st) {
           r.spec = false;
           c->spec_pending = false;
+          proj_ahead_done(c, false);
           return st;
         }
         if (!sdone) return QDEQ_OK;
         if ((st = guess_after_solve(c))) return st;
-        if ((st = proj_after_solve(c))) return st;
+        // (already queued with a stage launched ahead)
+        if (!r.spec && (st = proj_after_solve(c))) return st;
         if (c->timing == QDEQ_TIME_FAULT && (c->timed_seq++ % 8) == 0) {
           QDEQ_HIP(c, hipEventRecord(c->ev_t[0][0], c->stream));
           launch_fault_update(c, r.s);
@@ -1018,6 +1036,7 @@ static int rk_advance(qdeq_ctx *c, bool block, int *done) {
           r.spec = false;
           c->spec_pending = false;
           c->spec_abandoned++;
+          proj_ahead_done(c, false);
           mg_flush_stop(c, c->mg_next);
         }
         if (!accept) {

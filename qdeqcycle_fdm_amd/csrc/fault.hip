@@ -274,44 +274,6 @@ __device__ inline NodeRates update_node(int k, const NodeIn &n, const UpdateArgs
   return NodeRates{Vn, dp};
 }
 
-// Whether the work queued behind a solve goes on: with stop.nb it runs the
-// solve's last stop test itself (k_norm_gate's on one partial per thread, in
-// its order, so every workgroup takes the same decision; workgroup 0 records
-// it; the cap cannot be reached), else it reads the outcome in spec[2].
-// gate[0] is not written here: the start that follows reads gate[2] and sets
-// it.  Ends with a barrier; every thread of the workgroup calls it.
-__device__ inline bool solve_converged(const StopArgs &stop, const int *spec) {
-  if (stop.nb == 0) return !spec || spec[2] == 1;
-  __shared__ double sh[16];
-  const int tid = threadIdx.x;
-  const bool stopped = stop.gate[0] != 0;
-  const int before = stop.gate[2];
-  const double p = tid < stop.nb ? stop.part[tid] : 0.0;
-  const double v = sqrt(block_sum1(0.0 + p, sh));
-  const double thr = stop.rel ? stop.tol * stop.scal[SC_NORM0] : stop.tol;
-  int code = 0;
-  if (isnan(v) || isinf(v))
-    code = 2;
-  else if (!(v > thr))
-    code = 1;
-  if (blockIdx.x == 0 && tid == 0) {
-    const int seq = stop.gate[3] + 1;
-    stop.gate[3] = seq;
-    if (!stopped) {
-      const int cnt = stop.gate[1] + 1;
-      stop.gate[1] = cnt;
-      stop.gate[2] = code;
-      stop.scal[SC_NORM] = v;
-      stop.mb[SC_NORM] = v;
-      stop.mb[MB_COUNT] = (double)cnt;
-      stop.mb[MB_CODE] = (double)code;
-    }
-    __threadfence_system();
-    stop.mb[MB_SEQ] = (double)seq;
-  }
-  return stopped ? before == 1 : code == 1;
-}
-
 __global__ void k_fault_update(const double *u, int P, int nk, UpdateArgs ua) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x + 1;
   if (k > nk) return;

@@ -401,6 +401,7 @@ __global__ __launch_bounds__(NORM_THREADS) void k_start_gate(
   if (spec && gate[spec] != 1) {
     if (threadIdx.x == 0) {
       gate[0] = 1;
+      gate[4] = gate[5] = 0;  // nothing to copy or restore
       const int seq = gate[3] + 1;
       gate[3] = seq;
       mb[MB_CODE] = 4.0;
@@ -866,6 +867,36 @@ static void launch_plain_dev_start(qdeq_ctx *c, bool fuse) {
                      c->scal, mb_dev(c), c->gate, c->spec_launch ? c->spec_go : 0);
 }
 
+// The device start of a solve with a candidate: written over u's interior
+// with the plain start's interior kept at plain_interior (the projection
+// start), or in r (the learned guess).
+static void launch_cand_dev_start(qdeq_ctx *c) {
+  const LevelDims &d = c->lv[0];
+  const int rel = c->cfg.tol_mode == QDEQ_TOL_REL ? 1 : 0;
+  const bool in_u = c->cand_in_u;
+  c->cand_in_u = false;
+  const double *plain = in_u ? c->plain_interior : c->d[0].u;
+  const double *cand = in_u ? c->d[0].u : c->d[0].r;
+  hipLaunchKernelGGL(k_start_partials<true>, dim3(norm_blocks(c)), dim3(NORM_THREADS), 0,
+                     c->stream, plain, c->d[0].u, cand, c->d[0].cx, c->d[0].cz, d.N, d.K,
+                     d.P, d.DH * d.DH, rel, c->partial,
+                     (const int *)(c->spec_launch ? c->gate : nullptr), c->spec_go);
+  hipLaunchKernelGGL(k_start_gate, dim3(1), dim3(NORM_THREADS), 0, c->stream, c->partial,
+                     norm_blocks(c), 1, rel, c->cfg.tol, c->cfg.max_vcycles, c->scal,
+                     mb_dev(c), c->gate, c->spec_launch ? c->spec_go : 0);
+  if (in_u) {
+    // the plain start back over a candidate that was not chosen
+    hipLaunchKernelGGL(k_restore_if, dim3(std::min(d.N, 256)), dim3(256), 0, c->stream,
+                       c->d[0].u, plain, d.N, d.K, d.P, c->gate + 5);
+  } else {
+    // the chosen candidate from r into u
+    const size_t n = (size_t)d.N * d.P;
+    const unsigned blocks = (unsigned)std::min<size_t>((n + 255) / 256, 1024);
+    hipLaunchKernelGGL(k_copy_if, dim3(blocks), dim3(256), 0, c->stream, c->d[0].u,
+                       c->d[0].r, n, c->gate + 4);
+  }
+}
+
 StopArgs mg_take_stop(qdeq_ctx *c, MgSolve &m) {
   StopArgs a;
   if (!m.stop_due) return a;
@@ -934,39 +965,12 @@ int mg_begin(qdeq_ctx *c) {
   if (m.dev_start) {
     // norms, start choice and stop test on the device; the first batch is
     // launched at once, sized from the last solve
-    // the candidate is either written over u's interior with the plain
-    // start's interior kept at plain_interior (the projection start), or in
-    // r (the learned guess)
-    const LevelDims &d = c->lv[0];
-    const int rel = c->cfg.tol_mode == QDEQ_TOL_REL ? 1 : 0;
-    const bool in_u = m.cand && c->cand_in_u;
-    c->cand_in_u = false;
-    const double *plain = in_u ? c->plain_interior : c->d[0].u;
-    const double *cand = !m.cand ? nullptr : (in_u ? c->d[0].u : c->d[0].r);
     // a plain start launched kernel by kernel: its norms and test ride on
     // the first V-cycle's down kernels (the same decisions, no start launches)
-    if (!cand) {
+    if (m.cand)
+      launch_cand_dev_start(c);
+    else
       launch_plain_dev_start(c, launch_direct(c) && fused_start_fits(c));
-    } else {
-      hipLaunchKernelGGL(k_start_partials<true>, dim3(norm_blocks(c)), dim3(NORM_THREADS), 0,
-                         c->stream, plain, c->d[0].u, cand, c->d[0].cx, c->d[0].cz,
-                         d.N, d.K, d.P, d.DH * d.DH, rel, c->partial, (const int *)nullptr,
-                         2);
-      hipLaunchKernelGGL(k_start_gate, dim3(1), dim3(NORM_THREADS), 0, c->stream,
-                         c->partial, norm_blocks(c), 1, rel, c->cfg.tol,
-                         c->cfg.max_vcycles, c->scal, mb_dev(c), c->gate, 0);
-    }
-    if (in_u) {
-      // the plain start back over a candidate that was not chosen
-      hipLaunchKernelGGL(k_restore_if, dim3(std::min(d.N, 256)), dim3(256), 0,
-                         c->stream, c->d[0].u, plain, d.N, d.K, d.P, c->gate + 5);
-    } else if (m.cand) {
-      // the chosen candidate from r into u
-      const size_t n = (size_t)d.N * d.P;
-      const unsigned blocks = (unsigned)std::min<size_t>((n + 255) / 256, 1024);
-      hipLaunchKernelGGL(k_copy_if, dim3(blocks), dim3(256), 0, c->stream,
-                         c->d[0].u, c->d[0].r, n, c->gate + 4);
-    }
     c->seq_issued += 1;
     QDEQ_HIP(c, hipGetLastError());
     int st = launch_batch(c, first_batch(c));
@@ -1049,8 +1053,8 @@ int mg_begin_stage(qdeq_ctx *c, int kind, int s) {
 }
 
 // The next solve launched ahead, behind the current solve's launched
-// V-cycles (its fault update already queued by the caller): the plain
-// device start and a first batch, into c->mg_next, on the other mailbox
+// V-cycles (its fault update already queued by the caller): the device start,
+// plain or from the projection, and a first batch, into c->mg_next, on the other mailbox
 // page.  Its kernels go on only if the current solve ends converged with
 // the work already queued; if the current solve needs more V-cycles the
 // start abandons itself (outcome 4) and mg_poll resumes the gate before the
@@ -1065,9 +1069,15 @@ int mg_begin_spec(qdeq_ctx *c, int go) {
   c->mb_page = m.page;
   c->spec_launch = true;
   c->spec_go = go;
-  launch_plain_dev_start(c, fused_start_fits(c));
+  int st = proj_before_solve(c);
+  m.cand = c->cand_pending;
+  c->cand_pending = false;
+  if (m.cand)
+    launch_cand_dev_start(c);
+  else
+    launch_plain_dev_start(c, fused_start_fits(c));
   c->seq_issued += 1;
-  const int st = launch_batch_of(c, m, first_batch(c), true);
+  if (st == QDEQ_OK) st = launch_batch_of(c, m, first_batch(c), true);
   c->spec_launch = false;
   c->spec_go = 2;
   c->fuse_start_next = false;

@@ -21,6 +21,7 @@
 // themselves, so the previous solution (the plain start's interior) is
 // always at hand.
 
+#include <algorithm>
 #include <cmath>
 #include <string>
 
@@ -227,12 +228,15 @@ __global__ __launch_bounds__(PROJ_THREADS) void k_proj_coef(
 // Start on the interior columns (1..K-2) into cand; with copy_bnd the fault
 // and remote columns (and the pitch padding) are copied from u as well.
 // cand may be u itself (interior points only are written then).  The weight
-// w of W_R is formed by every thread alike, in the order above.
+// w of W_R is formed by every thread alike, in the order above.  Launched
+// ahead (spec), only if what it waits on went through.
 __global__ void k_proj_apply(const double *u, const double *__restrict__ wr,
                              const double *__restrict__ ring, size_t rstride,
                              const double *__restrict__ rr, ProjSlots sl,
                              const double *__restrict__ coef, int N, int K, int P,
-                             double *cand, int copy_bnd, double inject) {
+                             double *cand, int copy_bnd, double inject,
+                             const int *__restrict__ spec, int go) {
+  if (spec && spec[go] != 1) return;
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   const int j = blockIdx.y;
   if (k >= P || j >= N) return;
@@ -255,16 +259,22 @@ __global__ void k_proj_apply(const double *u, const double *__restrict__ wr,
 }
 
 // Stores the solution just found, its fault column and its remote value.
-__global__ void k_proj_commit(const double *__restrict__ u, int N, int K, int P,
-                              double *__restrict__ dst, double *__restrict__ g,
-                              double *__restrict__ r) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  const int j = blockIdx.y;
-  if (k >= P || j >= N) return;
-  const size_t c = (size_t)j * P + k;
-  dst[c] = u[c];
-  if (k == 0) g[j] = u[c];
-  if (j == 0 && k == K - 1) r[0] = u[c];
+// Launched behind a solve in flight (spec), only if that solve converged; its
+// last stop test runs here when it is due.  A workgroup per row, so that few
+// repeat the test.
+constexpr int COMMIT_THREADS = 256;
+__global__ __launch_bounds__(COMMIT_THREADS) void k_proj_commit(
+    const double *__restrict__ u, int N, int K, int P, double *__restrict__ dst,
+    double *__restrict__ g, double *__restrict__ r, const int *spec, StopArgs stop) {
+  if (!solve_converged(stop, spec)) return;
+  for (int j = blockIdx.x; j < N; j += gridDim.x)
+    for (int k = threadIdx.x; k < P; k += COMMIT_THREADS) {
+      const size_t c = (size_t)j * P + k;
+      const double v = u[c];
+      dst[c] = v;
+      if (k == 0) g[j] = v;
+      if (j == 0 && k == K - 1) r[0] = v;
+    }
 }
 
 }  // namespace
@@ -304,6 +314,7 @@ static hipError_t coef_lds_attr(int cnt, int N) {
 void proj_reset(qdeq_ctx *c) {
   c->proj_count = 0;
   c->proj_head = 0;
+  c->proj_undo.on = false;
 }
 
 void proj_free(qdeq_ctx *c) {
@@ -322,8 +333,18 @@ static ProjSlots proj_order(const qdeq_ctx *c) {
   return sl;
 }
 
+// The state that an abandoned launch ahead goes back to.
+static void proj_save(qdeq_ctx *c) {
+  if (c->proj_undo.on) return;
+  c->proj_undo.on = true;
+  c->proj_undo.count = c->proj_count;
+  c->proj_undo.head = c->proj_head;
+  c->proj_undo.predicted = c->g_predicted;
+}
+
 int proj_before_solve(qdeq_ctx *c) {
   if (c->proj_slots < 1 || c->proj_count < 1) return QDEQ_OK;
+  if (c->spec_launch) proj_save(c);
   const LevelDims &d = c->lv[0];
   const ProjSlots sl = proj_order(c);
   // the start's norms come with the solve (the same test as mg_begin's)
@@ -339,7 +360,8 @@ int proj_before_solve(qdeq_ctx *c) {
   hipLaunchKernelGGL(k_proj_apply, grd, blk, 0, c->stream, c->d[0].u, c->proj_wr,
                      c->proj_u, (size_t)d.N * d.P, c->proj_r, sl, c->proj_coef,
                      d.N, d.K, d.P, dev ? c->d[0].u : c->d[0].r, dev ? 0 : 1,
-                     c->proj_inject);
+                     c->proj_inject, (const int *)(c->spec_launch ? c->gate : nullptr),
+                     c->spec_go);
   if (!dev) launch_resnorm_of(c, c->d[0].r, 2 * kNormCap, SC_NORM_PRED);
   QDEQ_HIP(c, hipGetLastError());
   c->cand_pending = true;
@@ -349,18 +371,36 @@ int proj_before_solve(qdeq_ctx *c) {
   return QDEQ_OK;
 }
 
-int proj_after_solve(qdeq_ctx *c) {
-  if (c->proj_slots < 1) return QDEQ_OK;
+static int proj_commit(qdeq_ctx *c, const int *spec, const StopArgs &stop) {
   const LevelDims &d = c->lv[0];
   const int slot = c->proj_head;
-  const dim3 blk(256), grd((d.P + 255) / 256, d.N);
-  hipLaunchKernelGGL(k_proj_commit, grd, blk, 0, c->stream, c->d[0].u, d.N, d.K, d.P,
-                     c->proj_u + (size_t)slot * d.N * d.P,
-                     c->proj_g + (size_t)slot * d.N, c->proj_r + slot);
+  hipLaunchKernelGGL(k_proj_commit, dim3(std::min(d.N, 1024)), dim3(COMMIT_THREADS), 0,
+                     c->stream, c->d[0].u, d.N, d.K, d.P,
+                     c->proj_u + (size_t)slot * d.N * d.P, c->proj_g + (size_t)slot * d.N,
+                     c->proj_r + slot, spec, stop);
   QDEQ_HIP(c, hipGetLastError());
   c->proj_head = (c->proj_head + 1) % c->proj_slots;
   if (c->proj_count < c->proj_slots) c->proj_count++;
   return QDEQ_OK;
+}
+
+int proj_after_solve(qdeq_ctx *c) {
+  if (c->proj_slots < 1) return QDEQ_OK;
+  return proj_commit(c, nullptr, StopArgs{});
+}
+
+int proj_after_solve_ahead(qdeq_ctx *c, const StopArgs &stop) {
+  proj_save(c);
+  return proj_commit(c, c->gate, stop);
+}
+
+void proj_ahead_done(qdeq_ctx *c, bool taken) {
+  if (!taken && c->proj_undo.on) {
+    c->proj_count = c->proj_undo.count;
+    c->proj_head = c->proj_undo.head;
+    c->g_predicted = c->proj_undo.predicted;
+  }
+  c->proj_undo.on = false;
 }
 
 }  // namespace qdeq

@@ -287,6 +287,12 @@ struct qdeq_ctx {
   // each), their fault columns and remote values, the fit's coefficients,
   // and W_R
   int proj_slots = 0, proj_count = 0, proj_head = 0;
+  // the ring and the count of predictions before the work launched ahead
+  struct {
+    bool on = false;
+    int count = 0, head = 0;
+    long long predicted = 0;
+  } proj_undo;
   double proj_inject = 1.0;  // test hook: scales the start's change
   double *proj_u = nullptr, *proj_g = nullptr, *proj_r = nullptr,
          *proj_coef = nullptr, *proj_wr = nullptr;
@@ -340,6 +346,10 @@ int solve_unit_remote(qdeq_ctx *c, double *dst);
 // projection start (proj.hip)
 int proj_before_solve(qdeq_ctx *c);
 int proj_after_solve(qdeq_ctx *c);
+// The same behind a solve in flight (its last stop test with it, if due),
+// and the end of what was launched ahead: taken over or abandoned.
+int proj_after_solve_ahead(qdeq_ctx *c, const StopArgs &stop);
+void proj_ahead_done(qdeq_ctx *c, bool taken);
 void proj_reset(qdeq_ctx *c);
 void proj_free(qdeq_ctx *c);
 
@@ -465,6 +475,44 @@ __device__ inline double block_sum1(double v, double *sh) {
   double a[1] = {v};
   block_sums<1>(a, sh);
   return a[0];
+}
+
+// Whether the work queued behind a solve goes on: with stop.nb it runs the
+// solve's last stop test itself (k_norm_gate's on one partial per thread, in
+// its order, so every workgroup takes the same decision; workgroup 0 records
+// it; the cap cannot be reached), else it reads the outcome in spec[2].
+// gate[0] is not written here: the start that follows reads gate[2] and sets
+// it.  Ends with a barrier; every thread of the workgroup calls it.
+__device__ inline bool solve_converged(const StopArgs &stop, const int *spec) {
+  if (stop.nb == 0) return !spec || spec[2] == 1;
+  __shared__ double sh[16];
+  const int tid = threadIdx.x;
+  const bool stopped = stop.gate[0] != 0;
+  const int before = stop.gate[2];
+  const double p = tid < stop.nb ? stop.part[tid] : 0.0;
+  const double v = sqrt(block_sum1(0.0 + p, sh));
+  const double thr = stop.rel ? stop.tol * stop.scal[SC_NORM0] : stop.tol;
+  int code = 0;
+  if (isnan(v) || isinf(v))
+    code = 2;
+  else if (!(v > thr))
+    code = 1;
+  if (blockIdx.x == 0 && tid == 0) {
+    const int seq = stop.gate[3] + 1;
+    stop.gate[3] = seq;
+    if (!stopped) {
+      const int cnt = stop.gate[1] + 1;
+      stop.gate[1] = cnt;
+      stop.gate[2] = code;
+      stop.scal[SC_NORM] = v;
+      stop.mb[SC_NORM] = v;
+      stop.mb[MB_COUNT] = (double)cnt;
+      stop.mb[MB_CODE] = (double)code;
+    }
+    __threadfence_system();
+    stop.mb[MB_SEQ] = (double)seq;
+  }
+  return stopped ? before == 1 : code == 1;
 }
 
 // Entries of c->partial: the FP64 fast cycle's level-0 up kernel writes one

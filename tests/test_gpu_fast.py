@@ -438,10 +438,14 @@ def test_stages_launched_ahead_equal_waiting_runs(n, levels, timed, monkeypatch)
     (257, 5, dict(precision=config.PREC_FP32_IR)),
     (65, 3, dict(precision=config.PREC_FP32_IR)),
     (257, 5, dict(precision=config.PREC_FP32_IR, events=True)),
+    (257, 5, dict(slots=8)),
+    (129, 4, dict(slots=2, events=True)),
+    (65, 3, dict(slots=1)),
 ])
-def test_refinement_launched_ahead_equals_waiting_runs(n, levels, kw, monkeypatch):
+def test_other_starts_launched_ahead_equal_waiting_runs(n, levels, kw, monkeypatch):
     """The same for FP32 refinement, whose start and stop tests are kernels of
-    their own."""
+    their own, and with the projection start, whose ring of solutions goes
+    back when a stage is abandoned."""
     _ahead_equals_waiting(n, levels, kw, monkeypatch)
 
 
