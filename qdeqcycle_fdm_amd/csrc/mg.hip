@@ -23,7 +23,7 @@ constexpr int BX = 64, BY = 4;          // 256-thread tiles, 64-wide rows
 // NORM_BLOCKS: capacity of the row-partial layout; a launch uses
 // norm_blocks(c) = min(N, NORM_BLOCKS) blocks, one row each up to 2048 rows
 // (one block with twice the rows of the others would set the time)
-constexpr int NORM_BLOCKS = kNormCap, NORM_THREADS = 256;
+constexpr int NORM_BLOCKS = kNormCap, NORM_THREADS = kNormThreads;
 
 // ---------------------------------------------------------------------------
 // Kernels
@@ -173,22 +173,6 @@ __device__ inline int band_row() {
   return x * (n >> 3) + min(x, n & 7) + ((int)blockIdx.x >> 3);
 }
 
-// a[t] + a[t + NORM_THREADS] + ... of thread t, from 0.0 in this order, with
-// the loads of eight terms in flight (2048 partial sums: the stop test's
-// kernel 5.0 -> 4.1 us).
-__device__ inline double strided_sum(const double *__restrict__ a, int n) {
-  double acc = 0.0;
-  for (int i0 = threadIdx.x; i0 < n; i0 += 8 * NORM_THREADS) {
-    double v[8];
-#pragma unroll
-    for (int q = 0; q < 8; q++) v[q] = a[min(i0 + q * NORM_THREADS, n - 1)];
-#pragma unroll
-    for (int q = 0; q < 8; q++)
-      if (i0 + q * NORM_THREADS < n) acc += v[q];
-  }
-  return acc;
-}
-
 // Level-0 residual norm, pass 1: fixed-grid partial sums of r^2 (the
 // reference uses calcuDelta_dev + cublasDnrm2, odeSolver.cpp:693-700).
 // Optionally stores r as FP32 (the IR right-hand side).  Deterministic: fixed
@@ -263,7 +247,7 @@ __global__ __launch_bounds__(NORM_THREADS) void k_norm_final(
     const double *__restrict__ partial, int n, double *__restrict__ out,
     double *__restrict__ mb) {
   __shared__ double sh[NORM_THREADS];
-  const double s = block_sum_256(strided_sum(partial, n), sh);
+  const double s = block_sum_256(strided_sum(partial, n, threadIdx.x), sh);
   if (threadIdx.x == 0) {
     const double v = sqrt(s);
     out[0] = v;
@@ -284,7 +268,7 @@ __global__ __launch_bounds__(NORM_THREADS) void k_norm_gate(
     int cap) {
   __shared__ double sh[NORM_THREADS];
   const bool skip = gate[0] != 0;
-  const double s = block_sum_256(skip ? 0.0 : strided_sum(partial, n), sh);
+  const double s = block_sum_256(skip ? 0.0 : strided_sum(partial, n, threadIdx.x), sh);
   if (threadIdx.x == 0) {
     const int seq = gate[3] + 1;
     gate[3] = seq;
@@ -412,9 +396,9 @@ __global__ __launch_bounds__(NORM_THREADS) void k_start_gate(
   }
   // the three sums of k_norm_final's order, in one tree
   __shared__ double sh[3][NORM_THREADS];
-  double v3[3] = {strided_sum(partial, nb),
-                  rel ? strided_sum(partial + NORM_BLOCKS, BDRES_BLOCKS) : 0.0,
-                  cand ? strided_sum(partial + 2 * NORM_BLOCKS, nb) : 0.0};
+  double v3[3] = {strided_sum(partial, nb, threadIdx.x),
+                  rel ? strided_sum(partial + NORM_BLOCKS, BDRES_BLOCKS, threadIdx.x) : 0.0,
+                  cand ? strided_sum(partial + 2 * NORM_BLOCKS, nb, threadIdx.x) : 0.0};
   block_sums<3>(v3, &sh[0][0]);
   const double su = v3[0], sb = v3[1], sc = v3[2];
   if (threadIdx.x == 0) {
@@ -1017,6 +1001,8 @@ int mg_begin_stage(qdeq_ctx *c, int kind, int s) {
   m.dev_start = true;
   m.start_read = false;
   const int B = first_batch(c);
+  // the stop tests that the graph's next V-cycle runs (as in launch_batch_of)
+  const int nfold = fold_fits(c) ? std::min(B, c->cfg.max_vcycles) - 1 : 0;
   const int gk = (kind * 8 + s) * 8 + B;
   auto it = c->g_stage.find(gk);
   hipGraphExec_t ex = nullptr;
@@ -1032,7 +1018,12 @@ int mg_begin_stage(qdeq_ctx *c, int kind, int s) {
         launch_stage(c, s);
       launch_plain_dev_start(c, !m.ir && fused_start_fits(c));
       c->gate_ptr = c->gate;
-      for (int i = 0; i < B; i++) launch_iteration(c);
+      for (int i = 0; i < B; i++) {
+        c->fold_next = i > 0 && i <= nfold;
+        c->skip_gate = i < nfold;
+        launch_iteration(c);
+      }
+      c->fold_next = c->skip_gate = false;
       c->gate_ptr = nullptr;
       c->fuse_start_next = false;
       e = hipStreamEndCapture(c->stream, &g);
@@ -1045,6 +1036,7 @@ int mg_begin_stage(qdeq_ctx *c, int kind, int s) {
     c->g_stage[gk] = ex;
   }
   QDEQ_HIP(c, hipGraphLaunch(ex, c->stream));
+  c->folded_tests += std::max(nfold, 0);
   c->seq_issued += 1 + B;
   m.launched = B;
   m.seq_target = c->seq_issued;
@@ -1160,7 +1152,7 @@ static int launch_batch_of(qdeq_ctx *c, MgSolve &m, int k, bool allow_sample) {
   m.sample = false;
   // the stop test of every V-cycle but the batch's last (and one that could
   // reach the V-cycle cap) runs in the next V-cycle's level-0 down kernel
-  const bool fold = fold_fits(c), defer = defer_fits(c);
+  const bool fold = fold_fits(c) && launch_direct(c), defer = defer_fits(c);
   bool folded = false;
   struct FoldReset {  // also on an error return: no later launch folds
     qdeq_ctx *c;

@@ -478,7 +478,8 @@ struct StartArgs {
   // batch behind it, the mailbox step carries outcome 4)
   int spec;
   // DOWN_PLAIN at level 0: the stop test of the previous V-cycle (that of
-  // k_norm_gate, on its nb <= 256 norm partials at part) runs here
+  // k_norm_gate, on its nb norm partials at part, at most 256 in FP64) runs
+  // here
   int fold;
 };
 
@@ -502,7 +503,8 @@ __global__ __launch_bounds__(TILE_THREADS) void k_down(
   const int nthr = blockDim.x * blockDim.y;
   const int ltid = threadIdx.y * blockDim.x + threadIdx.x;
   const bool wg0 = blockIdx.x == 0 && blockIdx.y == 0 && ltid == 0;
-  const bool folding = SMODE == DOWN_PLAIN && !HAS_F && sa.fold;
+  // (FP64 has no right-hand side on level 0, FP32 refinement has one)
+  const bool folding = SMODE == DOWN_PLAIN && (!HAS_F || !EXACT) && sa.fold;
   // whether this launch does nothing: the solve has stopped, or (launched
   // ahead) what it waits on did not go through
   bool leave = false;
@@ -519,10 +521,11 @@ __global__ __launch_bounds__(TILE_THREADS) void k_down(
     quad_load<T, HAS_F>(t, q[i], uin, f, cx, cz, N, K, P, zero_u != 0);
   }
   // folded stop test: each of k_norm_gate's 256 threads (the first four
-  // wavefronts here) loads its partial with the tile and sums in
+  // wavefronts here) loads its partials with the tile and sums in
   // k_norm_gate's order, so every workgroup takes the same decision
   double fold_p = 0.0;
-  if (folding && ltid < sa.nb) fold_p = sa.part[ltid];
+  if (folding && EXACT && ltid < sa.nb) fold_p = 0.0 + sa.part[ltid];
+  if (folding && !EXACT && ltid < 256) fold_p = strided_sum(sa.part, sa.nb, ltid);
   // the start norms from the level-0 tiles' partials, summed by the whole
   // workgroup (every workgroup alike), four loads of a thread in flight
   double v2[2] = {0.0, 0.0};
@@ -550,7 +553,7 @@ __global__ __launch_bounds__(TILE_THREADS) void k_down(
     one_quad_at_a_time<T, S>();
   }
   if (folding && ltid < 256) {
-    const double w = wave_sum(0.0 + fold_p);
+    const double w = wave_sum(fold_p);
     if ((ltid & 63) == 0) sdec[ltid >> 6] = w;
   }
   if (SMODE == START_TEST)
@@ -1386,11 +1389,10 @@ static void launch_down(qdeq_ctx *c, LevelBufs<T> *B, int l, bool has_f,
     sa.cap = c->cfg.max_vcycles;
     sa.tol = c->cfg.tol;
   }
-  if (smode == DOWN_PLAIN && l == 0 && !has_f && c->fold_next && c->gate_ptr) {
-    const TileShape u0 = tile_shape(c, 0, false);
+  if (smode == DOWN_PLAIN && l == 0 && c->fold_next && c->gate_ptr) {
     sa.fold = 1;
     sa.part = c->partial;
-    sa.nb = ((d.K + u0.tx - 1) / u0.tx) * ((d.N + u0.ty - 1) / u0.ty);
+    sa.nb = norm_parts(c);
     sa.scal = c->scal;
     sa.mb = mb_dev(c);
     sa.gate = c->gate;
@@ -1403,28 +1405,40 @@ static void launch_down(qdeq_ctx *c, LevelBufs<T> *B, int l, bool has_f,
                      B[l].u, B[l].r, sa);
 }
 
-// Norm partials of an FP64 V-cycle on the tile kernels: the level-0 tiles of
-// its last launch.
+// Norm partials of a V-cycle on the tile kernels: the level-0 tiles of its last
+// launch in FP64, the rows of the FP64 residual in FP32 refinement.
 int norm_parts(const qdeq_ctx *c) {
+  if (c->cfg.precision == QDEQ_PREC_FP32_IR) return norm_blocks(c);
   const LevelDims &d = c->lv[0];
   const TileShape up = use_tiled(c) ? tile_shape(c, 0, false) : c->ref_plan[0].sh;
   return ((d.K + up.tx - 1) / up.tx) * ((d.N + up.ty - 1) / up.ty);
 }
 
-// Whether a kernel that follows a V-cycle launched kernel by kernel may run
-// its stop test: the FP64 tile kernels and at most 256 norm partials
-// (k_norm_gate's threads each sum one).
-bool defer_fits(const qdeq_ctx *c) {
-  return !c->fold_off && c->cfg.precision == QDEQ_PREC_FP64 && launch_direct(c) &&
-         (use_tiled(c) || use_ref_tiles(c)) && norm_parts(c) <= 256;
+// Whether a V-cycle's stop test may run in a kernel behind it: that of the tile
+// kernels, in FP64 with at most 256 norm partials (one for each of
+// k_norm_gate's threads; a register-bound kernel sums no more).
+static bool test_moves(const qdeq_ctx *c) {
+  return !c->fold_off && (use_tiled(c) || use_ref_tiles(c)) &&
+         (c->cfg.precision == QDEQ_PREC_FP32_IR || norm_parts(c) <= 256);
 }
 
-// Whether a batch may fold its stop tests into the next V-cycle's level-0
-// down kernel: that of the fast cycle, with a workgroup of four wavefronts or
-// more.
+// Whether the fault update that follows a batch launched kernel by kernel may
+// run its last stop test.
+bool defer_fits(const qdeq_ctx *c) { return launch_direct(c) && test_moves(c); }
+
+// Whether a batch (launched kernel by kernel, or captured as a stage's graph)
+// may fold its stop tests into the next V-cycle's level-0 down kernel: that
+// of the fast cycle, with a workgroup of four wavefronts or more.  FP32
+// refinement sums a partial per row in every workgroup: worth the stop test's
+// launch up to 8 workgroups a CU (1089 at 1025^2: 220.5 -> 215.7 us a solve,
+// 257^2: 135.5 -> 128.8; 4257 at 2049^2: 411.5 -> 413.5).
 bool fold_fits(const qdeq_ctx *c) {
-  return defer_fits(c) && use_tiled(c) && tail_entry_level(c) >= 1 &&
-         TX_THREADS * tile_shape(c, 0, true).tyt >= 256;
+  if (!test_moves(c) || !use_tiled(c) || tail_entry_level(c) < 1) return false;
+  const LevelDims &d = c->lv[0];
+  const TileShape dn = tile_shape(c, 0, true);
+  const long tiles = (long)((d.K + dn.tx - 1) / dn.tx) * ((d.N + dn.ty - 1) / dn.ty);
+  return TX_THREADS * dn.tyt >= 256 &&
+         (c->cfg.precision == QDEQ_PREC_FP64 || tiles <= 8 * 256);
 }
 
 // Whether the start of the next FP64 solve may be folded into its first

@@ -577,6 +577,70 @@ def test_stop_tests_folded_equal_separate_runs(n, levels, steps, monkeypatch):
     assert fa > 0
 
 
+@pytest.mark.parametrize("n,levels,kw", [
+    (257, 5, dict(precision=config.PREC_FP32_IR)),
+    (65, 3, dict(precision=config.PREC_FP32_IR)),
+    (2113, 8, dict(precision=config.PREC_FP32_IR)),  # more rows than norm partials
+    (129, 4, dict(graphs=True)),
+    (257, 5, dict(precision=config.PREC_FP32_IR, graphs=True)),
+])
+def test_other_stop_tests_folded_equal_separate_runs(n, levels, kw, monkeypatch):
+    """The same for FP32 refinement (a partial per row of the FP64 residual)
+    and within the V-cycles of a stage's graph."""
+    kw = dict(kw)
+    if kw.pop("graphs", False):
+        monkeypatch.setenv("QDEQ_GRAPH_LAUNCH", "1")
+    pb = config.make_bp1_problem(n, basin=True, levels=levels,
+                                 tol_mode=config.TOL_REL, tol=1e-10)
+    me = lib.build_mu_equi(pb.mu)
+    runs = []
+    for fold in (True, False):
+        if fold:
+            monkeypatch.delenv("QDEQ_FOLD_STOP", raising=False)
+        else:
+            monkeypatch.setenv("QDEQ_FOLD_STOP", "0")
+        with lib.Engine(pb, me, **{**PROD, **kw}) as eng:
+            eng.rk43_setup()
+            eng.rk43_step(12 if n > 1025 else 80)
+            runs.append((eng.state(), eng.folded_stop_tests()))
+    (a, fa), (b, fb) = runs
+    for key in ("t", "dt", "vcycles", "solves", "attempts"):
+        assert a["info"][key] == b["info"][key], key
+    for k in ("slip", "psi", "V", "U"):
+        np.testing.assert_array_equal(a[k], b[k])
+    assert fb == 0
+    assert fa > 0
+
+
+@pytest.mark.parametrize("cap", [2, 3, 5])
+def test_folded_refinement_stop_tests_stop_at_the_cap(cap, monkeypatch):
+    """The same for FP32 refinement, also in a stage's graph."""
+    pb = config.make_bp1_problem(129, basin=True, levels=4)
+    me = oracle.mu_equi(pb.mu)
+    U = _perturbed(pb, 11)
+    out = []
+    for fold in (True, False):
+        if fold:
+            monkeypatch.delenv("QDEQ_FOLD_STOP", raising=False)
+        else:
+            monkeypatch.setenv("QDEQ_FOLD_STOP", "0")
+        with lib.Engine(pb, me, **{**PROD, "tol": 1e-300, "max_vcycles": cap,
+                                   "precision": config.PREC_FP32_IR}) as eng:
+            V = U.copy()
+            with pytest.raises(lib.QdeqError) as ei:
+                eng.ode_solve(V)
+            assert ei.value.status == lib.QDEQ_ERR_MG_NOT_CONVERGED
+            with pytest.raises(lib.QdeqError) as ei:
+                eng.rk43_setup()
+                lib.ensemble_step([eng], 1)
+            out.append((V, eng.state()["U"], eng.folded_stop_tests()))
+    (va, ua, fa), (vb, ub, fb) = out
+    np.testing.assert_array_equal(va, vb)
+    np.testing.assert_array_equal(ua, ub)
+    assert fb == 0
+    assert fa >= 1
+
+
 @pytest.mark.parametrize("cap", [2, 3, 5])
 def test_folded_stop_tests_stop_at_the_cap(cap, monkeypatch):
     """A solve that cannot meet its tolerance stops at the V-cycle cap with
