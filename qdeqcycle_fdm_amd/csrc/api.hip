@@ -92,6 +92,7 @@ static void free_ctx(qdeq_ctx *c) {
   }
   (void)hipFree(c->mu_equi);
   (void)hipFree(c->cinv32);
+  (void)hipFree(c->cinv4);
   (void)hipFree(c->partial);
   (void)hipFree(c->gate);
   (void)hipFree(c->scal);

@@ -66,7 +66,8 @@ static void gauss_jordan(std::vector<double> &A, int n, std::vector<double> &X) 
 
 int build_coarse_inverse(qdeq_ctx *c) {
   (void)hipFree(c->cinv32);
-  c->cinv32 = nullptr;
+  (void)hipFree(c->cinv4);
+  c->cinv32 = c->cinv4 = nullptr;
   c->coarse_n = 0;
   if (c->cfg.cycle != QDEQ_CYCLE_FAST || c->cfg.n_coarse != 0) return QDEQ_OK;
   const LevelDims &d = c->lv[c->L - 1];
@@ -91,6 +92,16 @@ int build_coarse_inverse(qdeq_ctx *c) {
       xt32[(size_t)col * n + r] = (float)X[(size_t)r * n + col];
   QDEQ_HIP(c, hipMalloc(&c->cinv32, xt32.size() * sizeof(float)));
   QDEQ_HIP(c, hipMemcpyAsync(c->cinv32, xt32.data(), xt32.size() * sizeof(float),
+                             hipMemcpyHostToDevice, c->stream));
+  // and four columns of a row side by side (coarse_quad_at), padded with zeros
+  const int Q = coarse_chunks(n), C = coarse_chunk_len(n);
+  std::vector<float> x4((size_t)Q * coarse_chunk_quads(n) * n * 4, 0.0f);
+  for (int r = 0; r < n; r++)
+    for (int col = 0; col < n; col++)
+      x4[4 * coarse_quad_at(n, col / C, (col % C) / 4, r) + (col % C) % 4] =
+          (float)X[(size_t)r * n + col];
+  QDEQ_HIP(c, hipMalloc(&c->cinv4, x4.size() * sizeof(float)));
+  QDEQ_HIP(c, hipMemcpyAsync(c->cinv4, x4.data(), x4.size() * sizeof(float),
                              hipMemcpyHostToDevice, c->stream));
   QDEQ_HIP(c, hipStreamSynchronize(c->stream));
   c->coarse_n = n;

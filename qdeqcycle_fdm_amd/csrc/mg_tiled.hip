@@ -36,6 +36,10 @@ constexpr int TILE_THREADS = TX_THREADS * TY_THREADS;
 constexpr int TAIL_THREADS = 1024;
 constexpr int TAIL_MAX_N = 33;  // levels with N, K <= this run in the tail
 // one quad of a tail level per thread
+// threads of the tail of one level and the direct solve, whose coarsest level
+// has at most 17 x 15 unknowns
+constexpr int DIRECT_THREADS = 512;
+static_assert(((TAIL_MAX_N + 1) / 2) * ((TAIL_MAX_N + 1) / 2) <= DIRECT_THREADS, "tail quads");
 static_assert(((TAIL_MAX_N + 1) / 2) * ((TAIL_MAX_N + 1) / 2) <= TAIL_THREADS, "tail quads");
 
 // Update of one point with its quantity a = relax / (m1 + m2 + m3 + m4)
@@ -804,7 +808,8 @@ struct TailArgs {
   void *e_out;          // correction of the entry level (global)
   int nu_pre, nu_post, nu_coarse;
   double relax;
-  const void *minv;     // direct coarsest solve (column-major FP32 inverse) or null
+  const void *minv;     // direct coarsest solve (FP32 inverse: column-major cinv32 in
+                        // k_tail, else cinv4) or null
   int cn;               // coarsest unknowns for minv
   const int *gate;      // skip flag of a batched solve, or null
 };
@@ -934,56 +939,115 @@ struct TailScratch {
     for (int i = 0; i < a.nlev; i++) R += tail_level_words(a.lv[i].N, a.lv[i].K);
     E = R + tail_plane_words(a.lv[0].K);
     G = E + a.lv[0].N * a.lv[0].K;
-    part = G + a.cn;
+    part = G + a.cn + 4;
   }
 };
 
-// Column sums of the direct coarsest solve by thread: row `row` and columns
-// c0 .. c1-1 (the split of coarse_matvec), the first AHEAD of the inverse's
-// entries fetched early.
+// The chunks' sums of the direct coarsest solve added in order, into s.E with
+// its boundary columns; ends with a barrier.
+template <typename T, int THREADS>
+__device__ inline void tail_sum_chunks(const TailScratch<T> &s, int n, int Q, int K, int W) {
+  for (int i = threadIdx.x; i < n; i += THREADS) {
+    T v = s.part[i];
+    for (int ch = 1; ch < Q; ch++) v = v + s.part[ch * n + i];
+    const int j = i / W, k = i - j * W + 1;
+    s.E[j * K + k] = v;
+    if (k == 1) s.E[j * K] = T(0);
+    if (k == W) s.E[j * K + W + 1] = T(0);
+  }
+  __syncthreads();
+}
+
+// Direct coarsest solve from s.G into s.E (level L); starts after and ends
+// with a barrier.
+template <typename T>
+__device__ inline void tail_solve(const TailArgs &a, const TailScratch<T> &s, const TailLevel &L) {
+  const float *minv = reinterpret_cast<const float *>(a.minv);
+  const int n = a.cn, W = L.K - 2, Q = coarse_chunks(n), C = coarse_chunk_len(n);
+  const int ch = threadIdx.x / n, row = threadIdx.x - ch * n;
+  const int c0 = min(ch * C, n), c1 = ch < Q ? min((ch + 1) * C, n) : c0;
+  T acc = T(0);
+#pragma unroll 8
+  for (int col = c0; col < c1; col++)
+    acc = acc + (T)load_at<float>(minv, (unsigned)(col * n + row) * 4u) * s.G[col];
+  s.part[threadIdx.x] = acc;
+  __syncthreads();
+  tail_sum_chunks<T, TAIL_THREADS>(s, n, Q, L.K, W);
+}
+
+// The same by DIRECT_THREADS threads with the inverse's entries, in 16-byte
+// groups, fetched ahead: a thread has one row and whole chunks from ch0 on,
+// each with its own sum.
 template <typename T, int AHEAD>
 struct TailDirect {
-  float ahead[AHEAD > 0 ? AHEAD : 1];
-  int row, c0, c1;
+  float4 ahead[AHEAD];
+  int row, ch0;
+  unsigned off, end;  // next group and the last one, in bytes
+  __device__ void place(const TailArgs &a) {
+    const int n = a.cn, Q = coarse_chunks(n), GC = coarse_chunk_quads(n);
+    const int parts = min(Q, DIRECT_THREADS / n), per = (Q + parts - 1) / parts;
+    const int part = (int)threadIdx.x / n;
+    row = threadIdx.x - part * n;
+    ch0 = min(part * per, Q);
+    end = (unsigned)((Q * GC - 1) * n + row) * 16u;
+    off = min((unsigned)(ch0 * GC * n + row) * 16u, end);
+  }
+  template <int FROM, int TO>
   __device__ void fetch(const TailArgs &a) {
-    const float *minv = reinterpret_cast<const float *>(a.minv);
-    const int n = a.cn, tid = threadIdx.x;
-    const int Q = coarse_chunks(n), C = coarse_chunk_len(n), ch = tid / n;
-    row = tid - ch * n;
-    c0 = min(ch * C, n);
-    c1 = ch < Q ? min((ch + 1) * C, n) : c0;
-    // one 32-bit offset stepped from column to column (clamped to the last)
-    unsigned off = (unsigned)(min(c0, n - 1) * n + row) * 4u;
-    const unsigned end = (unsigned)((n - 1) * n + row) * 4u;
 #pragma unroll
-    for (int i = 0; i < AHEAD; i++) {
-      ahead[i] = load_at<float>(minv, off);
-      off = min(off + (unsigned)n * 4u, end);
+    for (int i = FROM; i < TO; i++) {
+      ahead[i] = load_at<float4>(reinterpret_cast<const float4 *>(a.minv), off);
+      off = min(off + (unsigned)a.cn * 16u, end);
     }
   }
-  // corrections E of the coarsest level L from s.G; starts after and ends
-  // with a barrier
+  // The group's four values of s.G are read two groups ahead.  Padding entries
+  // are zero and s.G has four zeros behind it, so no group needs a test.
   __device__ void solve(const TailArgs &a, const TailScratch<T> &s, const TailLevel &L) {
-    const float *minv = reinterpret_cast<const float *>(a.minv);
-    const int n = a.cn, tid = threadIdx.x, W = L.K - 2, Q = coarse_chunks(n);
+    const int n = a.cn, Q = coarse_chunks(n), C = coarse_chunk_len(n);
+    const int GC = coarse_chunk_quads(n), skip = C - 4 * (GC - 1);
+    int ch = ch0, left = GC, col = min(ch0 * C, n), left_col = GC;
+    struct Four {
+      T v[4];
+    } g[3];
+    auto read = [&](Four &f) {
+#pragma unroll
+      for (int e = 0; e < 4; e++) f.v[e] = s.G[col + e];
+      const bool end = --left_col == 0;
+      col = min(col + (end ? skip : 4), n);
+      if (end) left_col = GC;
+    };
     T acc = T(0);
+    auto add = [&](const float4 &m, const Four &f) {
+      acc = acc + (T)m.x * f.v[0];
+      acc = acc + (T)m.y * f.v[1];
+      acc = acc + (T)m.z * f.v[2];
+      acc = acc + (T)m.w * f.v[3];
+      if (--left == 0) {
+        if (ch < Q) s.part[ch * n + row] = acc;
+        acc = T(0);
+        ch++;
+        left = GC;
+      }
+    };
+    const int parts = min(Q, DIRECT_THREADS / n), most = (Q + parts - 1) / parts * GC;
+    read(g[0]);
+    read(g[1]);
 #pragma unroll
     for (int i = 0; i < AHEAD; i++)
-      if (c0 + i < c1) acc = acc + (T)ahead[i] * s.G[c0 + i];
-#pragma unroll 8
-    for (int col = c0 + AHEAD; col < c1; col++)
-      acc = acc + (T)load_at<float>(minv, (unsigned)(col * n + row) * 4u) * s.G[col];
-    s.part[tid] = acc;
-    __syncthreads();
-    for (int i = tid; i < n; i += TAIL_THREADS) {
-      T v = s.part[i];
-      for (int ch = 1; ch < Q; ch++) v = v + s.part[ch * n + i];
-      const int j = i / W, k = i - j * W + 1;
-      s.E[j * L.K + k] = v;
-      if (k == 1) s.E[j * L.K] = T(0);
-      if (k == W) s.E[j * L.K + W + 1] = T(0);
+      if (i < most) {
+        read(g[(i + 2) % 3]);
+        add(ahead[i], g[i % 3]);
+      }
+    for (int i = AHEAD; i < most; i++) {
+      const Four f = g[AHEAD % 3];
+      g[AHEAD % 3] = g[(AHEAD + 1) % 3];
+      read(g[(AHEAD + 1) % 3]);
+      add(load_at<float4>(reinterpret_cast<const float4 *>(a.minv),
+                          (unsigned)min((ch0 * GC + i) * n + row, (Q * GC - 1) * n + row) * 16u),
+          f);
     }
     __syncthreads();
+    tail_sum_chunks<T, DIRECT_THREADS>(s, n, Q, L.K, L.K - 2);
   }
 };
 
@@ -1021,10 +1085,8 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_tail(TailArgs a) {
                   direct && l + 1 == last ? s.G : nullptr, (T)C.DH2, C.N, C.K);
   }
   if (direct) {
-    TailDirect<T, 0> d;
-    d.fetch(a);
     if (last == 0) __syncthreads();
-    d.solve(a, s, LC);
+    tail_solve(a, s, LC);
   } else {
     const QTile<T, kTailPlane> t = tail_tile(base, a, last);
     tail_quad<T, EXACT>(t, p, LC, relax);
@@ -1063,10 +1125,17 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_tail(TailArgs a) {
 
 // The tail of the production cycle: one level and the direct coarsest solve.
 // The level's quads stay in registers from the load to the store, and each
-// thread fetches the first kTailAhead of its entries of the coarsest inverse
-// (255^2 floats at 1025^2, from the memory side) before the sweeps.
+// thread fetches its entries of the coarsest inverse (255^2 floats at 1025^2)
+// before they are needed, two chunks of a row in 128 registers: half of them
+// with the level's data, half behind the sweeps (all at once they hold up the
+// first sweep, at the 64 bytes a clock of one CU).  With 1024 threads
+// the registers held half of a thread's chunk and the rest was loaded during
+// the solve, which took 5.5 us between the other kernels of a V-cycle; 3.5
+// now, the FP32 to FP64 conversions and the products' issue (V-cycle at 1025^2
+// 80.7 -> 79.3 us; launched back to back, with the inverse in the L2, the
+// kernel takes 10.4 us either way).
 template <typename T, bool EXACT>
-__global__ __launch_bounds__(TAIL_THREADS) void k_tail_direct(TailArgs a) {
+__global__ __launch_bounds__(DIRECT_THREADS) void k_tail_direct(TailArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   T *base = reinterpret_cast<T *>(smem);
   const TailScratch<T> s(base, a);
@@ -1081,7 +1150,9 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_tail_direct(TailArgs a) {
     quad_load<T, true>(t, q, (const T *)nullptr, (const T *)a.f_in, (const T *)L.cx,
                        (const T *)L.cz, L.N, L.K, L.P, true);
   TailDirect<T, kTailAhead> d;
-  d.fetch(a);
+  d.place(a);
+  d.template fetch<0, kTailAhead / 2>(a);
+  if (threadIdx.x < 4) s.G[a.cn + threadIdx.x] = T(0);
   if (q.valid) {
     quad_factors<T, EXACT>(q, relax);
     quad_put(t, q);
@@ -1089,6 +1160,7 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_tail_direct(TailArgs a) {
   __syncthreads();
   if (leave) return;
   tail_sweep<T, EXACT>(t, q, a.nu_pre, DH2, relax);
+  d.template fetch<kTailAhead / 2, kTailAhead>(a);
   tail_restrict(t, q, s.R, DH2, tail_rhs(base, a, 1), s.G, (T)C.DH2, C.N, C.K);
   d.solve(a, s, C);
   if (q.valid) {
@@ -1102,6 +1174,63 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_tail_direct(TailArgs a) {
     quad_rc(t, q.id, j, k);
     quad_store(q, j, k, reinterpret_cast<T *>(a.e_out), L.N, L.K, L.P);
   }
+}
+
+// A tail of the direct coarsest solve alone (the next finer level is too large
+// for the tail): e = inverse (DH^2 f), COARSE_ROWS rows per workgroup, whose
+// entries of the inverse are staged in the LDS by all threads before one
+// wavefront sums a chunk of a row per lane.  In one workgroup (k_tail) 384
+// unknowns took 9.6 us, bound by one CU's loads; 5.5 us in 24
+// workgroups (V-cycle at 801 x 481 64 -> 60 us).
+constexpr int COARSE_ROWS = 16, COARSE_THREADS = 512;
+__host__ __device__ inline size_t coarse_rows_lds(int n, size_t esz) {
+  return (size_t)coarse_chunks(n) * coarse_chunk_quads(n) * COARSE_ROWS * 16 +
+         (n + 4 + 4 * COARSE_ROWS) * esz;
+}
+template <typename T>
+__global__ __launch_bounds__(COARSE_THREADS) void k_coarse_rows(TailArgs a) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  const TailLevel &L = a.lv[0];
+  const bool leave = a.gate && a.gate[0];  // the solve has converged
+  const int n = a.cn, W = L.K - 2, Q = coarse_chunks(n), C = coarse_chunk_len(n);
+  const int GC = coarse_chunk_quads(n), groups = Q * GC * COARSE_ROWS, tid = threadIdx.x;
+  float4 *M = reinterpret_cast<float4 *>(smem);
+  T *G = reinterpret_cast<T *>(M + groups), *part = G + n + 4;
+  const int row0 = blockIdx.x * COARSE_ROWS;
+  const float4 *inv = reinterpret_cast<const float4 *>(a.minv);
+#pragma unroll 4
+  for (int i = tid; i < groups; i += COARSE_THREADS)
+    M[i] = inv[(size_t)(i / COARSE_ROWS) * n + min(row0 + i % COARSE_ROWS, n - 1)];
+  for (int i = tid; i < n + 4; i += COARSE_THREADS) {
+    const int j = i / W, k = i - j * W + 1;
+    G[i] = i < n ? (T)L.DH2 * ((const T *)a.f_in)[(size_t)j * L.P + k] : T(0);
+  }
+  __syncthreads();
+  if (leave) return;
+  const int ch = tid / COARSE_ROWS, r = tid % COARSE_ROWS, row = row0 + r;
+  if (ch < Q) {
+    T acc = T(0);
+#pragma unroll 8
+    for (int g = 0; g < GC; g++) {
+      // padding entries are zero; so is G behind its end
+      const float4 m = M[(ch * GC + g) * COARSE_ROWS + r];
+      const T *p = G + min(ch * C + 4 * g, n);
+      acc = acc + (T)m.x * p[0];
+      acc = acc + (T)m.y * p[1];
+      acc = acc + (T)m.z * p[2];
+      acc = acc + (T)m.w * p[3];
+    }
+    part[tid] = acc;
+  }
+  __syncthreads();
+  if (ch != 0 || row >= n) return;
+  T v = part[r];
+  for (int q = 1; q < Q; q++) v = v + part[q * COARSE_ROWS + r];
+  const int j = row / W, k = row - j * W + 1;
+  T *e = (T *)a.e_out + (size_t)j * L.P;
+  e[k] = v;
+  if (k == 1) e[0] = T(0);
+  if (k == W) e[W + 1] = T(0);
 }
 
 // ---------------------------------------------------------------------------
@@ -1154,7 +1283,7 @@ static size_t tail_lds_bytes(const qdeq_ctx *c, int lt) {
   for (int l = lt; l < c->L; l++) n += tail_level_words(c->lv[l].N, c->lv[l].K);
   n += tail_plane_words(c->lv[lt].K);  // residuals
   n += (size_t)c->lv[lt].N * c->lv[lt].K;           // corrections
-  n += c->coarse_n;  // right-hand side of the direct coarsest solve
+  n += c->coarse_n + 4;  // right-hand side of the direct coarsest solve
   n += 1024;         // its partial sums
   return n * sizeof(T);
 }
@@ -1483,12 +1612,18 @@ static void launch_tail(qdeq_ctx *c, LevelBufs<T> *B, int lt) {
   a.minv = c->coarse_n > 0 ? (const void *)c->cinv32 : nullptr;
   a.gate = c->gate_ptr;
   const size_t lds = tail_lds_bytes<T>(c, lt);
-  if (FULL_TOP && a.nlev == 2 && a.minv)
-    hipLaunchKernelGGL((k_tail_direct<T, EXACT>), dim3(1), dim3(TAIL_THREADS), lds,
+  if (FULL_TOP && a.nlev == 1 && a.minv) {
+    a.minv = c->cinv4;
+    hipLaunchKernelGGL((k_coarse_rows<T>), dim3((a.cn + COARSE_ROWS - 1) / COARSE_ROWS),
+                       dim3(COARSE_THREADS), coarse_rows_lds(a.cn, sizeof(T)), c->stream, a);
+  } else if (FULL_TOP && a.nlev == 2 && a.minv) {
+    a.minv = c->cinv4;
+    hipLaunchKernelGGL((k_tail_direct<T, EXACT>), dim3(1), dim3(DIRECT_THREADS), lds,
                        c->stream, a);
-  else
+  } else {
     hipLaunchKernelGGL((k_tail<T, EXACT, FULL_TOP>), dim3(1), dim3(TAIL_THREADS), lds,
                        c->stream, a);
+  }
 }
 
 // Fast V-cycle for the FP64 solve (level 0 = the displacement, f = 0) or
@@ -1935,6 +2070,8 @@ int tiled_setup(qdeq_ctx *c) {
     SETA((k_up<float, true, false, PROL_REF, UP_ADD64, S>));
     SETA((k_up<float, true, false, PROL_NONE, UP_ADD64, S>));
   });
+  SETA((k_coarse_rows<double>));
+  SETA((k_coarse_rows<float>));
   SETA((k_tail_direct<double, true>));
   SETA((k_tail_direct<float, false>));
   SETA((k_tail<double, true, true>));

@@ -237,6 +237,7 @@ struct qdeq_ctx {
   // the coarsest operator, column-major, stored in FP32 (products and sums
   // in the solve's own precision)
   float *cinv32 = nullptr;
+  float *cinv4 = nullptr;      // the same in 16-byte groups (coarse_quad_at)
   int coarse_n = 0;
   // HIP-event timing of one kernel of the fast cycle (0 = off; see
   // qdeq_set_kernel_timing): on sampled V-cycles the cycle is launched
@@ -390,6 +391,16 @@ __host__ __device__ inline int coarse_chunks(int n) {
 __host__ __device__ inline int coarse_chunk_len(int n) {
   const int q = coarse_chunks(n);
   return (n + q - 1) / q;
+}
+// 16-byte groups of the inverse: four columns of one row, a chunk's columns
+// padded to whole groups; the group of chunk ch, columns 4 g.. of the chunk,
+// row r.  A chunk's groups, and consecutive chunks', follow each other at a
+// stride of n groups.
+__host__ __device__ inline int coarse_chunk_quads(int n) {
+  return (coarse_chunk_len(n) + 3) / 4;
+}
+__host__ __device__ inline size_t coarse_quad_at(int n, int ch, int g, int r) {
+  return ((size_t)ch * coarse_chunk_quads(n) + g) * n + r;
 }
 // e[row] (rows < n, all threads of the block) = sum_col minvT[col*n+row] g[col]
 // in the chunked order; part: >= 1024 LDS elements; ends with a barrier.
