@@ -306,8 +306,9 @@ int qdeq_projection_stats(qdeq_ctx *ctx, long long *offered,
  * one simulation launching kernel by kernel, each stage's fault update,
  * start and first V-cycles are queued behind the previous stage's solve and
  * run only if that solve converged with the V-cycles already queued; else
- * they abandon themselves and the solve goes on.  The same holds across
- * steps (the next step's stage 2 behind an accepted step's final stage 1)
+ * they abandon themselves and the solve goes on (either cycle, FP64 or FP32
+ * refinement, the plain or the projection start; not with the learned
+ * guess).  The same holds across steps (the next step's stage 2 behind an accepted step's final stage 1)
  * when the next step runs within the same call and neither per-step outputs
  * nor events are on.  Results are the same either way (QDEQ_SPECULATE=0 in
  * the environment at qdeq_create turns it off).  Counts of such solves taken
@@ -316,12 +317,14 @@ int qdeq_projection_stats(qdeq_ctx *ctx, long long *offered,
 int qdeq_launch_ahead_stats(qdeq_ctx *ctx, long long *taken, long long *abandoned,
                             long long *taken_next_step);
 
-/* Stop tests folded into the next V-cycle so far (no reference
- * counterpart): within a batch of V-cycles launched kernel by kernel (one
- * simulation, FP64 tiled cycle), the residual-norm test of every V-cycle
- * but the batch's last runs in the next V-cycle's level-0 down kernel
- * instead of a kernel of its own; every workgroup sums the norm partials in
- * the stop-test kernel's order, so the decisions and results are the same
+/* Stop tests run in the kernel behind their V-cycle so far (no reference
+ * counterpart): within a batch of V-cycles on the tile kernels, also one
+ * captured in a stage's graph, the residual-norm test of every V-cycle of the
+ * fast cycle but the batch's last runs in the next V-cycle's level-0 down
+ * kernel, and the last one, with the next stage launched ahead, in the fault
+ * update (or the projection's commit) behind the solve, instead of a kernel
+ * of its own; every workgroup sums the norm partials in the stop-test
+ * kernel's order, so the decisions and results are the same
  * (QDEQ_FOLD_STOP=0 in the environment at qdeq_create turns it off). */
 int qdeq_folded_stop_tests(qdeq_ctx *ctx, long long *folded);
 

@@ -7,7 +7,9 @@
 //           2 n_pre + 2 points, so the ring of redundant updates makes every
 //           interior value exactly what global sweeps would produce;
 //   k_tail  (levels with N <= TAIL_MAX_N): one workgroup runs the rest of the
-//           V-cycle in LDS with workgroup barriers only;
+//           V-cycle in LDS with workgroup barriers only (k_tail_direct: the
+//           production tail of one level and the direct coarsest solve;
+//           k_coarse_rows: a tail of that solve alone, over workgroups);
 //   k_up    (level l): bilinear prolongation + correction (folded into the
 //           tile load), n_post sweeps, and on level 0 either the
 //           residual-norm partials (FP64 solve) or the FP64 update u += e
