@@ -886,7 +886,7 @@ StopArgs mg_take_stop(qdeq_ctx *c, MgSolve &m) {
   if (!m.stop_due) return a;
   m.stop_due = false;
   a.part = c->partial;
-  a.nb = norm_parts(c);
+  a.nb = m.stop_parts;
   a.rel = c->cfg.tol_mode == QDEQ_TOL_REL ? 1 : 0;
   a.tol = c->cfg.tol;
   a.scal = c->scal;
@@ -900,7 +900,7 @@ void mg_flush_stop(qdeq_ctx *c, MgSolve &m) {
   if (!m.stop_due) return;
   m.stop_due = false;
   hipLaunchKernelGGL(k_norm_gate, dim3(1), dim3(NORM_THREADS), 0, c->stream, c->partial,
-                     norm_parts(c), c->scal, c->mbox_dev + m.page * SC_COUNT, c->gate,
+                     m.stop_parts, c->scal, c->mbox_dev + m.page * SC_COUNT, c->gate,
                      c->cfg.tol_mode == QDEQ_TOL_REL ? 1 : 0, c->cfg.tol,
                      c->cfg.max_vcycles);
 }
@@ -1170,6 +1170,7 @@ static int launch_batch_of(qdeq_ctx *c, MgSolve &m, int k, bool allow_sample) {
     if (folded) c->folded_tests++;
     // the last one's may run in the fault update behind the solve
     m.stop_due = defer && i + 1 == k && m.launched < c->cfg.max_vcycles;
+    if (m.stop_due) m.stop_parts = norm_parts(c);
     c->skip_gate = folded || m.stop_due;
     if (sample) {
       c->emit_events = true;

@@ -100,6 +100,7 @@ struct MgSolve {
   // the stop test of its last V-cycle is still to be launched: by the fault
   // update queued behind the solve (stop_args), or else by mg_flush_stop
   bool stop_due = false;
+  int stop_parts = 0;  // its norm partials (the tiles may change before it runs)
 };
 
 // The stop test of a solve's last V-cycle run by another kernel

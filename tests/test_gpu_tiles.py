@@ -134,3 +134,27 @@ def test_run_after_a_solve_that_fails_behind_a_queued_stage(n, levels, cap):
     for key in ("t", "vcycles", "solves"):
         assert a["info"][key] == b["info"][key], key
     np.testing.assert_array_equal(a["U"], b["U"])
+
+
+@pytest.mark.parametrize("precision", [config.PREC_FP64, config.PREC_FP32_IR])
+def test_untiled_solve_after_a_failed_run(precision):
+    """The stop test that a failed run leaves due belongs to the tiles it ran
+    on, also when the next solve runs without tiles."""
+    pb = config.make_bp1_problem(129, basin=True, levels=4, tol_mode=config.TOL_REL, tol=1e-10)
+    me = oracle.mu_equi(pb.mu)
+    U = _perturbed(pb, 24)
+    kw = {**PROD, "ini_dt": 1e5, "max_vcycles": 2, "precision": precision}
+    ends = []
+    for fail in (True, False):
+        with lib.Engine(pb, me, **kw) as eng:
+            if fail:
+                eng.rk43_setup()
+                with pytest.raises(lib.QdeqError):
+                    eng.rk43_step(60)
+            eng.set_tiles(False)
+            V = U.copy()
+            with pytest.raises(lib.QdeqError) as e:
+                eng.ode_solve(V)
+            assert e.value.status == lib.QDEQ_ERR_MG_NOT_CONVERGED
+            ends.append(V)
+    np.testing.assert_array_equal(ends[0], ends[1])
