@@ -37,12 +37,12 @@ constexpr int TY_THREADS = 16;   // 16 rows of lanes: 1024 threads per tile
 constexpr int TILE_THREADS = TX_THREADS * TY_THREADS;
 constexpr int TAIL_THREADS = 1024;
 constexpr int TAIL_MAX_N = 33;  // levels with N, K <= this run in the tail
-// one quad of a tail level per thread
 // threads of the tail of one level and the direct solve, whose coarsest level
 // has at most 17 x 15 unknowns
 constexpr int DIRECT_THREADS = 512;
+// one quad of a tail level per thread
 static_assert(((TAIL_MAX_N + 1) / 2) * ((TAIL_MAX_N + 1) / 2) <= DIRECT_THREADS, "tail quads");
-static_assert(((TAIL_MAX_N + 1) / 2) * ((TAIL_MAX_N + 1) / 2) <= TAIL_THREADS, "tail quads");
+static_assert(DIRECT_THREADS <= TAIL_THREADS, "tail quads");
 
 // Update of one point with its quantity a = relax / (m1 + m2 + m3 + m4)
 // (EXACT, the reference's form) or m1 + m2 + m3 + m4 (plain) formed once: the
@@ -1313,7 +1313,6 @@ static double pass_us(int tiles, int nq, int sweeps, double mbytes) {
   const int per_cu = (tiles + 255) / 256;
   return 3.3 + mbytes / 6.0 + 2 * sweeps * (0.17 + 0.017 * per_cu * nq / 64.0);
 }
-
 
 // Whether a shape fits the kernels: even sizes, tile rows (with halo) of at
 // most 320 points, and the LDS with 8 KiB to spare.
