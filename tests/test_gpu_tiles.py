@@ -158,3 +158,96 @@ def test_untiled_solve_after_a_failed_run(precision):
             assert e.value.status == lib.QDEQ_ERR_MG_NOT_CONVERGED
             ends.append(V)
     np.testing.assert_array_equal(ends[0], ends[1])
+
+
+@pytest.mark.parametrize("ni,nk,levels", [(129, 129, 3), (130, 97, 3), (66, 131, 2), (41, 57, 1),
+                                          (257, 65, 4), (100, 101, 2)])
+@pytest.mark.parametrize("sweeps", [(20, 21, 32), (5, 8, 3), (0, 1, 1)])
+def test_reference_cycle_fp32_on_tiles_equals_untiled(ni, nk, levels, sweeps):
+    """The same passes for the FP32 correction of refinement (a first pass from
+    zero, the last one added into the FP64 displacement), bit for bit against
+    one launch per half-sweep."""
+    pb = _problem(ni, nk, levels)
+    me = oracle.mu_equi(pb.mu)
+    U = _perturbed(pb, 25)
+    kw = dict(cycle=config.CYCLE_REFERENCE, n_pre=sweeps[0], n_post=sweeps[1],
+              n_coarse=sweeps[2], precision=config.PREC_FP32_IR)
+    ends = []
+    for tiled in (True, False):
+        with lib.Engine(pb, me, tol=1e-300, max_vcycles=2, **kw) as eng:
+            if not tiled:
+                eng.set_tiles(False, 8, 2)
+            V = U.copy()
+            with pytest.raises(lib.QdeqError) as e:
+                eng.ode_solve(V)
+            assert e.value.status == lib.QDEQ_ERR_MG_NOT_CONVERGED
+            ends.append(V)
+    assert not np.array_equal(ends[0], U)
+    np.testing.assert_array_equal(ends[0], ends[1])
+
+
+# default, then each device-side decision switched off
+SWITCHES = [{}, {"QDEQ_SPECULATE": "0"}, {"QDEQ_FOLD_STOP": "0"}, {"QDEQ_HOST_START": "1"},
+            {"QDEQ_GRAPH_LAUNCH": "1"}]
+
+
+@pytest.mark.parametrize("n,levels,sweeps", [(65, 3, (32, 32, 32)), (129, 4, (5, 8, 3))])
+@pytest.mark.parametrize("precision,start", [(config.PREC_FP64, "plain"),
+                                             (config.PREC_FP32_IR, "plain"),
+                                             (config.PREC_FP64, "projection"),
+                                             (config.PREC_FP32_IR, "projection"),
+                                             (config.PREC_FP64, "learned"),
+                                             (config.PREC_FP32_IR, "learned")])
+def test_reference_cycle_runs_equal_without_device_decisions(n, levels, sweeps, precision, start,
+                                                             monkeypatch):
+    """RK43 steps on the reference's cycle, with each kind of start: bit for bit
+    the same with stages launched ahead or not, stop tests in the kernel behind
+    or on their own, starts chosen on the device or by the host, and as graphs."""
+    pb = config.make_bp1_problem(n, basin=True, levels=levels, tol_mode=config.TOL_REL, tol=1e-10)
+    me = oracle.mu_equi(pb.mu)
+    names = {k for s in SWITCHES for k in s}
+    g = None
+    if start == "learned":  # zero weights: the previous solution and the remote edge's change
+        g = lib.Guess(n, hidden=128, capacity=1)
+        g.set_params(np.zeros(g.num_params, np.float32))
+    runs = []
+    for switch in SWITCHES:
+        for k in names:
+            monkeypatch.delenv(k, raising=False)
+        for k, v in switch.items():
+            monkeypatch.setenv(k, v)
+        with lib.Engine(pb, me, precision=precision, n_pre=sweeps[0], n_post=sweeps[1],
+                        n_coarse=sweeps[2], max_vcycles=200) as eng:
+            eng.rk43_setup()
+            if start == "projection":
+                eng.projection_enable(6)
+            if g is not None:
+                eng.attach_guess(g, lib.GUESS_PREDICT)
+            eng.rk43_step(25)
+            eng.rk43_step(1)
+            eng.rk43_step(15)
+            runs.append((eng.state(), eng.launch_ahead_stats()["taken"], eng.folded_stop_tests(),
+                         eng.projection_stats(), eng.guess_stats() if g is not None else None))
+            if g is not None:
+                eng.attach_guess(None, lib.GUESS_OFF)
+    a, ahead, folded, proj, learned = runs[0]
+    for switch, (b, b_ahead, b_folded, b_proj, b_learned) in zip(SWITCHES[1:], runs[1:]):
+        for key in ("t", "dt", "vcycles", "solves", "attempts"):
+            assert a["info"][key] == b["info"][key], (switch, key)
+        for k in ("slip", "psi", "V", "U"):
+            assert np.all(np.isfinite(b[k])), (switch, k)
+            np.testing.assert_array_equal(a[k], b[k], err_msg=str((switch, k)))
+        assert b_proj == proj and b_learned == learned, switch
+        if "QDEQ_SPECULATE" in switch:
+            assert b_ahead == 0
+        if "QDEQ_FOLD_STOP" in switch:
+            assert b_folded == 0
+    # (a candidate start of FP32 refinement waits for the host)
+    on_device = start == "plain" or (start == "projection" and precision == config.PREC_FP64)
+    assert (ahead > 0) == on_device
+    assert (folded > 0) == on_device
+    if start == "projection":
+        assert proj["used"] > 0
+    if g is not None:
+        assert learned["predicted"] > 0
+        g.close()
