@@ -198,7 +198,7 @@ int qdeq_create(const qdeq_config *cfg, const double *mu,
       return QDEQ_ERR_HIP;
     }
   }
-  CREATE_HIP(alloc_zero(&c->partial, kPartialCap, c->stream));
+  CREATE_HIP(alloc_zero(&c->partial, kPartialWords, c->stream));
   CREATE_HIP(alloc_zero(&c->scal, SC_COUNT, c->stream));
   CREATE_HIP(alloc_zero(&c->flags, 4, c->stream));
   CREATE_HIP(hipHostMalloc(&c->scal_host, SC_COUNT * sizeof(double)));

@@ -1240,10 +1240,12 @@ __global__ __launch_bounds__(COARSE_THREADS) void k_coarse_rows(TailArgs a) {
 // ---------------------------------------------------------------------------
 
 // The sizes of tiles that the shape checks accept: three words per point of
-// the tile and its halo, one more with a right-hand side (or, for a level-0
-// down tile, beyond eight residuals per thread) within the LDS.  The quads
-// need less of everything at every such size: one word per point of LDS, and
-// at most kMaxQuads quads per thread of 1024 threads.
+// the tile and its halo (an up kernel's of 2 n_post + 1), one more with a
+// right-hand side (or, for a level-0 down tile, beyond eight residuals per
+// thread) within the LDS.  The quads need one word per point, and a workgroup
+// holds kMaxQuads per thread of 1024 threads: enough at every such size but the
+// FP64 level-0 up kernel's with one more ring of halo, whose tiles of two or
+// four columns and 1000 rows or more (n_post = 0) are cut (up_shape).
 static size_t tile_budget_bytes(int TX, int TY, int H, bool has_f, size_t esz,
                                 bool down, int threads) {
   const size_t R = TY + 2 * H, C = TX + 2 * H;
@@ -1304,6 +1306,23 @@ TileShape tile_shape(const qdeq_ctx *c, int level, bool down) {
   if (c->tuned) return down ? c->tdown[level] : c->tup[level];
   if (c->user_tiles) return TileShape{c->tile_tx, c->tile_ty, TY_THREADS};
   return down ? c->mdown[level] : c->mup[level];
+}
+
+// Rows of an up kernel's halo: the norm's ring on level 0 in FP64.
+static int up_halo_of(const qdeq_ctx *c, int level) {
+  return up_halo(c->cfg.n_post, level == 0 && c->cfg.precision != QDEQ_PREC_FP32_IR);
+}
+
+// The up kernel's tile of a level as it is launched: the chosen shape, with no
+// more rows than the quads that a workgroup holds.  The results do not depend
+// on it.
+static TileShape up_shape(const qdeq_ctx *c, int level) {
+  TileShape s = tile_shape(c, level, false);
+  const int H = up_halo_of(c, level);
+  const int most = TILE_THREADS * (c->cfg.precision != QDEQ_PREC_FP32_IR ? kMaxQuads<double>
+                                                                         : kMaxQuads<float>);
+  s.ty = std::min(s.ty, 2 * (most / (s.tx / 2 + H)) - 2 * H);
+  return s;
 }
 
 // Model of a launch's time in us, from launches measured back to back: start,
@@ -1540,7 +1559,7 @@ static void launch_down(qdeq_ctx *c, LevelBufs<T> *B, int l, bool has_f,
 int norm_parts(const qdeq_ctx *c) {
   if (c->cfg.precision == QDEQ_PREC_FP32_IR) return norm_blocks(c);
   const LevelDims &d = c->lv[0];
-  const TileShape up = use_tiled(c) ? tile_shape(c, 0, false) : c->ref_plan[0].sh;
+  const TileShape up = use_tiled(c) ? up_shape(c, 0) : c->ref_plan[0].sh;
   return ((d.K + up.tx - 1) / up.tx) * ((d.N + up.ty - 1) / up.ty);
 }
 
@@ -1579,7 +1598,7 @@ bool fused_start_fits(const qdeq_ctx *c) {
   if (c->cfg.precision != QDEQ_PREC_FP64 || !use_tiled(c) || tail_entry_level(c) < 2)
     return false;
   const LevelDims &d = c->lv[0];
-  const TileShape dn = tile_shape(c, 0, true), up = tile_shape(c, 0, false);
+  const TileShape dn = tile_shape(c, 0, true), up = up_shape(c, 0);
   const long nd = (long)((d.K + dn.tx - 1) / dn.tx) * ((d.N + dn.ty - 1) / dn.ty);
   const long nu = (long)((d.K + up.tx - 1) / up.tx) * ((d.N + up.ty - 1) / up.ty);
   return nd <= kStartCap && nu <= kStartOff;
@@ -1590,7 +1609,7 @@ static void launch_up_t(qdeq_ctx *c, LevelBufs<T> *B, int l, double *partial,
                         double *u64, int *nblocks) {
   const int nu = c->cfg.n_post;
   const int n = run_up<T, EXACT, HAS_F, PROL_FULL, MODE>(
-      c, B, l, tile_shape(c, l, false), up_halo(nu, MODE == UP_NORM), nu, false, B[l].r,
+      c, B, l, up_shape(c, l), up_halo(nu, MODE == UP_NORM), nu, false, B[l].r,
       B[l].u, partial, u64);
   if (nblocks) *nblocks = n;
 }

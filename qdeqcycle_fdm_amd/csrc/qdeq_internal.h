@@ -545,8 +545,9 @@ __device__ inline bool solve_converged(const StopArgs &stop, const int *spec) {
 
 // Entries of c->partial: the FP64 fast cycle's level-0 up kernel writes one
 // norm partial per tile, so a level-0 tiling may have at most this many
-// tiles (qdeq_set_tiles, set_tile_shapes and the autotuner enforce it).
-constexpr int kPartialCap = 16384;
+// tiles (qdeq_set_tiles, set_tile_shapes and the autotuner enforce it).  Tiles
+// that are cut at launch (up_shape) are at most twice as many.
+constexpr int kPartialCap = 16384, kPartialWords = 2 * kPartialCap;
 
 // Row-partial layout of the level-0 residual norms (mg.hip): one block per
 // row, at most kNormCap blocks; plain norms at partial[0..), boundary data

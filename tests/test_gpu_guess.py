@@ -272,3 +272,18 @@ def test_training_step_is_adam_on_the_gradient():
         np.testing.assert_array_equal(u, v)
     g.close()
     h.close()
+
+
+def test_gradient_does_not_depend_on_earlier_batches():
+    """The K splits of the products, and so the order of their sums, come from
+    the call's own shape: the same bits before and after a larger batch."""
+    g = lib.Guess(513, hidden=512, capacity=1)
+    rng = np.random.default_rng(5)
+    x = rng.standard_normal((300, 513)).astype(np.float32)
+    t = (0.1 * rng.standard_normal((300, g.nout))).astype(np.float32)
+    first = g.forward_backward(x[:100], t[:100]) + (g.forward(x[:100]),)
+    g.forward_backward(x, t)
+    again = g.forward_backward(x[:100], t[:100]) + (g.forward(x[:100]),)
+    for a, b in zip(first, again):
+        np.testing.assert_array_equal(a, b)
+    g.close()

@@ -251,3 +251,29 @@ def test_reference_cycle_runs_equal_without_device_decisions(n, levels, sweeps, 
     if g is not None:
         assert learned["predicted"] > 0
         g.close()
+
+
+@pytest.mark.parametrize("ni,nk,levels", [(129, 129, 3), (129, 1601, 7)])
+def test_level0_up_tiles_taller_than_a_workgroup_holds(ni, nk, levels):
+    """Without post-smoothing the shape checks accept up tiles of two or four
+    columns and more rows than the quads of one workgroup: they run, cut, and
+    are reported as they were given."""
+    pb = _problem(ni, nk, levels)
+    me = oracle.mu_equi(pb.mu)
+    U = _perturbed(pb, 26)
+    p = pb.params
+    mg = oracle.MG(ni, nk, p.dh, levels, me, relax=PROD["relax"])
+    mg.set_cycle(1, 0, 0, True)
+    ref = U.copy()
+    mg.solve(ref, oracle.ORC_TOL_ABS, 1e-300, 2)
+    for up in [(2, 1360, 4), (2, 1362, 16), (2, 1600, 16), (4, 1020, 16), (4, 1060, 1)]:
+        with lib.Engine(pb, me, **{**PROD, "n_post": 0, "tol": 1e-300, "max_vcycles": 2}) as eng:
+            shapes = eng.tile_shapes()
+            shapes[0] = (shapes[0][0], up)
+            eng.set_tile_shapes(shapes)
+            assert tuple(eng.tile_shapes()[0][1]) == up
+            V = U.copy()
+            with pytest.raises(lib.QdeqError) as e:
+                eng.ode_solve(V)
+            assert e.value.status == lib.QDEQ_ERR_MG_NOT_CONVERGED
+        np.testing.assert_array_equal(V, ref, err_msg=str(up))
