@@ -89,6 +89,10 @@ void refresh_bf16(qdeq_guess *g, hipStream_t st) {
 }
 
 int ensure_train_bufs(qdeq_guess *g, int Mb) {
+  const size_t M = (size_t)Mb, wmax = (size_t)std::max(g->F0, g->H);
+  // from this call's rows, not from the buffer, which keeps the size of the
+  // largest call: the K splits fix the order of the FP32 sums
+  g->split_n = (size_t)64 * M * wmax;
   if (g->tb_M >= Mb) return QDEQ_OK;
   void *old[] = {g->X, g->Tg, g->Y, g->dZ0, g->dY, g->dYT, g->split,
                  g->mse_part, g->loss};
@@ -102,7 +106,6 @@ int ensure_train_bufs(qdeq_guess *g, int Mb) {
     (void)hipFree(g->dZbT[i]);
   }
   g->tb_M = 0;
-  const size_t M = (size_t)Mb, wmax = (size_t)std::max(g->F0, g->H);
   GHIP(g, dalloc(&g->X, M * g->nk));
   GHIP(g, dalloc(&g->Tg, M * g->noutp));
   GHIP(g, dalloc(&g->Y, M * g->noutp));
@@ -118,7 +121,6 @@ int ensure_train_bufs(qdeq_guess *g, int Mb) {
     GHIP(g, dalloc(&g->dZb[i], M * g->H));
     GHIP(g, dalloc(&g->dZbT[i], M * g->H));
   }
-  g->split_n = (size_t)64 * M * wmax;
   GHIP(g, dalloc(&g->split, g->split_n));
   GHIP(g, dalloc(&g->mse_part, (M / 128) * (size_t)(g->noutp / 128)));
   GHIP(g, dalloc(&g->loss, (size_t)1 << 16));
