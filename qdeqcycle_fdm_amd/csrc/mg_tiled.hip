@@ -977,8 +977,22 @@ __device__ inline void tail_solve(const TailArgs &a, const TailScratch<T> &s, co
   tail_sum_chunks<T, TAIL_THREADS>(s, n, Q, L.K, W);
 }
 
+// 16-byte groups of the inverse that a thread of TailDirect sums, and the most
+// over the sizes of the level below an entry level.
+__host__ __device__ constexpr int tail_direct_groups(int n) {
+  const int Q = coarse_chunks(n), fit = DIRECT_THREADS / n, parts = Q < fit ? Q : fit;
+  return (Q + parts - 1) / parts * coarse_chunk_quads(n);
+}
+constexpr int tail_direct_most() {
+  constexpr int N = (TAIL_MAX_N + 1) / 2;
+  int most = 0;
+  for (int n = 1; n <= N * (N - 2); n++) most = std::max(most, tail_direct_groups(n));
+  return most;
+}
+static_assert(tail_direct_most() <= kTailAhead, "the inverse's entries of a thread");
+
 // The same by DIRECT_THREADS threads with the inverse's entries, in 16-byte
-// groups, fetched ahead: a thread has one row and whole chunks from ch0 on,
+// groups, all fetched ahead: a thread has one row and whole chunks from ch0 on,
 // each with its own sum.
 template <typename T, int AHEAD>
 struct TailDirect {
@@ -1031,7 +1045,7 @@ struct TailDirect {
         left = GC;
       }
     };
-    const int parts = min(Q, DIRECT_THREADS / n), most = (Q + parts - 1) / parts * GC;
+    const int most = tail_direct_groups(n);
     read(g[0]);
     read(g[1]);
 #pragma unroll
@@ -1040,14 +1054,6 @@ struct TailDirect {
         read(g[(i + 2) % 3]);
         add(ahead[i], g[i % 3]);
       }
-    for (int i = AHEAD; i < most; i++) {
-      const Four f = g[AHEAD % 3];
-      g[AHEAD % 3] = g[(AHEAD + 1) % 3];
-      read(g[(AHEAD + 1) % 3]);
-      add(load_at<float4>(reinterpret_cast<const float4 *>(a.minv),
-                          (unsigned)min((ch0 * GC + i) * n + row, (Q * GC - 1) * n + row) * 16u),
-          f);
-    }
     __syncthreads();
     tail_sum_chunks<T, DIRECT_THREADS>(s, n, Q, L.K, L.K - 2);
   }
@@ -1068,10 +1074,7 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_tail(TailArgs a) {
     T *F = tail_rhs(base, a, 0);
     for (int i = tid; i < L0.N * L0.K; i += TAIL_THREADS) {
       const int j = i / L0.K, k = i - j * L0.K;
-      const T v = ((const T *)a.f_in)[(size_t)j * L0.P + k];
-      F[i] = v;
-      if (direct && last == 0 && k >= 1 && k <= L0.K - 2)
-        s.G[j * (L0.K - 2) + k - 1] = (T)L0.DH2 * v;
+      F[i] = ((const T *)a.f_in)[(size_t)j * L0.P + k];
     }
   }
   Quad<T> p;
@@ -1086,8 +1089,7 @@ __global__ __launch_bounds__(TAIL_THREADS) void k_tail(TailArgs a) {
     tail_restrict(t, p, s.R, (T)L.DH2, tail_rhs(base, a, l + 1),
                   direct && l + 1 == last ? s.G : nullptr, (T)C.DH2, C.N, C.K);
   }
-  if (direct) {
-    if (last == 0) __syncthreads();
+  if (direct) {  // below two levels or more (k_coarse_rows, k_tail_direct else)
     tail_solve(a, s, LC);
   } else {
     const QTile<T, kTailPlane> t = tail_tile(base, a, last);

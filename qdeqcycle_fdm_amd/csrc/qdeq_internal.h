@@ -385,11 +385,11 @@ inline void timing_mark(qdeq_ctx *c, int which, int pos) {
 // row's columns into coarse_chunks(n) consecutive chunks of
 // coarse_chunk_len(n) columns, summed in column order from zero, and adds
 // the chunk sums in chunk order (one thread per row and chunk, <= 1024).
-__host__ __device__ inline int coarse_chunks(int n) {
+__host__ __device__ constexpr int coarse_chunks(int n) {
   const int q = 1024 / n;
   return q < 1 ? 1 : (q > 4 ? 4 : q);
 }
-__host__ __device__ inline int coarse_chunk_len(int n) {
+__host__ __device__ constexpr int coarse_chunk_len(int n) {
   const int q = coarse_chunks(n);
   return (n + q - 1) / q;
 }
@@ -397,7 +397,7 @@ __host__ __device__ inline int coarse_chunk_len(int n) {
 // padded to whole groups; the group of chunk ch, columns 4 g.. of the chunk,
 // row r.  A chunk's groups, and consecutive chunks', follow each other at a
 // stride of n groups.
-__host__ __device__ inline int coarse_chunk_quads(int n) {
+__host__ __device__ constexpr int coarse_chunk_quads(int n) {
   return (coarse_chunk_len(n) + 3) / 4;
 }
 __host__ __device__ inline size_t coarse_quad_at(int n, int ch, int g, int r) {
