@@ -103,8 +103,9 @@ struct MgSolve {
   int stop_parts = 0;  // its norm partials (the tiles may change before it runs)
 };
 
-// The stop test of a solve's last V-cycle run by another kernel
-// (k_norm_gate's, on at most 256 partials; nb = 0: none).
+// The stop test of a solve's last V-cycle run by another kernel (k_norm_gate's;
+// nb = 0: none).  FP64 hands over at most 256 partials, one per tile, FP32
+// refinement one per row, at most kNormCap.
 struct StopArgs {
   const double *part = nullptr;
   int nb = 0, rel = 0;
@@ -511,7 +512,8 @@ __device__ inline double strided_sum(const double *__restrict__ a, int n, int t)
 // workgroup of 256 threads takes the same decision; workgroup 0 records it;
 // the cap cannot be reached), else it reads the outcome in spec[2].
 // gate[0] is not written here: the start that follows reads gate[2] and sets
-// it.  Ends with a barrier; every thread of the workgroup calls it.
+// it.  Every thread of the workgroup calls it.  Only the test passes a barrier
+// (block_sum1's); callers order no memory by this call.
 __device__ inline bool solve_converged(const StopArgs &stop, const int *spec) {
   if (stop.nb == 0) return !spec || spec[2] == 1;
   __shared__ double sh[16];
