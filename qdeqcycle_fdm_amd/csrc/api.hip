@@ -957,12 +957,7 @@ static int rk_advance(qdeq_ctx *c, bool block, int *done) {
           c->spec_abandoned++;
           proj_ahead_done(c, false);
         }
-        if (st) {
-          r.spec = false;
-          c->spec_pending = false;
-          proj_ahead_done(c, false);
-          return st;
-        }
+        if (st) return st;
         if (!sdone) return QDEQ_OK;
         if ((st = guess_after_solve(c))) return st;
         // (already queued with a stage launched ahead)
@@ -1096,6 +1091,17 @@ static int rk_request(qdeq_ctx *c, int nsteps) {
   return QDEQ_OK;
 }
 
+// Ends a request that failed: no solve is in progress, and what was launched
+// ahead of the failure belongs to no later step (each of its kernels waits on
+// a decision that the device has taken, as the host has).
+static void rk_fail(qdeq_ctx *c) {
+  c->rk.phase = RK_IDLE;
+  c->rk.spec = false;
+  c->spec_pending = false;
+  proj_ahead_done(c, false);
+  c->mg.phase = 0;
+}
+
 int qdeq_rk43_step(qdeq_ctx *c, int nsteps, qdeq_step_info *info) {
   if (!c || nsteps < 0) return set_error(c, QDEQ_ERR_ARG, "bad argument");
   int st = rk_request(c, nsteps);
@@ -1103,8 +1109,7 @@ int qdeq_rk43_step(qdeq_ctx *c, int nsteps, qdeq_step_info *info) {
   int done = 0;
   while (!done) {
     if ((st = rk_advance(c, true, &done))) {
-      c->rk.phase = RK_IDLE;
-      c->mg.phase = 0;
+      rk_fail(c);
       return st;
     }
   }
@@ -1157,7 +1162,7 @@ int qdeq_ensemble_step(qdeq_ctx **ctxs, int n, int nsteps, int *status) {
         if (st != QDEQ_OK) {
           // let the member's queued work drain before it is reused
           (void)hipStreamSynchronize(c->stream);
-          c->mg.phase = 0;
+          rk_fail(c);
           st_all = st;
         }
         c->rk.phase = RK_IDLE;

@@ -441,11 +441,12 @@ __global__ __launch_bounds__(1024) void k_combine(
     const double r1 = sqrt(e1), r2 = sqrt(e2);
     const double err = r1 / (sqrt((double)nk) * 1.0) + r2 / (sqrt((double)nk) * 1.0);
     out[0] = err;
-    // the accept test the host applies first (odeSolver.cpp:1596), for
-    // work launched ahead of the host's decision
-    gate[7] = err < totTol ? 1 : 0;
+    // the tests the host applies first (the NaN flag, then odeSolver.cpp:1596),
+    // for work launched ahead of the host's decision
+    const int flag = flags[0];
+    gate[7] = !flag && err < totTol ? 1 : 0;
     mb[MB_ERR] = err;
-    mb[MB_FLAG] = (double)flags[0];
+    mb[MB_FLAG] = (double)flag;
     __threadfence_system();
     mb[MB_RKSEQ] = seq;
   }

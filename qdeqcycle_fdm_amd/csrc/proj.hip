@@ -176,15 +176,17 @@ __device__ inline void cholesky(const double (&G)[M * (M + 1) / 2], bool drop,
 // d = g* - g_0), then the tree sums.  Output coef[i] = c_i, the weight of
 // (Z_i - Z_0), i = 1..cnt-1 (0 for a column left out, and beyond cnt),
 // coef[PROJ_MAX_SLOTS] = ||d - fit|| / ||d||, coef[PROJ_MAX_SLOTS + 1] =
-// columns kept.
+// columns kept.  Launched ahead (spec), written only if what it waits on went
+// through, so that the last fit stays that of a solve.
 template <int M>
 __global__ __launch_bounds__(PROJ_THREADS) void k_proj_coef(
     const double *__restrict__ u, int N, int P, const double *__restrict__ g,
-    ProjSlots sl, double *__restrict__ coef) {
+    ProjSlots sl, double *__restrict__ coef, const int *__restrict__ spec, int go) {
   constexpr int NP = M * (M + 1) / 2;
   extern __shared__ __align__(16) double lds[];
   __shared__ double Gs[NP];
   const int tid = threadIdx.x;
+  const bool leave = spec && spec[go] != 1;
   double *A = lds;
   double *Pt = lds + (size_t)M * N;
   unsigned keep = (1u << (M - 1)) - 1u;  // the D columns
@@ -245,7 +247,7 @@ __global__ __launch_bounds__(PROJ_THREADS) void k_proj_coef(
     c[i] = ((keep >> i) & 1u) ? acc / G[pidx<M>(i, i)] : 0.0;
   }
   const int kept = __builtin_popcount(keep);
-  if (tid == 0) {
+  if (tid == 0 && !leave) {
     coef[0] = 0.0;
 #pragma unroll
     for (int i = 1; i < PROJ_MAX_SLOTS; i++) coef[i] = i < M ? c[i - 1] : 0.0;
@@ -314,7 +316,8 @@ static size_t proj_lds_bytes(int slots, int N) {
          sizeof(double);
 }
 
-using CoefKernel = void (*)(const double *, int, int, const double *, ProjSlots, double *);
+using CoefKernel = void (*)(const double *, int, int, const double *, ProjSlots, double *,
+                            const int *, int);
 
 static CoefKernel coef_kernel(int cnt) {
   switch (cnt) {
@@ -383,7 +386,8 @@ int proj_before_solve(qdeq_ctx *c) {
   if (sl.cnt >= 2)
     hipLaunchKernelGGL(coef_kernel(sl.cnt), dim3(1), dim3(PROJ_THREADS),
                        proj_lds_bytes(sl.cnt, d.N), c->stream, c->d[0].u, d.N, d.P,
-                       c->proj_g, sl, c->proj_coef);
+                       c->proj_g, sl, c->proj_coef,
+                       (const int *)(c->spec_launch ? c->gate : nullptr), c->spec_go);
   const dim3 blk(256), grd((d.P + 255) / 256, d.N);
   // on the device path the start is written over u's interior (the plain
   // start's interior is the newest stored solution); on the host path into r
@@ -497,7 +501,8 @@ int qdeq_projection_fit(qdeq_ctx *c, const double *g_new, const double *g_old,
     for (int i = 0; i < cnt; i++) sl.s[i] = i;
     // the new column as a one-column field (pitch 1)
     hipLaunchKernelGGL(coef_kernel(cnt), dim3(1), dim3(PROJ_THREADS),
-                       proj_lds_bytes(cnt, N), c->stream, u, N, 1, g, sl, cf);
+                       proj_lds_bytes(cnt, N), c->stream, u, N, 1, g, sl, cf,
+                       (const int *)nullptr, 0);
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);

@@ -699,3 +699,47 @@ def test_accepted_case_launched_ahead_equal_waiting_runs_with_rejections(monkeyp
     assert attempts >= steps + 3         # rejected attempts happened
     assert sb["taken"] == 0
     assert sa["abandoned"] > 0 and sa["taken"] > 0
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(precision=config.PREC_FP32_IR), dict(slots=6),
+                                dict(cycle=config.CYCLE_REFERENCE, n_pre=8, n_post=8, n_coarse=8,
+                                     relax=1.0)])
+def test_steps_after_a_nan_equal_waiting_runs(kw, monkeypatch):
+    """A first step size that makes the friction law's slip rate NaN ends the
+    call while the accepted case is queued behind the combination.  Nothing of
+    it is kept: the state is that of a waiting run, and so are the state and
+    the status of a further call, and of a solve after it."""
+    pb = config.make_bp1_problem(65, basin=True, levels=3, tol_mode=config.TOL_REL, tol=1e-10)
+    me = oracle.mu_equi(pb.mu)
+    U = _perturbed(pb, 12)
+    kw = dict(kw)
+    slots = kw.pop("slots", 0)
+    runs = []
+    for spec in (True, False):
+        if spec:
+            monkeypatch.delenv("QDEQ_SPECULATE", raising=False)
+        else:
+            monkeypatch.setenv("QDEQ_SPECULATE", "0")
+        with lib.Engine(pb, me, **{**PROD, "ini_dt": 1e9, "tmax": 1e30, **kw}) as eng:
+            eng.rk43_setup()
+            if slots:
+                eng.projection_enable(slots)
+            states, status = [], []
+            for _ in range(3):
+                with pytest.raises(lib.QdeqError) as e:
+                    eng.rk43_step(5)
+                status.append(e.value.status)
+                states.append(eng.state())
+            V = U.copy()
+            eng.ode_solve(V)
+            runs.append((states, status, eng.projection_stats(), V))
+    (sa, ea, pa, va), (sb, eb, pb_, vb) = runs
+    assert ea[0] == lib.QDEQ_ERR_NAN_FRICTION
+    assert ea == eb
+    for a, b in zip(sa, sb):
+        for key in ("t", "dt", "it", "vcycles", "solves"):
+            assert a["info"][key] == b["info"][key], key
+        for k in ("slip", "psi", "V", "U"):
+            np.testing.assert_array_equal(a[k], b[k])
+    assert pa == pb_
+    np.testing.assert_array_equal(va, vb)
