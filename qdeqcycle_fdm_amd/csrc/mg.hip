@@ -278,14 +278,8 @@ __global__ __launch_bounds__(NORM_THREADS) void k_norm_gate(
       mb[SC_NORM] = v;
       const int cnt = gate[1] + 1;
       gate[1] = cnt;
-      const double thr = rel ? tol * scal[SC_NORM0] : tol;
-      int code = 0;
-      if (isnan(v) || isinf(v))
-        code = 2;
-      else if (!(v > thr))
-        code = 1;
-      else if (cnt >= cap)
-        code = 3;
+      int code = stop_code(v, rel, tol, scal);
+      if (!code && cnt >= cap) code = 3;
       if (code) gate[0] = 1;
       gate[2] = code;
       mb[MB_COUNT] = (double)cnt;

@@ -612,12 +612,7 @@ __global__ __launch_bounds__(TILE_THREADS) void k_down(
   }
   if (folding) {
     const double v = sqrt(((sdec[0] + sdec[1]) + sdec[2]) + sdec[3]);
-    const double thr = sa.rel ? sa.tol * sa.scal[SC_NORM0] : sa.tol;
-    int code = 0;
-    if (isnan(v) || isinf(v))
-      code = 2;
-    else if (!(v > thr))
-      code = 1;
+    const int code = stop_code(v, sa.rel, sa.tol, sa.scal);
     if (wg0) {
       // what k_norm_gate records (the V-cycle cap is left to it: the host
       // folds no test that could reach the cap)

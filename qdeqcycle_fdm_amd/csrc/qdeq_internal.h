@@ -507,6 +507,15 @@ __device__ inline double strided_sum(const double *__restrict__ a, int n, int t)
   return acc;
 }
 
+// Decision of the stop test behind a V-cycle on its residual norm v, in every
+// kernel that makes it: 0 go on, 1 converged, 2 not finite.  The threshold is tol times the
+// boundary-data norm (rel) or tol, the comparisons those of the host loop.
+__device__ inline int stop_code(double v, int rel, double tol, const double *scal) {
+  const double thr = rel ? tol * scal[SC_NORM0] : tol;
+  if (isnan(v) || isinf(v)) return 2;
+  return v > thr ? 0 : 1;
+}
+
 // Whether the work queued behind a solve goes on: with stop.nb it runs the
 // solve's last stop test itself (k_norm_gate's, in its order, so every
 // workgroup of 256 threads takes the same decision; workgroup 0 records it;
@@ -521,12 +530,7 @@ __device__ inline bool solve_converged(const StopArgs &stop, const int *spec) {
   const bool stopped = stop.gate[0] != 0;
   const int before = stop.gate[2];
   const double v = sqrt(block_sum1(strided_sum(stop.part, stop.nb, tid), sh));
-  const double thr = stop.rel ? stop.tol * stop.scal[SC_NORM0] : stop.tol;
-  int code = 0;
-  if (isnan(v) || isinf(v))
-    code = 2;
-  else if (!(v > thr))
-    code = 1;
+  const int code = stop_code(v, stop.rel, stop.tol, stop.scal);
   if (blockIdx.x == 0 && tid == 0) {
     const int seq = stop.gate[3] + 1;
     stop.gate[3] = seq;
