@@ -598,15 +598,20 @@ static void launch_norm_final(qdeq_ctx *c, int nparts) {
                        c->partial, nparts, c->scal + SC_NORM, mb_dev(c) + SC_NORM);
 }
 
+// Level-0 residual as r32 for IR, with its norm's partials.
+static void launch_residual32(qdeq_ctx *c) {
+  const LevelDims &d = c->lv[0];
+  hipLaunchKernelGGL((k_resnorm_partial<true>), dim3(norm_blocks(c)), dim3(NORM_THREADS), 0,
+                     c->stream, c->d[0].u, c->d[0].cx, c->d[0].cz, d.N, d.K, d.P, d.DH * d.DH,
+                     c->partial, c->s[0].f, (const int *)c->gate_ptr, (const int *)nullptr, 0);
+}
+
 // Level-0 residual norm into scal[SC_NORM] (and r32 for IR).
 static void launch_resnorm(qdeq_ctx *c, bool store32) {
   const LevelDims &d = c->lv[0];
   const double DH2 = d.DH * d.DH;
   if (store32)
-    hipLaunchKernelGGL((k_resnorm_partial<true>), dim3(norm_blocks(c)),
-                       dim3(NORM_THREADS), 0, c->stream, c->d[0].u, c->d[0].cx,
-                       c->d[0].cz, d.N, d.K, d.P, DH2, c->partial, c->s[0].f,
-                       (const int *)c->gate_ptr, (const int *)nullptr, 0);
+    launch_residual32(c);
   else
     hipLaunchKernelGGL((k_resnorm_partial<false>), dim3(norm_blocks(c)),
                        dim3(NORM_THREADS), 0, c->stream, c->d[0].u, c->d[0].cx,
@@ -1218,6 +1223,7 @@ int mg_poll(qdeq_ctx *c, bool block, int *done) {
       goto out;
     for (int i : {SC_NORM, SC_NORM0, SC_NORM_PRED}) c->scal_host[i] = mb[i];
     m.delta = c->scal_host[SC_NORM];
+    bool used = false;
     if (m.cand) {
       // used only if its residual is finite and below the previous solution's
       const double pn = c->scal_host[SC_NORM_PRED];
@@ -1226,9 +1232,9 @@ int mg_poll(qdeq_ctx *c, bool block, int *done) {
         QDEQ_HIP(c, hipMemcpyAsync(c->d[0].u, c->d[0].r,
                                    (size_t)d.N * d.P * sizeof(double),
                                    hipMemcpyDeviceToDevice, c->stream));
-        if (m.ir) launch_resnorm(c, true);  // FP32 residual of the new start
         m.delta = pn;
         c->g_accepted++;
+        used = true;
       }
     }
     m.delta0 = m.delta;
@@ -1243,6 +1249,10 @@ int mg_poll(qdeq_ctx *c, bool block, int *done) {
       return mg_finish(c, set_error(c, QDEQ_ERR_MG_NOT_CONVERGED,
                                     "multigrid: V-cycle cap reached"));
     }
+    // FP32 residual of the new start.  Its norm is known, and none is written:
+    // a solve that ends here leaves nothing in flight that writes to a mailbox
+    // slot, which the next solve arms for its own norms.
+    if (m.ir && used) launch_residual32(c);
     QDEQ_HIP(c, hipMemsetAsync(c->gate, 0, 3 * sizeof(int), c->stream));
     if ((st = launch_batch(c, batch_size(c, m.delta, m.thr)))) goto out;
     mg_flush_stop(c, m);

@@ -14,6 +14,10 @@
   and an absurd or non-finite start (fault injection) is never used: the
   run then equals the plain run bit for bit on both paths.
 """
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -23,6 +27,7 @@ from qdeqcycle_fdm_amd import config, lib
 pytestmark = pytest.mark.gpu
 
 LEVELS = {129: 4, 257: 5, 1025: 7}
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def _engine(n, tol=1e-10, **kw):
@@ -171,3 +176,37 @@ def test_bad_projection_start_falls_back_bit_for_bit(factor, host, monkeypatch):
         assert sa["info"]["vcycles"] == sb["info"]["vcycles"]
         for k in ("slip", "psi", "V", "U"):
             np.testing.assert_array_equal(sa[k], sb[k])
+
+
+_IR_RUN = """
+import sys
+import numpy as np
+from qdeqcycle_fdm_amd import config, lib
+pb = config.make_bp1_problem(2049, basin=True, levels=8, tol_mode=config.TOL_REL, tol=1e-10)
+with lib.Engine(pb, cycle=config.CYCLE_FAST, n_pre=1, n_post=3, n_coarse=0, relax=1.15,
+                precision=config.PREC_FP32_IR) as eng:
+    eng.projection_enable(6)
+    eng.rk43_setup()
+    eng.rk43_step(12)
+    st = eng.state()
+    np.savez(sys.argv[1], t=st["info"]["t"], solves=st["info"]["solves"],
+             vcycles=st["info"]["vcycles"], used=eng.projection_stats()["used"],
+             **{k: st[k] for k in ("slip", "psi", "V", "U")})
+"""
+
+
+def test_refinement_start_is_read_once_its_own_norm_has_landed(tmp_path):
+    """A start of FP32 refinement that already meets the tolerance ends its
+    solve with work in flight; the next solve reads its own norms, not what that
+    work writes: large grids run as they do with every launch waited for."""
+    runs = []
+    for blocking in ("0", "1"):
+        path = tmp_path / f"run{blocking}.npz"
+        env = {**os.environ, "HIP_LAUNCH_BLOCKING": blocking, "PYTHONPATH": ROOT}
+        subprocess.run([sys.executable, "-c", _IR_RUN, str(path)], check=True, timeout=100,
+                       cwd=ROOT, env=env)
+        runs.append(np.load(path))
+    a, b = runs
+    assert b["used"] > 0
+    for k in a.files:
+        np.testing.assert_array_equal(a[k], b[k], err_msg=k)
